@@ -13,13 +13,16 @@
 //             scan (token count, last token start) across the block and, by a decoupled
 //             look-back, across blocks, and write (kind, start, end) of every non-ignored token
 //             through LDS staging, coalesced.
-//   parser: one scan at the level of key positions. parse_keys2 maps every window of q + k token
-//           kinds to its pair entry; pscan_* scan the entries' totals (brackets, productions,
-//           depth, lowest depth, sum of arity - 1); parse_expand2 writes every position's
-//           brackets and productions (load-balanced, with two levels of adjacent bracket
-//           cancellation) and the tree's node and span words; bracket_match and parse_parents
-//           run a wave-cooperative "previous smaller-or-equal" search over 64-element chunks and
-//           a 64-ary min hierarchy.
+//   parser: one scan at the level of key positions. parse_keys_tree maps every window of q + k token
+//           kinds to its pair entry; pscan_* scan the totals of 256-position tiles (productions,
+//           depth, lowest depth, open ends); parse_tree matches every tile's pops and pushes of
+//           stack symbols in LDS, which checks the brackets and gives the parents, and writes the
+//           tree; link_tiles matches what the tiles leave open.
+//           Pair tables that do not have that form take the element-level kernels: parse_keys2,
+//           pscan_*, parse_expand2 (every position's brackets and productions, load-balanced, with
+//           two levels of adjacent bracket cancellation, and the node and span words), then
+//           bracket_match and parse_parents, a wave-cooperative "previous smaller-or-equal" search
+//           over 64-element chunks and a 64-ary min hierarchy.
 //
 // All arithmetic is integer. Tables are produced by alpacc_amd/gen (the restated generator).
 
@@ -31,6 +34,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/alpacc_hip.h"
@@ -1157,17 +1161,19 @@ __device__ __forceinline__ int hibit64(uint64_t m) { return 63 - __clzll((long l
 //
 // ds_bpermute selects the source lane by address bits 7:2 and reads no memory, so lane indexes
 // are kept as byte addresses and a negative one merely reads some lane whose value goes unused.
-__device__ __forceinline__ int lift_left(int32_t x, int pos, int32_t v) {
+__device__ __forceinline__ void lift_build(int32_t x, int32_t (&M)[6]) {
   const int lane = threadIdx.x & (WAVE - 1);
   // M[k] at lane l: min of x_l .. x_{l+2^k-1}. Windows running past lane 63 wrap around and hold
   // wrong minima, but no query below reads a window that ends past x_63.
-  int32_t M[6];
   M[0] = x;
 #pragma unroll
   for (int k = 1; k < 6; ++k) {
     const int s = 1 << (k - 1);
     M[k] = min(M[k - 1], __builtin_amdgcn_ds_bpermute(((lane + s) & (WAVE - 1)) << 2, M[k - 1]));
   }
+}
+
+__device__ __forceinline__ int lift_query(const int32_t (&M)[6], int pos, int32_t v) {
   int p4 = pos << 2;
 #pragma unroll
   for (int k = 5; k >= 0; --k) {
@@ -1178,9 +1184,15 @@ __device__ __forceinline__ int lift_left(int32_t x, int pos, int32_t v) {
   }
   pos = p4 >> 2;
   // the steps add up to 63: from pos = 64 the loop stops at 1 without having looked at x_0
-  const int32_t x0 = __builtin_amdgcn_readlane(x, 0);
+  const int32_t x0 = __builtin_amdgcn_readlane(M[0], 0);
   if (pos == 1 && x0 > v) pos = 0;
   return pos;
+}
+
+__device__ __forceinline__ int lift_left(int32_t x, int pos, int32_t v) {
+  int32_t M[6];
+  lift_build(x, M);
+  return lift_query(M, pos, v);
 }
 
 // Last j with y_j <= v among 64 values held in reverse (lane l holds y_{63-l}; INT32_MAX for
@@ -1475,6 +1487,17 @@ struct PArgs {
   uint32_t *flags;         // [0] reject
   uint64_t ntiles;
   int subst;               // single document: terminal productions pair up with the tokens
+  uint32_t tshift;         // log2 of the positions per tile: 10 (PK_TILE) or 8 (FT_TILE)
+  // the tree parser's tables (see parse_tree)
+  const uint2 *tent;       // [E]
+  const uint32_t *tbr;     // [nstack]
+  const uint2 *tprod;      // [nprod]
+  const uint4 *trow;       // [3 * (E + 1)] one row per entry, when every entry fits (FT_ROW)
+  uint32_t t_rec, t_slots, t_query;  // its LDS words per wavefront: node records, slots per lane
+                                     // (a power of two), queries
+  uint32_t t_prods, t_pops, t_pushes;  // largest counts of any entry
+  uint2 *links;            // records of the tiles' open ends (see parse_tree)
+  int32_t *tile_low, *tile_low1;  // lowest depth of every tile, and of every 64 tiles
   // batched mode: every document's positions start a new tile; element offsets run through the
   // documents, depths, s and ranks restart in every document
   struct PDoc *pdocs;        // [ndocs]
@@ -1526,14 +1549,15 @@ struct PosView {
   int subst;
 };
 
-template <bool BATCH>
+// TP: positions per tile
+template <bool BATCH, int TP = PK_TILE>
 __device__ __forceinline__ PosView pos_view(const PArgs &a, uint64_t tile) {
   PosView v;
   if (!BATCH) {
     v.kinds = a.kinds;
     v.kinds8 = a.kinds8;
     v.P = a.T_dev ? std::min<uint64_t>(*a.T_dev, a.T) + 2 : a.P;
-    v.p0 = (int64_t)(tile * PK_TILE);
+    v.p0 = (int64_t)(tile * TP);
     v.tok_base = 0;
     v.doc = 0;
     v.reset = tile == 0;
@@ -1545,7 +1569,7 @@ __device__ __forceinline__ PosView pos_view(const PArgs &a, uint64_t tile) {
     v.kinds = a.kinds + doc.tok_base;
     v.kinds8 = a.kinds8 ? a.kinds8 + doc.tok_base : nullptr;
     v.P = (uint64_t)doc.T + 2;
-    v.p0 = (int64_t)lt * PK_TILE;
+    v.p0 = (int64_t)lt * TP;
     v.tok_base = doc.tok_base;
     v.doc = d;
     v.reset = lt == 0;
@@ -1558,7 +1582,8 @@ __device__ __forceinline__ PosView pos_view(const PArgs &a, uint64_t tile) {
 template <bool BATCH>
 __device__ __forceinline__ uint64_t pk_ntiles(const PArgs &a) {
   if (BATCH) return *a.ntiles_dev;
-  if (a.T_dev) return (std::min<uint64_t>(*a.T_dev, a.T) + 2 + PK_TILE - 1) / PK_TILE;
+  if (a.T_dev)
+    return (std::min<uint64_t>(*a.T_dev, a.T) + 2 + (1ull << a.tshift) - 1) >> a.tshift;
   return a.ntiles;
 }
 
@@ -1594,22 +1619,22 @@ __device__ __forceinline__ uint32_t pk_hash_lookup(const PArgs &a, uint64_t di) 
 
 // PosView of tile `tile` (an empty view past the tile count) and the symbols of the key windows of
 // this thread's PK_IPT positions in it.
-template <bool BATCH, int KW>
+template <bool BATCH, int KW, int TP = PK_TILE>
 __device__ __forceinline__ void keys_window(const PArgs &a, uint64_t tile, uint64_t ntiles,
                                             uint32_t W, PosView &pv,
                                             uint32_t (&sym)[PK_IPT + KW - 1], bool &raw,
                                             uint32_t &off) {
   if (tile < ntiles) {
-    pv = pos_view<BATCH>(a, tile);
+    pv = pos_view<BATCH, TP>(a, tile);
   } else {
     pv = PosView{a.kinds, a.kinds8, 0, 0, 0, 0, false, 0};  // every field set: the view stays in registers
   }
-  const int64_t lp0 = pv.p0 + (int64_t)(threadIdx.x % PK_THREADS) * PK_IPT;  // in the document
+  const int64_t lp0 = pv.p0 + (int64_t)(threadIdx.x % (TP / PK_IPT)) * PK_IPT;  // in the document
   // A tile away from both ends of byte kinds (uniform over its threads): a thread's 7 symbols
   // are 7 consecutive bytes, read as the three aligned words around them (raw; keys_symbols
   // takes the bytes out). 16 positions of margin keep the words inside the kinds.
   raw = KW == 4 && tile < ntiles && pv.kinds8 != nullptr && pv.p0 >= (int64_t)a.q + 4 &&
-        pv.p0 + PK_TILE + 16 <= (int64_t)pv.P;
+        pv.p0 + TP + 16 <= (int64_t)pv.P;
   if (raw) {
     const uintptr_t addr = (uintptr_t)(pv.kinds8 + (lp0 - (int64_t)a.q - 1));
     off = (uint32_t)(addr & 3);
@@ -1783,6 +1808,147 @@ parse_keys2(PArgs a) {
   if (!BATCH && __ballot(miss) != 0ull && lane == 0) atomicOr(a.flags, 1u);
 }
 
+// ----------------------------------------------------------------------------------------------
+// The tree parser. When every entry of the pair table pops a run of stack symbols (right brackets)
+// and then pushes a run (left brackets), and its productions fill exactly the popped symbols and
+// push exactly the pushed ones (build_tree_tables simulates every entry), a production's parent is
+// the production that pushed the symbol it fills: the parents of parser.fut:286-296 and the bracket
+// matching of :174-184 are one matching, at the level of stack symbols. It is done tile by tile in
+// LDS while the tree is written, with no bracket stream, no s per node and no search over either
+// (they were 1.2 GB of traffic per 256 MiB JSON document and two search kernels):
+//   parse_keys_tree : key -> entry of every position, totals of every tile of FT_TILE positions
+//   pscan_*         : exclusive scan of the tile totals, depth validity
+//   parse_tree      : one wavefront per tile: match pops with pushes, write node, span, parent; the
+//                     pops and pushes left open (about 6 of 280 per tile) go to `links`
+//   link_tiles      : the open pops of all tiles against the open pushes of earlier ones
+
+constexpr int FT_TILE = WAVE * PK_IPT;  // positions per tile: one wavefront, PK_IPT per lane
+constexpr uint32_t FT_NO_NODE = 0x7FFu;      // a pop without a production (tiles have fewer nodes)
+constexpr uint32_t FT_ROOT = 0xFFFEu;        // parent of the node that fills an unowned symbol
+constexpr uint32_t FT_OPEN = 0xFFFFu;        // parent in an earlier tile
+
+// Word x of a pair entry: productions | terminal productions << 4 | pops << 8 | pushes << 12. Word
+// y: first bracket | first production << 16.
+__device__ __forceinline__ uint32_t ft_np(uint32_t f) { return f & 15u; }
+__device__ __forceinline__ uint32_t ft_nt(uint32_t f) { return (f >> 4) & 15u; }
+__device__ __forceinline__ int32_t ft_pops(uint32_t f) { return (int32_t)((f >> 8) & 15u); }
+__device__ __forceinline__ int32_t ft_pushes(uint32_t f) { return (int32_t)((f >> 12) & 15u); }
+
+// As parse_keys2, for the tree parser: a wavefront owns a tile, so that no workgroup barrier and
+// no LDS exchange stand between the lookups and the tile's totals. ET: the entry ids' type (u8 with
+// 0xFF for none below 255 entries, else u16). Tile totals in PTup: nb = records the tile leaves
+// open (pops and pushes), np, dd, mind (at most 0), nt.
+template <bool IDX8, bool BATCH, int KW, typename ET>
+__global__ void __launch_bounds__(PKK_THREADS) __attribute__((amdgpu_waves_per_eu(KW == 4 ? 8 : 1)))
+parse_keys_tree(PArgs a) {
+  extern __shared__ __align__(16) uint8_t pk_smem[];
+  __shared__ uint32_t s_ent[256];
+  if (IDX8) {
+    for (uint32_t i = threadIdx.x; i < a.index_len; i += blockDim.x) pk_smem[i] = a.index8[i];
+    for (uint32_t i = threadIdx.x; i < a.E; i += blockDim.x) s_ent[i] = a.tent[i].x;
+    __syncthreads();
+  }
+  constexpr uint32_t NONE = sizeof(ET) == 1 ? 0xFFu : 0xFFFFu;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const uint32_t W = a.q + a.k;
+  const uint64_t ntiles = pk_ntiles<BATCH>(a);
+  const uint64_t stride = (uint64_t)gridDim.x * (PKK_THREADS / WAVE);
+  bool miss = false, odd = false;
+  PosView npv;
+  uint32_t nsym[PK_IPT + KW - 1];
+  bool nraw = false;
+  uint32_t noff = 0;
+  uint64_t tile = (uint64_t)blockIdx.x * (PKK_THREADS / WAVE) + w;
+  if (tile < ntiles)
+    keys_window<BATCH, KW, FT_TILE>(a, tile, ntiles, W, npv, nsym, nraw, noff);
+  for (; tile < ntiles; tile += stride) {
+    const PosView pv = npv;
+    uint32_t sym[PK_IPT + KW - 1];
+    if (nraw) {
+      keys_symbols<KW>(nsym, noff, sym);
+    } else {
+#pragma unroll
+      for (int j = 0; j < PK_IPT + KW - 1; ++j) sym[j] = nsym[j];
+    }
+    if (tile + stride < ntiles)
+      keys_window<BATCH, KW, FT_TILE>(a, tile + stride, ntiles, W, npv, nsym, nraw, noff);
+    const int64_t lp0 = pv.p0 + (int64_t)lane * PK_IPT;  // in the document
+    // every symbol checked once, not once per window it falls into
+    uint32_t unknown = 0;
+#pragma unroll
+    for (int j = 0; j < PK_IPT + KW - 1; ++j) {
+      if (sym[j] >= a.nT) {
+        unknown |= 1u << j;
+        sym[j] = 0;
+      }
+      // tokens of the start or end terminal itself (no lexer makes them): the entries of the ends
+      // may then stand anywhere, which the tree parser does not take
+      if (!pv.kinds8 && j >= (int)a.q && j < (int)a.q + PK_IPT) {
+        const int64_t p = lp0 + j - (int64_t)a.q;
+        odd |= p > 0 && p + 1 < (int64_t)pv.P && (sym[j] == a.start_t || sym[j] == a.end_t);
+      }
+    }
+    uint32_t ids[PK_IPT], cnt = 0;  // cnt: productions | terminal productions << 16
+    int32_t d = 0, low = 0;         // depth after the lane's positions, lowest depth among them
+    bool wmiss = false;
+#pragma unroll
+    for (int i = 0; i < PK_IPT; ++i) {
+      ids[i] = NONE;
+      if (lp0 + i >= (int64_t)pv.P) continue;  // past the document: expands to nothing
+      uint32_t id;
+      if (IDX8) {
+        uint32_t di = 0;  // below 52 K
+#pragma unroll
+        for (int j = 0; j < KW; ++j)
+          if (j < (int)W) di = __umul24(di, a.nT) + sym[i + j];
+        id = pk_smem[di];
+        if (id == 0xFFu) id = 0xFFFFFFFFu;
+      } else {
+        uint64_t di = 0;
+#pragma unroll
+        for (int j = 0; j < KW; ++j)
+          if (j < (int)W) di = di * a.nT + sym[i + j];
+        id = a.index32 ? a.index32[di] : pk_hash_lookup(a, di);
+      }
+      if (id == 0xFFFFFFFFu || ((unknown >> i) & ((1u << W) - 1u)) != 0u) {
+        wmiss = true;  // expands to nothing: rejected anyway
+        continue;
+      }
+      ids[i] = id;
+      const uint32_t f = IDX8 ? s_ent[id] : a.tent[id].x;
+      cnt += ft_np(f) | (ft_nt(f) << 16);
+      low = min(low, d - ft_pops(f));
+      d += ft_pushes(f) - ft_pops(f);
+    }
+    if (BATCH) {
+      if (__ballot(wmiss) != 0ull && lane == 0) atomicOr(a.doc_flags + pv.doc, 1u);
+    } else {
+      miss |= wmiss;
+    }
+    // every slot of a tile is written, those past the document's positions with no entry
+    const uint64_t slot = tile * FT_TILE + (uint64_t)lane * PK_IPT;
+    if (sizeof(ET) == 1) {
+      reinterpret_cast<uint32_t *>(a.ent)[slot / 4] =
+          ids[0] | (ids[1] << 8) | (ids[2] << 16) | (ids[3] << 24);
+    } else {
+      *reinterpret_cast<uint2 *>(a.ent + slot) =
+          make_uint2(ids[0] | (ids[1] << 16), ids[2] | (ids[3] << 16));
+    }
+    const int32_t dincl = wave_incl_i32(d, 0, OpAdd());
+    const int32_t tlow = wave_min_i32(dincl - d + low);  // at most 0 (lane 0 starts at 0)
+    const uint32_t ctot = wave_sum_u32(cnt);             // both halves below 2^11
+    const int32_t dd = __builtin_amdgcn_readlane(dincl, WAVE - 1);
+    if (lane == 0)
+      a.tiles[tile] = PTup{dd - 2 * tlow, (int32_t)(ctot & 0xFFFFu), dd, tlow, 0,
+                           (int32_t)(ctot >> 16)};
+  }
+  if (!BATCH) {
+    if (__ballot(miss) != 0ull && lane == 0) atomicOr(a.flags, 1u);
+    if (__ballot(odd) != 0ull && lane == 0) atomicOr(a.flags + 2, 1u);
+  }
+}
+
 // Segmented tile totals: element counts (nb, np) run through all tiles, the other fields restart
 // at a tile that starts a document (batched mode).
 struct SegTup {
@@ -1916,10 +2082,22 @@ __global__ void __launch_bounds__(PSB) pscan_down(PArgs a, const SegTup *bpre) {
     if (v.f) out = PTup{ex.t.nb, ex.t.np, 0, INT32_MAX, 0, 0};
     a.pre[t] = out;
   }
+  if (a.tile_low) {
+    // the tree parser's tiles: the lowest depth of every tile, and of 64 of them
+    const int32_t low = t < ntiles ? (v.f ? 0 : ex.t.dd) + v.t.mind : INT32_MAX;
+    if (t < ntiles) a.tile_low[t] = low;
+    const int32_t low64 = wave_min_i32(low);
+    if ((threadIdx.x & (WAVE - 1)) == 0) a.tile_low1[t / WAVE] = low64;
+  }
 }
 
-// Batched parser set-up: per document, positions T + 2 when the lexer accepted it, in tiles of
-// PK_TILE; the first tile of every document (exclusive sum) and the tile count.
+// position tiles of a document of T tokens
+__device__ __forceinline__ uint32_t pk_doc_tiles(const PArgs &a, uint32_t T) {
+  return (uint32_t)(((uint64_t)T + 2 + (1u << a.tshift) - 1) >> a.tshift);
+}
+
+// Batched parser set-up: per document, positions T + 2 when the lexer accepted it, in tiles; the first
+// tile of every document (exclusive sum) and the tile count.
 __global__ void __launch_bounds__(PS_THREADS) pb_setup(PArgs a, const LexDoc *ldocs,
                                                         const uint32_t *doc_res,
                                                         uint64_t *ntiles_out) {
@@ -1934,7 +2112,7 @@ __global__ void __launch_bounds__(PS_THREADS) pb_setup(PArgs a, const LexDoc *ld
   for (uint32_t d = lo; d < hi; ++d) {
     const uint32_t ok = doc_res[2 * d];
     const uint32_t T = doc_res[2 * d + 1];
-    acc += ok ? (uint32_t)((T + 2 + PK_TILE - 1) / PK_TILE) : 0u;
+    acc += ok ? pk_doc_tiles(a, T) : 0u;
   }
   const uint32_t incl = (uint32_t)wave_incl_i32((int32_t)acc, 0, OpAdd());
   if (lane == WAVE - 1) s_w[w] = incl;
@@ -1950,7 +2128,7 @@ __global__ void __launch_bounds__(PS_THREADS) pb_setup(PArgs a, const LexDoc *ld
     pd.T = T;
     pd.lex_ok = ok;
     pd.ptile_base = base;
-    pd.ptiles = ok ? (uint32_t)((T + 2 + PK_TILE - 1) / PK_TILE) : 0u;
+    pd.ptiles = ok ? pk_doc_tiles(a, T) : 0u;
     pd.status = ok;
     pd.subst = 0;
     a.pdocs[d] = pd;
@@ -2435,6 +2613,485 @@ __device__ void parents_run(uint64_t N, const Levels &lv, uint32_t *parent, cons
   }
 }
 
+// An entry of at most 3 pops, 4 pushes and 4 productions as one row of three 16-byte words: its
+// word x, its pops, its pushes, its productions' records; row E is empty, for positions without an
+// entry.
+constexpr uint32_t FT_ROW_POPS = 3, FT_ROW_PUSHES = 4, FT_ROW_PRODS = 4;
+
+// LDS of parse_tree, in 32-bit words: the tables, then per wavefront the node records, the slots
+// (t_slots per lane and one of padding) and the open pops.
+__host__ __device__ inline uint32_t ft_table_words(bool rows, uint32_t E, uint32_t nstack,
+                                                   uint32_t nprod) {
+  return (rows ? 12 * (E + 1) : 2 * E + ((nstack + 1) & ~1u)) + 2 * ((nprod + 1) & ~1u);
+}
+__host__ __device__ inline uint32_t ft_slot_words(uint32_t slots) { return WAVE * (slots + 1); }
+
+// Step 3 of parse_tree: the tile's nodes in order, four chunks of 64 in flight. TOK: the spans of
+// its terminal nodes are in LDS (s_tok), so that no load stands among the stores (loads and stores
+// share a counter, and a load's wait would be for the stores before it too); else read from
+// starts / ends, which begin at the tile's first token.
+template <typename S, bool TOK>
+__device__ __forceinline__ void ft_write_nodes(const uint32_t *s_rec, const uint2 *s_prod,
+                                               const uint2 *s_tok, uint32_t node0, uint32_t nnode,
+                                               uint32_t docnode0, int subst, const S *starts,
+                                               const S *ends, uint32_t *parent, uint32_t *node,
+                                               S *span) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const uint32_t nend = node0 + nnode;
+  uint32_t rank = 0;  // terminal nodes of the tile before this chunk
+  constexpr int NC = 4;
+  for (uint32_t c0 = node0 & ~(uint32_t)(WAVE - 1); c0 < nend; c0 += NC * WAVE) {
+    uint32_t rec[NC], pw[NC];
+    S s0[NC], s1[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const uint32_t g = c0 + k * WAVE + lane;
+      rec[k] = s_rec[g >= node0 && g < nend ? g - node0 : 0u];
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) pw[k] = s_prod[rec[k] & 0xFFFFu].y;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const uint32_t g = c0 + k * WAVE + lane;
+      const bool term = subst && g >= node0 && g < nend && (pw[k] >> 16) != 0u;
+      const uint64_t tm = __ballot(term);
+      const uint32_t r =
+          rank + __builtin_amdgcn_mbcnt_hi((uint32_t)(tm >> 32),
+                                           __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
+      rank += (uint32_t)__popcll(tm);
+      pw[k] = term ? (ALPACC_NODE_TERMINAL | ((pw[k] >> 16) - 1u)) : (pw[k] & 0xFFFFu);
+      if (TOK) {
+        const uint2 x = s_tok[term ? r : 0u];
+        s0[k] = term ? (S)x.x : (S)0;
+        s1[k] = term ? (S)x.y : (S)0;
+      } else {
+        s0[k] = s1[k] = 0;
+        if (term) {
+          s0[k] = starts[r];
+          s1[k] = ends[r];
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+      const uint32_t g = c0 + k * WAVE + lane;
+      if (g >= node0 && g < nend) {
+        // streamed out: the tree is not read back
+        const uint32_t par = rec[k] >> 16;
+        __builtin_nontemporal_store(par == FT_ROOT ? 0u : node0 - docnode0 + par, parent + g);
+        __builtin_nontemporal_store(pw[k], node + g);
+        if (sizeof(S) == 4) {
+          __builtin_nontemporal_store((uint64_t)(uint32_t)s0[k] | ((uint64_t)(uint32_t)s1[k] << 32),
+                                      reinterpret_cast<uint64_t *>(span) + g);
+        } else {
+          span[2 * (uint64_t)g] = s0[k];
+          span[2 * (uint64_t)g + 1] = s1[k];
+        }
+      }
+    }
+  }
+}
+
+// What a wavefront loads of a tile before it works on it: the lane's entry ids, the words of the
+// tile's prefix (lanes 0-5) and totals (6-11) and its document (12), and the words of that document
+// (first token slot in lanes 0 and 1, first node in 2, whether tokens take terminal nodes in 3).
+template <typename ET>
+struct FtTile {
+  typename std::conditional<sizeof(ET) == 1, uint32_t, uint64_t>::type ids;
+  uint32_t word, doc;
+};
+
+__device__ __forceinline__ void ft_ids(uint32_t x, uint32_t (&ids)[PK_IPT]) {
+#pragma unroll
+  for (int i = 0; i < PK_IPT; ++i) ids[i] = (x >> (8 * i)) & 0xFFu;
+}
+__device__ __forceinline__ void ft_ids(uint64_t x, uint32_t (&ids)[PK_IPT]) {
+#pragma unroll
+  for (int i = 0; i < PK_IPT; ++i) ids[i] = (uint32_t)(x >> (16 * i)) & 0xFFFFu;
+}
+
+template <typename ET>
+__device__ __forceinline__ uint32_t ft_word(const FtTile<ET> &t, int k) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)t.word, k);
+}
+
+template <bool BATCH, typename ET>
+__device__ __forceinline__ void ft_load(const PArgs &a, uint64_t tile, FtTile<ET> &t) {
+  static_assert(sizeof(PTup) == 24, "the lanes below take six words");
+  const int lane = threadIdx.x & (WAVE - 1);
+  t.ids = reinterpret_cast<const decltype(t.ids) *>(a.ent)[tile * WAVE + lane];
+  const uint32_t *p = reinterpret_cast<const uint32_t *>(lane < 6 ? a.pre + tile : a.tiles + tile) +
+                      (lane < 6 ? lane : min(lane - 6, 5));
+  if (BATCH && lane == 12) p = a.ptile_doc + tile;
+  t.word = *p;
+}
+
+template <typename ET>
+__device__ __forceinline__ void ft_load_doc(const PArgs &a, FtTile<ET> &t) {
+  const PDoc *d = a.pdocs + (ft_word(t, 12) & 0x7FFFFFFFu);
+  const uint32_t *p = reinterpret_cast<const uint32_t *>(&d->tok_base);
+  const int lane = threadIdx.x & (WAVE - 1);
+  if (lane == 1) p += 1;
+  if (lane == 2) p = reinterpret_cast<const uint32_t *>(&d->node_off);
+  if (lane == 3) p = &d->subst;
+  t.doc = *p;
+}
+
+// One wavefront per tile of FT_TILE positions, PK_IPT consecutive positions per lane, in three steps.
+//  1. Every lane runs its positions' pops and pushes on a stack of its own in LDS. Stack heights
+//     are known from a scan, so a push is one store to slot (height mod t_slots) and a pop one
+//     load, with no address depending on a load; a wavefront's LDS operations keep their order.
+//     A pop below the lane's own pushes goes to the list of open pops (52% of the pops on JSON).
+//  2. An open pop at height h ends at the last earlier lane whose lowest height is at most h (that
+//     lane's slot h is its match): binary lifting over the 64 lowest heights, 64 pops at a time.
+//     The tile's pushes that stay open are found the same way, seen from past the last lane.
+//     What has no match in the tile is written to links, U open pops (the k-th one at the k-th
+//     height below the tile's start) and then the open pushes (upwards from the lowest height).
+//  3. Every node's record (production word | parent in the tile << 16) is read back in node order,
+//     64 nodes at a time, and the node, span and parent are written, coalesced.
+// The sequential walk per lane needs a few instructions per position where a cooperative search
+// over 64 elements needed 160, and the matches are read from LDS instead of written and searched.
+// 256 MiB JSON document: 415 us and link_tiles 30, against 567 + 125 + 349 us of parse_expand2,
+// bracket_match and parse_parents; 256 MiB batch of sexp documents: 510 + 41 against 805 + 105 + 588.
+// It is bound by VALU issue (about 1100 per tile, 4 wavefronts per SIMD) close to the 1.75 GB it
+// moves. On the way: entry rows and straight-line step 1 760 -> 700 us, no load among the stores
+// 700 -> 598, the next tile's words loaded ahead 598 -> 425, a larger grid 425 -> 415.
+// ROWS: the entries come as rows, and step 1 runs the four positions' operations in straight line,
+// every load issued before the first is used (an operation that a position does not have goes to
+// the lane's padding word); else (larger entries) it loops over each position's own counts, one
+// dependent load after the other.
+template <typename S, bool BATCH, typename ET, bool ROWS>
+__global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, const S *ends,
+                                                  uint32_t *node, S *span, uint32_t *parent,
+                                                  int write_nodes) {
+  extern __shared__ __align__(16) uint32_t ft_smem[];
+  uint2 *const s_prod = reinterpret_cast<uint2 *>(ft_smem);
+  uint32_t *const s_tab = ft_smem + 2 * ((a.nprod + 1) & ~1u);
+  const uint4 *const s_row = reinterpret_cast<const uint4 *>(s_tab);
+  const uint2 *const s_ent = reinterpret_cast<const uint2 *>(s_tab);
+  uint32_t *const s_br = s_tab + 2 * a.E;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const uint32_t wpb = blockDim.x / WAVE;
+  const uint32_t wave_words = a.t_rec + ft_slot_words(a.t_slots) + a.t_query;
+  uint32_t *const s_rec = ft_smem + ft_table_words(ROWS, a.E, a.nstack, a.nprod) + w * wave_words;
+  uint32_t *const s_slot = s_rec + a.t_rec;
+  uint32_t *const s_query = s_slot + ft_slot_words(a.t_slots);
+  uint32_t *const my_slot = s_slot + lane * (a.t_slots + 1);
+  const int32_t smask = (int32_t)a.t_slots - 1;
+  for (uint32_t i = threadIdx.x; i < a.nprod; i += blockDim.x) s_prod[i] = a.tprod[i];
+  if (ROWS) {
+    for (uint32_t i = threadIdx.x; i < 3 * (a.E + 1); i += blockDim.x)
+      const_cast<uint4 *>(s_row)[i] = a.trow[i];
+  } else {
+    for (uint32_t i = threadIdx.x; i < a.E; i += blockDim.x) const_cast<uint2 *>(s_ent)[i] = a.tent[i];
+    for (uint32_t i = threadIdx.x; i < a.nstack; i += blockDim.x) s_br[i] = a.tbr[i];
+  }
+  __syncthreads();
+  const uint64_t ntiles = BATCH ? (batch_elems_fit(a) ? *a.ntiles_dev : 0) : a.ntiles;
+  const uint64_t stride = (uint64_t)gridDim.x * wpb;
+  uint64_t tile = (uint64_t)blockIdx.x * wpb + w;
+  FtTile<ET> nxt;
+  if (tile < ntiles) {
+    ft_load<BATCH, ET>(a, tile, nxt);
+    if (BATCH) ft_load_doc(a, nxt);
+  }
+  for (; tile < ntiles; tile += stride) {
+    const FtTile<ET> cur = nxt;
+    uint32_t ids[PK_IPT];
+    ft_ids(cur.ids, ids);
+    const uint32_t pre_nb = ft_word(cur, 0), pre_nt = ft_word(cur, 5);
+    const uint32_t node0 = ft_word(cur, 1);                   // the tile's first node
+    const uint32_t nnode = ft_word(cur, 7), nterm = ft_word(cur, 11);
+    const int32_t tdd = (int32_t)ft_word(cur, 8);             // depth after the tile
+    const int32_t tlow = (int32_t)ft_word(cur, 9);            // lowest depth in it, at most 0
+    uint64_t tok0 = pre_nt;                                   // the tile's first token
+    uint32_t docnode0 = 0;                                    // the document's first node
+    int subst = a.subst;
+    if (BATCH) {
+      tok0 += (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)cur.doc, 0) |
+              ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)cur.doc, 1) << 32);
+      docnode0 = (uint32_t)__builtin_amdgcn_readlane((int)cur.doc, 2);
+      subst = __builtin_amdgcn_readlane((int)cur.doc, 3);
+    }
+    // the spans of the tile's terminal nodes, a contiguous run of tokens: loaded now, used in step 3
+    const bool tok_regs = sizeof(S) == 4 && write_nodes && subst && nterm <= (uint32_t)FT_TILE;
+    uint32_t ts[PK_IPT], te[PK_IPT];
+#pragma unroll
+    for (int u = 0; u < PK_IPT; ++u) {
+      ts[u] = te[u] = 0;
+      const uint32_t t = u * WAVE + lane;
+      if (tok_regs && t < nterm) {
+        ts[u] = (uint32_t)starts[tok0 + t];
+        te[u] = (uint32_t)ends[tok0 + t];
+      }
+    }
+    if (tile + stride < ntiles) ft_load<BATCH, ET>(a, tile + stride, nxt);
+    // ---- the lane's first node and depth, its lowest depth, its open pops
+    constexpr uint32_t NONE = sizeof(ET) == 1 ? 0xFFu : 0xFFFFu;
+    uint32_t f[PK_IPT], at[PK_IPT];
+    uint4 ra[PK_IPT], rb[PK_IPT], rc[PK_IPT];
+    uint32_t np = 0;
+    int32_t d = 0;
+#pragma unroll
+    for (int i = 0; i < PK_IPT; ++i) {
+      if (ROWS) {
+        const uint32_t r = 3 * (ids[i] != NONE ? ids[i] : a.E);
+        ra[i] = s_row[r];
+        rb[i] = s_row[r + 1];
+        rc[i] = s_row[r + 2];
+        f[i] = ra[i].x;
+      } else {
+        const uint2 x = ids[i] != NONE ? s_ent[ids[i]] : make_uint2(0u, 0u);
+        f[i] = x.x;
+        at[i] = x.y;
+      }
+      np += ft_np(f[i]);
+      d += ft_pushes(f[i]) - ft_pops(f[i]);
+    }
+    const int32_t d0 = wave_incl_i32(d, 0, OpAdd()) - d;  // depth before the lane, 0 before the tile
+    uint32_t nb = (uint32_t)wave_incl_i32((int32_t)np, 0, OpAdd()) - np;
+    int32_t low = d0;
+    {
+      int32_t dc = d0;
+#pragma unroll
+      for (int i = 0; i < PK_IPT; ++i) {
+        low = min(low, dc - ft_pops(f[i]));
+        dc += ft_pushes(f[i]) - ft_pops(f[i]);
+      }
+    }
+    const int32_t u = d0 - low;
+    const int32_t uincl = wave_incl_i32(u, 0, OpAdd());
+    const int32_t nopen = __builtin_amdgcn_readlane(uincl, WAVE - 1);
+    // the k-th open pop of the lane is at height d0 - 1 - k and goes to list place uincl - u + k
+    const int32_t uheight = d0 + uincl - u - 1;  // height + list place of all of them
+    // ---- step 1
+    bool mism = false;
+    if (ROWS) {
+      const uint32_t trash = a.t_rec + (uint32_t)lane * (a.t_slots + 1) + a.t_slots;  // from s_rec
+      uint32_t nbi[PK_IPT], sl[PK_IPT][FT_ROW_POPS];
+      int32_t dci[PK_IPT], lowi[PK_IPT];
+      int32_t dc = d0, lowc = d0;
+#pragma unroll
+      for (int i = 0; i < PK_IPT; ++i) {
+        const int32_t pops = ft_pops(f[i]), pushes = ft_pushes(f[i]);
+        const uint32_t npi = ft_np(f[i]);
+        const uint32_t rcw[FT_ROW_PRODS] = {rc[i].x, rc[i].y, rc[i].z, rc[i].w};
+        const uint32_t rbw[FT_ROW_PUSHES] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
+        nbi[i] = nb;
+        dci[i] = dc;
+        lowi[i] = lowc;
+#pragma unroll
+        for (uint32_t j = 0; j < FT_ROW_PRODS; ++j)
+          if (j < a.t_prods) s_rec[j < npi ? nb + j : trash] = rcw[j] + (nb << 16);
+#pragma unroll
+        for (uint32_t r = 0; r < FT_ROW_POPS; ++r) {
+          sl[i][r] = 0;
+          if (r < a.t_pops) sl[i][r] = my_slot[(dc - 1 - (int32_t)r) & smask];
+        }
+        dc -= pops;
+        lowc = min(lowc, dc);
+#pragma unroll
+        for (uint32_t l = 0; l < FT_ROW_PUSHES; ++l)
+          if (l < a.t_pushes)
+            my_slot[(int32_t)l < pushes ? (dc + (int32_t)l) & smask : (int32_t)a.t_slots] =
+                rbw[l] + (nb << 16);
+        dc += pushes;
+        nb += npi;
+      }
+#pragma unroll
+      for (int i = 0; i < PK_IPT; ++i) {
+        const int32_t pops = ft_pops(f[i]);
+        const uint32_t raw[FT_ROW_POPS] = {ra[i].y, ra[i].z, ra[i].w};
+#pragma unroll
+        for (uint32_t r = 0; r < FT_ROW_POPS; ++r) {
+          if (r < a.t_pops) {
+            const int32_t h = dci[i] - 1 - (int32_t)r;
+            const bool valid = (int32_t)r < pops;
+            const bool local = valid && h >= lowi[i];
+            const bool owned = raw[r] < 0xFFFF0000u;
+            const uint32_t nd = nbi[i] + (raw[r] >> 16);
+            mism |= local && ((sl[i][r] ^ raw[r]) & 0x7FFFu) != 0u;
+            reinterpret_cast<uint16_t *>(s_rec)[2 * (local && owned ? nd : trash) + 1] =
+                (uint16_t)(sl[i][r] >> 16);
+            const uint32_t qi = a.t_rec + ft_slot_words(a.t_slots) + (uint32_t)(uheight - h);
+            s_rec[valid && !local ? qi : trash] = (owned ? nd : FT_NO_NODE) |
+                                                  ((uint32_t)lane << 11) | ((raw[r] & 0x7FFFu) << 17);
+          }
+        }
+      }
+    } else {
+      int32_t dc = d0, lowc = d0;
+#pragma unroll
+      for (int i = 0; i < PK_IPT; ++i) {
+        const uint32_t br0 = at[i] & 0xFFFFu, pr0 = at[i] >> 16;
+        const int32_t pops = ft_pops(f[i]), pushes = ft_pushes(f[i]);
+        const uint32_t npi = ft_np(f[i]);
+        for (uint32_t j = 0; j < npi; ++j) s_rec[nb + j] = s_prod[pr0 + j].x + (nb << 16);
+        for (int32_t r = 0; r < pops; ++r) {
+          const uint32_t b = s_br[br0 + (uint32_t)r];
+          const int32_t h = dc - 1 - r;
+          const bool owned = b < 0xFFFF0000u;
+          if (h >= lowc) {
+            const uint32_t sl = my_slot[h & smask];
+            mism |= ((sl ^ b) & 0x7FFFu) != 0u;
+            if (owned)
+              reinterpret_cast<uint16_t *>(s_rec)[2 * (nb + (b >> 16)) + 1] = (uint16_t)(sl >> 16);
+          } else {
+            s_query[uheight - h] =
+                (owned ? nb + (b >> 16) : FT_NO_NODE) | ((uint32_t)lane << 11) | ((b & 0x7FFFu) << 17);
+          }
+        }
+        dc -= pops;
+        lowc = min(lowc, dc);
+        for (int32_t l = 0; l < pushes; ++l)
+          my_slot[(dc + l) & smask] = s_br[br0 + (uint32_t)(pops + l)] + (nb << 16);
+        dc += pushes;
+        nb += npi;
+      }
+    }
+    wave_lds_sync();
+    // every load above has arrived by now: waited for here, before the first store (loads and
+    // stores share a counter, and a load's wait would be for the stores before it too)
+    asm volatile("" : "+v"(nxt.ids), "+v"(nxt.word), "+v"(ts[0]), "+v"(ts[1]), "+v"(ts[2]),
+                 "+v"(ts[3]), "+v"(te[0]), "+v"(te[1]), "+v"(te[2]), "+v"(te[3]));
+    if (BATCH) ft_load_doc(a, nxt);
+    // ---- step 2
+    {
+      int32_t M[6];
+      lift_build(low, M);
+      const int32_t total = nopen + tdd - tlow;
+      for (int32_t q0 = 0; q0 < total; q0 += WAVE) {
+        const int32_t q = q0 + lane;
+        const bool pop = q < nopen;
+        const uint32_t qw = pop ? s_query[q] : 0u;
+        const int ql = pop ? (int)((qw >> 11) & 63u) : WAVE;
+        const int32_t hq = __builtin_amdgcn_ds_bpermute(ql << 2, uheight) - q;
+        const int32_t h = pop ? hq : tlow + (q - nopen);
+        const int p = lift_query(M, ql, h);
+        const uint32_t sl = p > 0 ? s_slot[(uint32_t)(p - 1) * (a.t_slots + 1) + (uint32_t)(h & smask)] : 0u;
+        if (pop) {
+          const uint32_t nd = qw & 0x7FFu;
+          uint32_t par = FT_OPEN;
+          if (p > 0) {
+            mism |= ((sl ^ (qw >> 17)) & 0x7FFFu) != 0u;
+            par = sl >> 16;
+          } else {
+            a.links[(uint64_t)pre_nb + (uint32_t)(-1 - h)] =
+                make_uint2(nd == FT_NO_NODE ? 0xFFFFFFFFu : node0 + nd, qw >> 17);
+          }
+          if (nd != FT_NO_NODE) reinterpret_cast<uint16_t *>(s_rec)[2 * nd + 1] = (uint16_t)par;
+        } else if (q < total) {
+          const uint32_t own = sl >> 16;
+          a.links[(uint64_t)pre_nb + (uint32_t)(h - 2 * tlow)] =
+              make_uint2(own == FT_ROOT ? 0u : node0 - docnode0 + own, sl & 0x7FFFu);
+        }
+      }
+    }
+    if (__ballot(mism) != 0ull && lane == 0) {
+      if (BATCH) atomicOr(a.doc_flags + (ft_word(cur, 12) & 0x7FFFFFFFu), 2u);
+      else atomicOr(a.flags, 1u);
+    }
+    wave_lds_sync();
+    if (!write_nodes) continue;
+    // ---- step 3 (the slots' LDS now holds the token spans)
+    uint2 *const s_tok = reinterpret_cast<uint2 *>(s_slot);
+    if (tok_regs) {
+#pragma unroll
+      for (int k = 0; k < PK_IPT; ++k) s_tok[k * WAVE + lane] = make_uint2(ts[k], te[k]);
+      wave_lds_sync();
+    }
+    if (tok_regs)
+      ft_write_nodes<S, true>(s_rec, s_prod, s_tok, node0, nnode, docnode0, subst, nullptr, nullptr,
+                              parent, node, span);
+    else
+      ft_write_nodes<S, false>(s_rec, s_prod, s_tok, node0, nnode, docnode0, subst,
+                               starts + tok0, ends + tok0, parent, node, span);
+    wave_lds_sync();  // the next tile writes the records again
+  }
+}
+
+// The open pops of every tile (links[pre.nb ..), the k-th one at the k-th height below the tile's
+// start) against the open pushes of earlier tiles (behind the pops, upwards from the tile's lowest
+// height): the match is in the last earlier tile whose lowest height is at most the pop's. One
+// workgroup (a column of them where there are few groups) per 64 tiles, its wavefronts taking turns
+// at their pops, 64 at a time: binary lifting over the 64 lowest heights, and a climb of the 64-ary
+// min hierarchy over all tiles for those that leave them. Documents as they come leave 6 pops open
+// per tile and nearly all end inside the 64 tiles; deep nesting leaves up to some 500 per tile, most
+// of them ending far away, which is what the many wavefronts per group are for.
+constexpr int LINK_THREADS = 512;
+template <bool BATCH>
+__global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv, uint32_t *parent,
+                                                           int write_nodes) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const uint64_t ntiles = BATCH ? (batch_elems_fit(a) ? *a.ntiles_dev : 0) : a.ntiles;
+  const uint64_t ngroups = (ntiles + WAVE - 1) / WAVE;
+  const int32_t w0 = (int32_t)(blockIdx.y * LINK_THREADS + threadIdx.x / WAVE * WAVE);
+  const int32_t wstep = (int32_t)(gridDim.y * LINK_THREADS);
+  for (uint64_t grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
+    const uint64_t t = grp * WAVE + lane;
+    int32_t d0 = 0, low = INT32_MAX, u = 0, v = 0, off = 0;
+    uint32_t doc = 0;
+    if (t < ntiles) {
+      const PTup pre = a.pre[t], tot = a.tiles[t];
+      d0 = pre.dd;
+      u = -tot.mind;
+      low = d0 - u;
+      v = tot.dd + u;
+      off = pre.nb;
+      if (BATCH) doc = a.ptile_doc[t] & 0x7FFFFFFFu;
+    }
+    int32_t M[6];
+    lift_build(low, M);
+    const int32_t uincl = wave_incl_i32(u, 0, OpAdd());
+    const int32_t total = __builtin_amdgcn_readlane(uincl, WAVE - 1);
+    for (int32_t q0 = w0; q0 < total; q0 += wstep) {
+      const int32_t q = q0 + lane;
+      const bool pop = q < total;
+      // the tile of pop q: the number of tiles whose pops all come before it
+      int l4 = 0;
+#pragma unroll
+      for (int step = WAVE / 2; step >= 1; step >>= 1)
+        if (__builtin_amdgcn_ds_bpermute(l4 + 4 * (step - 1), uincl) <= q) l4 += 4 * step;
+      if (!pop) l4 = 0;
+      const int l = l4 >> 2;
+      const int32_t k = q - (__builtin_amdgcn_ds_bpermute(l4, uincl) - __builtin_amdgcn_ds_bpermute(l4, u));
+      const int32_t h = __builtin_amdgcn_ds_bpermute(l4, d0) - 1 - k;
+      const uint32_t lnk = (uint32_t)__builtin_amdgcn_ds_bpermute(l4, off) + (uint32_t)k;
+      const int p = lift_query(M, l, h);
+      const int s4 = (p - 1) << 2;
+      uint32_t soff = (uint32_t)__builtin_amdgcn_ds_bpermute(s4, off);
+      int32_t su = __builtin_amdgcn_ds_bpermute(s4, u), sv = __builtin_amdgcn_ds_bpermute(s4, v);
+      int32_t slow = __builtin_amdgcn_ds_bpermute(s4, low);
+      const uint32_t qdoc = BATCH ? (uint32_t)__builtin_amdgcn_ds_bpermute(l4, (int)doc) : 0u;
+      if (pop) {
+        const uint2 me = a.links[lnk];
+        bool found = p > 0;
+        if (!found) {
+          const int64_t far = prev_le_far(lv, grp, h);
+          if (far >= 0) {
+            const PTup pre = a.pre[far], tot = a.tiles[far];
+            su = -tot.mind;
+            sv = tot.dd + su;
+            slow = pre.dd - su;
+            soff = (uint32_t)pre.nb;
+            found = true;
+          }
+        }
+        // (in a rejected document the found tile may be another document's: no push at h then)
+        found = found && h - slow < sv;
+        uint2 at = make_uint2(0u, 0xFFFFFFFFu);
+        if (found) at = a.links[(uint64_t)soff + (uint32_t)(su + (h - slow))];
+        if (at.y != me.y) {
+          if (BATCH) atomicOr(a.doc_flags + qdoc, 2u);
+          else atomicOr(a.flags, 1u);
+        }
+        if (write_nodes && me.x != 0xFFFFFFFFu) parent[me.x] = at.x;
+      }
+    }
+  }
+}
+
 inline unsigned grid_for(uint64_t n, unsigned block, unsigned cap = 1u << 16) {
   uint64_t g = (n + block - 1) / block;
   if (g == 0) g = 1;
@@ -2504,11 +3161,14 @@ enum Stage {
   S_PARSE_EXPAND,   // parse_expand2
   S_BRACKET_MATCH,  // bracket_match
   S_PARSE_PARENTS,  // parse_parents
+  S_PARSE_TREE,     // parse_tree (grammars that take it; the three above otherwise)
+  S_LINK_TILES,     // the min levels over the tiles and link_tiles
   NSTAGE
 };
 static const char *kStageNames[NSTAGE] = {"lex_reduce",    "lex_scan",     "lex_emit",
                                           "parse",         "parse_keys",   "parse_expand",
-                                          "bracket_match", "parse_parents"};
+                                          "bracket_match", "parse_parents", "parse_tree",
+                                          "link_tiles"};
 
 struct alpacc_ctx {
   int device = 0;
@@ -2544,6 +3204,14 @@ struct alpacc_ctx {
   uint32_t *d_ecan = nullptr;  // per entry: trailing lefts | leading rights << 8 | brackets between << 16
   uint32_t max_nb = 0, max_np = 0;
   size_t nstackw = 0, nprodw = 0;
+  // the tree parser (see parse_tree): whether the grammar's entries take it, its tables, its LDS
+  bool tree_ok = false;
+  uint2 *d_tent = nullptr, *d_tprod = nullptr;
+  uint32_t *d_tbr = nullptr;
+  uint4 *d_trow = nullptr;  // (only when every entry fits a row)
+  uint32_t t_rec = 0, t_slots = 0, t_query = 0, t_prods = 0, t_pops = 0, t_pushes = 0;
+  unsigned tree_threads = 0, tree_bpc = 1;
+  size_t tree_lds = 0;
   // scratch (grow-only)
   std::vector<std::pair<void *, size_t>> scratch;
   uint64_t table_bytes = 0;  // device bytes of the uploaded tables
@@ -2586,7 +3254,7 @@ struct alpacc_ctx {
   void prof_drop(int s) {
     rec[s] = false;
     if (s == S_PARSE)
-      for (int i = S_PARSE_KEYS; i <= S_PARSE_PARENTS; ++i) rec[i] = false;
+      for (int i = S_PARSE_KEYS; i < NSTAGE; ++i) rec[i] = false;
   }
   // element counts of the last call: tokens, positions, brackets, productions
   uint64_t last_counts[4] = {0, 0, 0, 0};
@@ -2678,6 +3346,9 @@ enum BufId {
   B_TILE_REC,
   B_CHUNKS,
   B_CHUNK_BASE,
+  B_LINKS,
+  B_TILE_LOW,
+  B_TILE_LOW1,
 };
 
 template <typename T>
@@ -3158,6 +3829,92 @@ void parse_args_init(alpacc_ctx *ctx, PArgs &a) {
   a.ecan = ctx->d_ecan;
   a.nstack = (uint32_t)ctx->nstackw;
   a.nprod = (uint32_t)ctx->nprodw;
+  a.tshift = 10;
+}
+
+// Switches the arguments to the tree parser's tiles and tables; false when an arena for
+// ntiles_max tiles cannot be allocated.
+bool parse_args_tree(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max) {
+  a.tshift = 8;
+  a.tent = ctx->d_tent;
+  a.tbr = ctx->d_tbr;
+  a.tprod = ctx->d_tprod;
+  a.t_rec = ctx->t_rec;
+  a.t_slots = ctx->t_slots;
+  a.t_query = ctx->t_query;
+  a.trow = ctx->d_trow;
+  a.t_prods = ctx->t_prods;
+  a.t_pops = ctx->t_pops;
+  a.t_pushes = ctx->t_pushes;
+  // (whole scan blocks: pscan_down writes the minima of all its wavefronts)
+  const uint64_t nb = (ntiles_max + PSB - 1) / PSB + 1;
+  a.tile_low = (int32_t *)ctx->buf(B_TILE_LOW, (ntiles_max + 16) * sizeof(int32_t));
+  a.tile_low1 = (int32_t *)ctx->buf(B_TILE_LOW1, (nb * (PSB / WAVE) + 16) * sizeof(int32_t));
+  return a.tile_low && a.tile_low1;
+}
+
+constexpr unsigned TREE_WAVES = 16;
+
+// tiles of `positions` key positions, of the tree parser or the element-level one
+inline uint64_t tile_count(bool tree, uint64_t positions) {
+  return tree ? (positions + FT_TILE - 1) / FT_TILE : (positions + PK_TILE - 1) / PK_TILE;
+}
+
+// The key lookups of the tree parser.
+template <bool BATCH>
+void launch_keys_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles_max, hipStream_t st) {
+  constexpr uint64_t wpb = PKK_THREADS / WAVE;
+  const unsigned g = (unsigned)std::max<uint64_t>(
+      1, std::min<uint64_t>((ntiles_max + wpb - 1) / wpb,
+                            (uint64_t)std::max(1, ctx->cus) * ctx->keys_bpc));
+  const bool small_w = ctx->q + ctx->k <= 4, ent8 = ctx->E < 255;
+  if (ctx->d_index8 && small_w)
+    parse_keys_tree<true, BATCH, 4, uint8_t><<<g, PKK_THREADS, ctx->index_len, st>>>(a);
+  else if (ctx->d_index8)
+    parse_keys_tree<true, BATCH, PK_MAXW, uint8_t><<<g, PKK_THREADS, ctx->index_len, st>>>(a);
+  else if (small_w && ent8)
+    parse_keys_tree<false, BATCH, 4, uint8_t><<<g, PKK_THREADS, 0, st>>>(a);
+  else if (ent8)
+    parse_keys_tree<false, BATCH, PK_MAXW, uint8_t><<<g, PKK_THREADS, 0, st>>>(a);
+  else if (small_w)
+    parse_keys_tree<false, BATCH, 4, uint16_t><<<g, PKK_THREADS, 0, st>>>(a);
+  else
+    parse_keys_tree<false, BATCH, PK_MAXW, uint16_t><<<g, PKK_THREADS, 0, st>>>(a);
+}
+
+// The tree of about ntiles tiles by workgroups striding over them (each wavefront loads its next
+// tile's words while it works on one): up to TREE_WAVES times as many as the GPU holds at once, which
+// measured 510 us on a 256 MiB batch of sexp documents and 416 us on a 256 MiB JSON document against
+// 586 and 426 us with once (the wavefronts then write and compute in step).
+template <typename S, bool BATCH>
+void launch_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const S *starts, const S *ends,
+                 uint32_t *node, S *span, uint32_t *parent, int write_nodes, hipStream_t st) {
+  const uint64_t wpb = ctx->tree_threads / WAVE;
+  const unsigned g = (unsigned)std::max<uint64_t>(
+      1, std::min<uint64_t>((ntiles + wpb - 1) / wpb, (uint64_t)std::max(1, ctx->cus) * ctx->tree_bpc * TREE_WAVES));
+  auto run = [&](auto kernel) {
+    kernel<<<g, ctx->tree_threads, ctx->tree_lds, st>>>(a, starts, ends, node, span, parent,
+                                                        write_nodes);
+  };
+  if (ctx->E < 255 && ctx->d_trow) run(parse_tree<S, BATCH, uint8_t, true>);
+  else if (ctx->E < 255) run(parse_tree<S, BATCH, uint8_t, false>);
+  else if (ctx->d_trow) run(parse_tree<S, BATCH, uint16_t, true>);
+  else run(parse_tree<S, BATCH, uint16_t, false>);
+}
+
+// The links between the tiles of a tree (lv: the min hierarchy over the tiles' lowest depths).
+template <bool BATCH>
+int launch_links(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const Levels &lv,
+                 uint32_t *parent, int write_nodes, hipStream_t st) {
+  Levels none;
+  none.nlev = 0;
+  const int rc = fill_levels(ctx, lv, none, st);
+  if (rc) return rc;
+  const unsigned groups = grid_for(ntiles, WAVE, 1u << 14);
+  const dim3 grid(groups, std::min(32u, std::max(1u, 1024u / groups)));
+  link_tiles<BATCH><<<grid, LINK_THREADS, 0, st>>>(a, lv, parent, write_nodes);
+  ctx->launches++;
+  return 0;
 }
 
 // keys, tile totals and the tile scan (ntiles_max: tiles to cover, the device count in batch)
@@ -3169,7 +3926,9 @@ int parse_phase1(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max, hipStream_t st,
   const unsigned kgrid =
       (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(nsuper, (uint64_t)std::max(1, ctx->cus) * ctx->keys_bpc));
   const bool small_w = ctx->q + ctx->k <= 4;
-  if (ctx->d_index8 && small_w)
+  if (a.tshift == 8)
+    launch_keys_tree<BATCH>(ctx, a, ntiles_max, st);
+  else if (ctx->d_index8 && small_w)
     parse_keys2<true, BATCH, 4><<<kgrid, PKK_THREADS, ctx->index_len, st>>>(a);
   else if (ctx->d_index8)
     parse_keys2<true, BATCH, PK_MAXW><<<kgrid, PKK_THREADS, ctx->index_len, st>>>(a);
@@ -3255,7 +4014,7 @@ template <typename S>
 int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *ends,
                      uint64_t T, uint32_t *parent, uint32_t *node, S *span, uint64_t cap,
                      uint64_t *num_nodes, hipStream_t st, bool productions_only = false,
-                     bool lexed = false, const uint8_t *kinds8 = nullptr) {
+                     bool lexed = false, const uint8_t *kinds8 = nullptr, bool may_tree = true) {
   if (!ctx->has_parser) {
     ctx->err = "bundle has no parser";
     return ALPACC_ERR_NO_PARSER;
@@ -3267,9 +4026,12 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
     ctx->err = "token stream too long for 32-bit element counts";
     return ALPACC_ERR_ARG;
   }
-  uint64_t ntiles = (P + PK_TILE - 1) / PK_TILE;
+  const bool tree = may_tree && ctx->tree_ok;
+  uint64_t ntiles = tile_count(tree, P);
   uint32_t *small = (uint32_t *)ctx->buf(B_SMALL, 64 * sizeof(uint32_t));
-  uint16_t *ent = (uint16_t *)ctx->buf(B_ENT, (ntiles * PK_TILE + 8) * sizeof(uint16_t));
+  uint16_t *ent = (uint16_t *)ctx->buf(
+      B_ENT, tree && ctx->E < 255 ? ntiles * FT_TILE + 16
+                                  : (ntiles * (tree ? FT_TILE : PK_TILE) + 8) * sizeof(uint16_t));
   PTup *tiles = (PTup *)ctx->buf(B_PTILES, (ntiles + 1) * sizeof(PTup));
   PTup *pre = (PTup *)ctx->buf(B_PPRE, (ntiles + 1) * sizeof(PTup));
   if (!small || !ent || !tiles || !pre) {
@@ -3291,6 +4053,10 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
   a.total = total;
   a.flags = flags;
   a.ntiles = ntiles;
+  if (tree && !parse_args_tree(ctx, a, ntiles)) {
+    ctx->err = "scratch allocation failed";
+    return ALPACC_ERR_HIP;
+  }
   ctx->prof_begin(S_PARSE, st);
   clear_u32<<<1, 64, 0, st>>>(flags, 4);
   ctx->launches++;
@@ -3313,13 +4079,16 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
       ctx->err = "token stream too long for 32-bit element counts";
       return ALPACC_ERR_ARG;
     }
-    ntiles = (P + PK_TILE - 1) / PK_TILE;
+    ntiles = tile_count(tree, P);
     a.T = T;
     a.P = P;
     a.ntiles = ntiles;
     a.T_dev = nullptr;  // from here on the counts are known on the host
   }
   const uint32_t *hs = ctx->h_small + sh;
+  if (tree && hs[2])  // start or end terminals among the tokens: the tree parser does not take them
+    return run_parse_tokens<S>(ctx, kinds, starts, ends, T, parent, node, span, cap, num_nodes, st,
+                               productions_only, false, kinds8, false);
   if (hs[0]) return ALPACC_REJECT;  // a missing pair (to_keys, parser.fut:235-240)
   PTup tot;
   memcpy(&tot, hs + 8, sizeof(PTup));
@@ -3334,17 +4103,36 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
   ctx->last_counts[3] = N;
   *num_nodes = N;
   const int write_nodes = N <= cap ? 1 : 0;
-  ElemBufs e;
-  rc = elem_bufs(ctx, B, N, e, st);
-  if (rc) return rc;
-  const size_t xlds = px_lds_bytes(ctx->nstackw, ctx->nprodw, ctx->E);
-  ctx->prof_begin(S_PARSE_EXPAND, st);
-  parse_expand2<S, false><<<(unsigned)ntiles, PK_THREADS, xlds, st>>>(
-      a, starts, ends, e.depth, e.br, e.dl1, e.sx, e.sl1, node, span, write_nodes);
-  ctx->prof_end(S_PARSE_EXPAND, st);
-  ctx->launches++;
-  CK(hipGetLastError());
-  rc = run_search<false>(ctx, a, e, B, write_nodes ? N : 0, parent, flags, st);
+  if (tree) {
+    a.links = (uint2 *)ctx->buf(B_LINKS, (B + 16) * sizeof(uint2));
+    if (!a.links) {
+      ctx->err = "scratch allocation failed";
+      return ALPACC_ERR_HIP;
+    }
+    Levels lv;
+    rc = plan_levels(ctx, a.tile_low, a.tile_low1, ntiles, lv, B_LEVELS);
+    if (rc) return rc;
+    ctx->prof_begin(S_PARSE_TREE, st);
+    launch_tree<S, false>(ctx, a, ntiles, starts, ends, node, span, parent, write_nodes, st);
+    ctx->prof_end(S_PARSE_TREE, st);
+    ctx->launches++;
+    ctx->prof_begin(S_LINK_TILES, st);
+    rc = launch_links<false>(ctx, a, ntiles, lv, parent, write_nodes, st);
+    ctx->prof_end(S_LINK_TILES, st);
+    CK(hipGetLastError());
+  } else {
+    ElemBufs e;
+    rc = elem_bufs(ctx, B, N, e, st);
+    if (rc) return rc;
+    const size_t xlds = px_lds_bytes(ctx->nstackw, ctx->nprodw, ctx->E);
+    ctx->prof_begin(S_PARSE_EXPAND, st);
+    parse_expand2<S, false><<<(unsigned)ntiles, PK_THREADS, xlds, st>>>(
+        a, starts, ends, e.depth, e.br, e.dl1, e.sx, e.sl1, node, span, write_nodes);
+    ctx->prof_end(S_PARSE_EXPAND, st);
+    ctx->launches++;
+    CK(hipGetLastError());
+    rc = run_search<false>(ctx, a, e, B, write_nodes ? N : 0, parent, flags, st);
+  }
   if (rc) return rc;
   ctx->prof_end(S_PARSE, st);
   if (!write_nodes || N == 0) {
@@ -3409,6 +4197,8 @@ struct ParseBatchPlan {
   uint32_t *h_words;  // pinned copy of the result words small[0 .. 32)
   size_t xlds;
   unsigned search_bs, search_cap;
+  int tree;      // the tree parser
+  Levels lvt;    // its min hierarchy over the tiles
 };
 
 int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets,
@@ -3419,10 +4209,12 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   uint64_t nbytes = 0, tiles_max = 0;
   for (uint32_t d = 0; d < ndocs; ++d) {
     nbytes += lengths[d];
-    tiles_max += (lengths[d] + 3 + PK_TILE - 1) / PK_TILE;
+    tiles_max += tile_count(ctx->tree_ok, lengths[d] + 3);
   }
+  pl.tree = ctx->tree_ok ? 1 : 0;
+  const uint64_t tpos = pl.tree ? FT_TILE : PK_TILE;
   const uint64_t tslots = nbytes + ndocs + 1;
-  if (tslots >= (1ull << 32) - 1 || tiles_max >= (1ull << 32) / PK_TILE) {
+  if (tslots >= (1ull << 32) - 1 || tiles_max >= (1ull << 32) / tpos) {
     ctx->err = "batch too large: token slots and key positions must stay below 2^32";
     return ALPACC_ERR_ARG;
   }
@@ -3443,25 +4235,35 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   PDoc *pdocs = (PDoc *)ctx->buf(B_PDOCS, (ndocs + 1) * sizeof(PDoc));
   uint32_t *doc_flags = (uint32_t *)ctx->buf(B_DOC_FLAGS, (ndocs + 1) * 4);
   uint32_t *ptile_doc = (uint32_t *)ctx->buf(B_PTILE_DOC, (tiles_max + 1) * 4);
-  uint16_t *ent = (uint16_t *)ctx->buf(B_ENT, (tiles_max * PK_TILE + 8) * sizeof(uint16_t));
+  uint16_t *ent = (uint16_t *)ctx->buf(
+      B_ENT, pl.tree && ctx->E < 255 ? tiles_max * tpos + 16
+                                     : (tiles_max * tpos + 8) * sizeof(uint16_t));
   PTup *tiles = (PTup *)ctx->buf(B_PTILES, (tiles_max + 1) * sizeof(PTup));
   PTup *pre = (PTup *)ctx->buf(B_PPRE, (tiles_max + 1) * sizeof(PTup));
   pl.d_results = (alpacc_doc_result *)ctx->buf(B_RESULTS, (ndocs + 1) * sizeof(alpacc_doc_result));
   const uint64_t nbs = std::max<uint64_t>(1, (tiles_max + PSB - 1) / PSB);
   pl.btot = (SegTup *)ctx->buf(B_BTOT, (nbs + 1) * sizeof(SegTup));
-  pl.e.depth = (int32_t *)ctx->buf(B_DEPTH, (bcap + 16) * sizeof(int32_t));
-  pl.e.br = (uint16_t *)ctx->buf(B_BR, (bcap + 16) * sizeof(uint16_t));
-  pl.e.dl1 = (int32_t *)ctx->buf(B_DL1, (nbc + 16) * sizeof(int32_t));
-  pl.e.sx = (int32_t *)ctx->buf(B_SX, (ncap + 16) * sizeof(int32_t));
-  pl.e.sl1 = (int32_t *)ctx->buf(B_SL1, (npc + 16) * sizeof(int32_t));
-  uint32_t *chunk_doc = (uint32_t *)ctx->buf(B_CHUNK_DOC, (npc + 2) * 4);
-  uint32_t *chunk_base = (uint32_t *)ctx->buf(B_CHUNK_BASE, (npc + 2) * 4);
+  uint32_t *chunk_doc = nullptr, *chunk_base = nullptr;
+  uint2 *links = nullptr;
+  bool elems = true;
+  if (pl.tree) {
+    links = (uint2 *)ctx->buf(B_LINKS, (bcap + 16) * sizeof(uint2));
+    elems = links != nullptr;
+  } else {
+    pl.e.depth = (int32_t *)ctx->buf(B_DEPTH, (bcap + 16) * sizeof(int32_t));
+    pl.e.br = (uint16_t *)ctx->buf(B_BR, (bcap + 16) * sizeof(uint16_t));
+    pl.e.dl1 = (int32_t *)ctx->buf(B_DL1, (nbc + 16) * sizeof(int32_t));
+    pl.e.sx = (int32_t *)ctx->buf(B_SX, (ncap + 16) * sizeof(int32_t));
+    pl.e.sl1 = (int32_t *)ctx->buf(B_SL1, (npc + 16) * sizeof(int32_t));
+    chunk_doc = (uint32_t *)ctx->buf(B_CHUNK_DOC, (npc + 2) * 4);
+    chunk_base = (uint32_t *)ctx->buf(B_CHUNK_BASE, (npc + 2) * 4);
+    elems = pl.e.depth && pl.e.br && pl.e.dl1 && pl.e.sx && pl.e.sl1 && chunk_doc && chunk_base;
+  }
   const size_t docs_bytes = ((ndocs + 1) * sizeof(LexDoc) + 255) & ~(size_t)255;
   const size_t res_bytes = ((ndocs + 1) * sizeof(alpacc_doc_result) + 255) & ~(size_t)255;
   uint8_t *stg = ctx->stage(docs_bytes + res_bytes + 256, st);
   if (!kinds || !starts || !ends || !doc_res || !pdocs || !doc_flags || !ptile_doc || !ent ||
-      !tiles || !pre || !pl.d_results || !pl.btot || !pl.e.depth || !pl.e.br || !pl.e.dl1 ||
-      !pl.e.sx || !pl.e.sl1 || !chunk_doc || !chunk_base || !stg) {
+      !tiles || !pre || !pl.d_results || !pl.btot || !elems || !stg) {
     ctx->err = "scratch allocation failed";
     return ALPACC_ERR_HIP;
   }
@@ -3490,14 +4292,19 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   a.chunk_base = chunk_base;
   a.bcap = bcap;
   a.ncap = ncap;
+  a.links = links;
+  if (pl.tree && !parse_args_tree(ctx, a, tiles_max)) {
+    ctx->err = "scratch allocation failed";
+    return ALPACC_ERR_HIP;
+  }
   pl.tiles_max = tiles_max;
-  // parse_expand2's grid: the tiles of an estimate of the key positions (p_per_byte of the input,
-  // grown to what calls needed; the bound from the input bytes is several times the count), and
-  // a striding pass over any tiles past it
+  // the grid of parse_tree / parse_expand2: the tiles of an estimate of the key positions
+  // (p_per_byte of the input, grown to what calls needed; the bound from the input bytes is several
+  // times the count); parse_tree strides over any tiles past it, parse_expand2 has a striding pass
   pl.tiles_est = std::min<uint64_t>(
-      tiles_max, (uint64_t)(ctx->p_per_byte * (double)nbytes) / PK_TILE + ndocs + 1);
+      tiles_max, (uint64_t)(ctx->p_per_byte * (double)nbytes) / tpos + ndocs + 1);
   pl.stride_blocks =
-      pl.tiles_est < tiles_max ? (unsigned)std::max(1, ctx->cus) * 4 : 0u;
+      !pl.tree && pl.tiles_est < tiles_max ? (unsigned)std::max(1, ctx->cus) * 4 : 0u;
   pl.nbc = nbc;
   pl.npc = npc;
   pl.parent = parent;
@@ -3506,13 +4313,27 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   pl.starts = starts;
   pl.ends = ends;
   pl.lvb.nlev = pl.lvs.nlev = 0;
-  if (bcap > 0) rc = plan_levels(ctx, pl.e.depth, pl.e.dl1, bcap, pl.lvb, B_LEVELS);
-  if (!rc && ncap > 0) rc = plan_levels(ctx, pl.e.sx, pl.e.sl1, ncap, pl.lvs, B_LEVELS_S);
+  if (pl.tree)
+    rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, pl.lvt, B_LEVELS);
+  else if (bcap > 0)
+    rc = plan_levels(ctx, pl.e.depth, pl.e.dl1, bcap, pl.lvb, B_LEVELS);
+  if (!rc && ncap > 0 && !pl.tree) rc = plan_levels(ctx, pl.e.sx, pl.e.sl1, ncap, pl.lvs, B_LEVELS_S);
   if (rc) return rc;
   pl.xlds = px_lds_bytes(ctx->nstackw, ctx->nprodw, ctx->E);
   pl.search_bs = ctx->search_bs;
   pl.search_cap = ctx->search_cap;
   return 0;
+}
+
+// The end of a planned call: the documents' results, and their copies to the host.
+void finish_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t st) {
+  const uint32_t ndocs = pl.lx.ndocs;
+  pb_finish<<<(ndocs + 255) / 256, 256, 0, st>>>(pl.a, pl.d_results);
+  ctx->launches++;
+  ctx->prof_end(S_PARSE, st);
+  (void)hipMemcpyAsync(pl.h_results, pl.d_results, ndocs * sizeof(alpacc_doc_result),
+                       hipMemcpyDeviceToHost, st);
+  (void)hipMemcpyAsync(pl.h_words, pl.lx.small, 32 * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
 }
 
 // Queues the planned call on `st`: copies and kernels only (no allocation, no synchronisation).
@@ -3527,6 +4348,19 @@ void enqueue_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t 
   ctx->launches += 2;
   (void)parse_phase1<true>(ctx, a, pl.tiles_max, st, pl.btot);
   pb_docs<<<(ndocs + 255) / 256, 256, 0, st>>>(a);
+  if (pl.tree) {
+    ctx->launches++;
+    ctx->prof_begin(S_PARSE_TREE, st);
+    launch_tree<uint32_t, true>(ctx, a, pl.tiles_est, pl.starts, pl.ends, pl.node, pl.span,
+                                pl.parent, 1, st);
+    ctx->prof_end(S_PARSE_TREE, st);
+    ctx->launches++;
+    ctx->prof_begin(S_LINK_TILES, st);
+    (void)launch_links<true>(ctx, a, pl.tiles_est, pl.lvt, pl.parent, 1, st);
+    ctx->prof_end(S_LINK_TILES, st);
+    finish_parse_batch(ctx, pl, st);
+    return;
+  }
   elem_init<<<grid_for(std::max(pl.nbc, pl.npc) + 16, 256, 4096), 256, 0, st>>>(
       pl.e.dl1, pl.nbc + 16, pl.e.sl1, pl.npc + 16);
   ctx->launches += 2;
@@ -3561,12 +4395,7 @@ void enqueue_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t 
     ctx->prof_end(S_PARSE_PARENTS, st);
     ctx->launches++;
   }
-  pb_finish<<<(ndocs + 255) / 256, 256, 0, st>>>(a, pl.d_results);
-  ctx->launches++;
-  ctx->prof_end(S_PARSE, st);
-  (void)hipMemcpyAsync(pl.h_results, pl.d_results, ndocs * sizeof(alpacc_doc_result),
-                       hipMemcpyDeviceToHost, st);
-  (void)hipMemcpyAsync(pl.h_words, pl.lx.small, 32 * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
+  finish_parse_batch(ctx, pl, st);
 }
 
 // Runs a planned call on `st`: queued directly, or through a HIP graph. graph_mode 1 captures
@@ -3633,10 +4462,11 @@ int run_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offset
   *total_nodes = 0;
   uint64_t nbytes = 0;
   for (uint32_t d = 0; d < ndocs; ++d) nbytes += lengths[d];
-  // brackets: at most max_nb per key position (T + 2 <= length + 2 per document)
+  // brackets (the tree parser: open ends, fewer): at most max_nb per key position (T + 2 <= length + 2 per document)
   const uint64_t b_bound = (nbytes + 2ull * ndocs) * std::max<uint32_t>(ctx->max_nb, 1);
   uint64_t bcap = std::min<uint64_t>(
-      b_bound, std::max<uint64_t>(4096, (uint64_t)(ctx->b_per_byte * (double)nbytes)));
+      b_bound, std::max<uint64_t>(ctx->tree_ok ? 256 : 4096,
+                                  (uint64_t)(ctx->b_per_byte * (double)nbytes)));
   for (int attempt = 0; attempt < 2; ++attempt) {
     ParseBatchPlan pl;
     int rc = plan_parse_batch(ctx, d_in, offsets, lengths, ndocs, parent, node, span, cap, bcap,
@@ -3663,7 +4493,8 @@ int run_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offset
     const uint64_t B = (uint32_t)tot.nb, N = (uint32_t)tot.np;
     *total_nodes = N;
     ctx->last_counts[0] = 0;
-    ctx->last_counts[1] = ntiles * PK_TILE;
+    const uint64_t positions = ntiles << pl.a.tshift;
+    ctx->last_counts[1] = positions;
     ctx->last_counts[2] = B;
     ctx->last_counts[3] = N;
     if (N > cap) {
@@ -3672,7 +4503,7 @@ int run_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offset
     }
     if (ntiles > pl.tiles_est && nbytes)  // the striding pass ran: widen the estimate
       ctx->p_per_byte = std::min(
-          4.0, std::max(ctx->p_per_byte, 1.25 * (double)(ntiles * PK_TILE) / (double)nbytes));
+          4.0, std::max(ctx->p_per_byte, 1.25 * (double)positions / (double)nbytes));
     if (B > bcap) {  // the first pass wrote nothing: size the brackets for this batch
       bcap = B + B / 8 + 4096;
       if (nbytes) ctx->b_per_byte = std::max(ctx->b_per_byte, (double)bcap / (double)nbytes);
@@ -3874,6 +4705,129 @@ bool build_parser_tables(alpacc_ctx *ctx, const alpacc_tables *t, std::string &e
   return err.empty();
 }
 
+// The tables of the tree parser (see parse_tree), for grammars whose pair entries it takes: every
+// entry's brackets are pops, then pushes, its productions fill the popped symbols in order and
+// leave the pushed ones open (simulated by arity), and only the entries of the start and end
+// terminals' own positions push or pop symbols that no production owns or fills. Then bracket depth
+// and s = exscan(arity - 1) rise and fall together behind the first position, so the previous
+// smaller-or-equal s of a production (its parent) is found in the entry that holds the left
+// bracket matching the production's right bracket. Other grammars keep the element-level kernels.
+bool build_tree_tables(alpacc_ctx *ctx, const alpacc_tables *t, std::string &err) {
+  constexpr uint32_t MAX_RUN = 8, MAX_PROD = 7;
+  const uint32_t E = t->num_pair_entries;
+  std::vector<uint2> ent(E), prod;
+  std::vector<uint32_t> br;
+  std::vector<uint8_t> ends(E, 0);  // 1: pushes unowned symbols, 2: pops symbols nothing fills
+  uint32_t max_np = 1, max_pops = 1, max_pushes = 1;
+  bool any_ends = false;
+  for (uint32_t e = 0; e < E; ++e) {
+    const uint32_t *e4 = t->pair_entry + 4ull * e;
+    const uint32_t nb = e4[1] - e4[0], np = e4[3] - e4[2];
+    uint32_t pops = 0;
+    while (pops < nb && !(t->stacks[e4[0] + pops] & 0x8000u)) ++pops;
+    const uint32_t pushes = nb - pops;
+    for (uint32_t s = e4[0] + pops; s < e4[1]; ++s)
+      if (!(t->stacks[s] & 0x8000u)) return true;
+    if (np > MAX_PROD || pops > MAX_RUN || pushes > MAX_RUN) return true;
+    std::vector<uint32_t> open;                  // owners of the symbols left open
+    std::vector<uint32_t> fills(pops, 0xFFFFu);  // production that fills every popped symbol
+    uint32_t filled = 0, nt = 0;
+    const uint32_t pst = (uint32_t)prod.size();
+    for (uint32_t j = 0; j < np; ++j) {
+      const uint16_t pr = t->productions[e4[2] + j];
+      const int32_t ar = t->arities[pr], term = t->prod_to_terminal[pr];
+      if (ar < 0 || ar > 1024) return true;
+      uint32_t own = 0;
+      if (!open.empty()) {
+        own = open.back();
+        open.pop_back();
+      } else {
+        if (filled == pops) return true;
+        fills[filled++] = j;
+      }
+      open.insert(open.end(), (size_t)ar, j);
+      nt += term >= 0 ? 1 : 0;
+      prod.push_back(make_uint2((pst + j) | (own << 16), (uint32_t)pr | ((uint32_t)(term + 1) << 16)));
+    }
+    if (np == 0 && pops == 0 && pushes > 0) ends[e] = 1;
+    else if (pushes == 0 && open.empty() && filled < pops) ends[e] = 2;
+    else if (filled != pops || open.size() != pushes) return true;
+    any_ends |= ends[e] != 0;
+    const uint32_t sst = (uint32_t)br.size();
+    for (uint32_t r = 0; r < pops; ++r)
+      br.push_back((uint32_t)(t->stacks[e4[0] + r] & 0x7FFFu) | (fills[r] << 16));
+    for (uint32_t l = 0; l < pushes; ++l)
+      br.push_back((uint32_t)(t->stacks[e4[0] + pops + l] & 0x7FFFu) |
+                   ((ends[e] == 1 ? FT_ROOT : open[l]) << 16));
+    ent[e] = make_uint2(np | (nt << 4) | (pops << 8) | (pushes << 12), sst | (pst << 16));
+    max_np = std::max(max_np, np);
+    max_pops = std::max(max_pops, pops);
+    max_pushes = std::max(max_pushes, pushes);
+  }
+  if (any_ends) {
+    // only at the start and end terminals' own positions: the window's symbol at lookback
+    if (t->k == 0) return true;
+    uint64_t div = 1;
+    for (uint32_t j = 0; j + 1 < t->k; ++j) div *= t->num_terminals;
+    auto misplaced = [&](uint64_t key, uint32_t e) {
+      const uint64_t sym = key / div % t->num_terminals;
+      return (ends[e] == 1 && sym != t->start_terminal) || (ends[e] == 2 && sym != t->end_terminal);
+    };
+    for (uint64_t i = 0; i < t->pair_index_len; ++i)
+      if (t->pair_index[i] != 0xFFFFFFFFu && misplaced(i, t->pair_index[i])) return true;
+    for (uint64_t i = 0; i < t->pair_hash_len; ++i)
+      if (t->pair_hash_keys[i] != ~0ull && misplaced(t->pair_hash_keys[i], t->pair_hash_vals[i]))
+        return true;
+    // and no lexer token is one of them
+    if (t->num_endos > 0)
+      for (uint64_t i = 0; i < (uint64_t)t->num_states * t->num_classes; ++i) {
+        const uint32_t lab = t->dfa_step[i] >> 9;
+        if (lab == t->start_terminal || lab == t->end_terminal) return true;
+      }
+  }
+  uint32_t slots = 8;
+  while (slots < PK_IPT * max_pushes) slots *= 2;
+  ctx->t_rec = FT_TILE * max_np;
+  ctx->t_slots = slots;
+  ctx->t_query = FT_TILE * max_pops;
+  if (br.empty()) br.push_back(0);
+  if (prod.empty()) prod.push_back(make_uint2(0, 0));
+  // (the array lengths are those of build_parser_tables: a.nstack, a.nprod)
+  const bool rows = max_pops <= FT_ROW_POPS && max_pushes <= FT_ROW_PUSHES && max_np <= FT_ROW_PRODS;
+  const size_t tables = 4ull * ft_table_words(rows, E, (uint32_t)br.size(), (uint32_t)prod.size());
+  const size_t wave = 4ull * (ctx->t_rec + ft_slot_words(slots) + ctx->t_query);
+  unsigned waves = 4;
+  while (waves > 1 && tables + waves * wave > (64u << 10)) waves /= 2;
+  if (tables + waves * wave > (64u << 10)) return true;
+  ctx->t_prods = max_np;
+  ctx->t_pops = max_pops;
+  ctx->t_pushes = max_pushes;
+  ctx->tree_threads = waves * WAVE;
+  ctx->tree_lds = tables + waves * wave;
+  // workgroups a CU holds: by their LDS, and 4 wavefronts per SIMD by their registers
+  ctx->tree_bpc = (unsigned)std::max<size_t>(1, std::min<size_t>((160u << 10) / ctx->tree_lds, 16 / waves));
+  if (rows) {
+    std::vector<uint32_t> row(12ull * (E + 1), 0);
+    for (uint32_t e = 0; e < E; ++e) {
+      const uint32_t f = ent[e].x, sst = ent[e].y & 0xFFFFu, pst = ent[e].y >> 16;
+      const uint32_t np = f & 15u, pops = (f >> 8) & 15u, pushes = (f >> 12) & 15u;
+      uint32_t *r = row.data() + 12ull * e;
+      r[0] = f;
+      for (uint32_t i = 0; i < pops; ++i) r[1 + i] = br[sst + i];
+      for (uint32_t i = 0; i < pushes; ++i) r[4 + i] = br[sst + pops + i];
+      for (uint32_t i = 0; i < np; ++i) r[8 + i] = prod[pst + i].x;
+    }
+    ctx->d_trow = (uint4 *)upload(row.data(), row.size(), err);
+    ctx->table_bytes += row.size() * 4;
+  }
+  ctx->d_tent = upload(ent.data(), ent.size(), err);
+  ctx->d_tbr = upload(br.data(), br.size(), err);
+  ctx->d_tprod = upload(prod.data(), prod.size(), err);
+  ctx->table_bytes += ent.size() * 8 + br.size() * 4 + prod.size() * 8;
+  ctx->tree_ok = err.empty();
+  return err.empty();
+}
+
 }  // namespace
 
 extern "C" {
@@ -3961,7 +4915,7 @@ alpacc_ctx *alpacc_create(const alpacc_tables *t, int device) {
     ctx->end_t = t->end_terminal;
     ctx->empty_t = t->empty_terminal;
     ctx->E = t->num_pair_entries;
-    if (!build_parser_tables(ctx, t, err)) {
+    if (!build_parser_tables(ctx, t, err) || !build_tree_tables(ctx, t, err)) {
       alpacc_destroy(ctx);
       return nullptr;
     }
@@ -3977,7 +4931,8 @@ void alpacc_destroy(alpacc_ctx *ctx) {
   void *tabs[] = {ctx->d_cls,    ctx->d_step,     ctx->d_comp,   ctx->d_apply,
                   ctx->d_walk,   ctx->d_pair_index, ctx->d_index8,
                   ctx->d_hkeys,  ctx->d_hvals,
-                  ctx->d_einfo,  ctx->d_stackw,   ctx->d_prodw,  ctx->d_ecan};
+                  ctx->d_einfo,  ctx->d_stackw,   ctx->d_prodw,  ctx->d_ecan,
+                  ctx->d_tent,   ctx->d_tbr,      ctx->d_tprod,  ctx->d_trow};
   for (void *p : tabs)
     if (p) (void)hipFree(p);
   if (ctx->h_small) (void)hipHostFree(ctx->h_small);

@@ -428,6 +428,9 @@ def main():
     #   lex_reduce    : n                       reads the document
     #   lex_emit      : n + 12 T                reads it again, writes (kind, start, end) u32; inside
     #                   n + 9 T                 alpacc_parse the kinds are bytes
+    #   parse_tree    : P + 8 T + 16 N          pair entries in (a byte each); token spans in; parent,
+    #                                           node word and span per node out. Grammars that the
+    #                                           tree parser does not take run the next three instead:
     #   parse_expand  : 2 P + 8 T + 6 B + 16 N  pair entries in; token spans gathered; depth + symbol
     #                                           per bracket; s, node word and span per node out
     #   bracket_match : 6 B                     depth + symbol per bracket
@@ -437,7 +440,7 @@ def main():
     alg = {"lex_reduce": n, "lex_emit": n + (9 if args.workload == "parse" else 12) * T}
     if args.workload == "parse":
         alg.update({"parse_expand": 2 * P + 8 * T + 6 * B + 16 * N_, "bracket_match": 6 * B,
-                    "parse_parents": 8 * N_})
+                    "parse_parents": 8 * N_, "parse_tree": P + 8 * T + 16 * N_})
     dom = max((k for k in alg if stage_ms.get(k, 0) > 0), key=lambda k: stage_ms[k])
     dom_gbs = alg[dom] / (stage_ms[dom] / 1000.0) / 1e9 if alg[dom] else 0.0
     roof = {"bound": "hbm", "kernel": dom, "achieved": round(dom_gbs, 1),
@@ -447,7 +450,8 @@ def main():
     # workload (scaled by a plain copy of known size); only for the workload they were taken on
     tpath = os.path.join(ROOT, "profiles", "json_lex_parse_256MiB.traffic.json")
     kernel_of = {"lex_reduce": "lex_reduce", "lex_emit": "lex_emit", "parse_expand": "parse_expand2",
-                 "bracket_match": "bracket_match", "parse_parents": "parse_parents"}
+                 "bracket_match": "bracket_match", "parse_parents": "parse_parents",
+                 "parse_tree": "parse_tree"}
     if (args.workload == "parse" and args.mib == 256 and args.seed == 42
             and os.path.exists(tpath)):
         tk = json.load(open(tpath))["kernels"].get(kernel_of.get(dom, ""))
