@@ -167,6 +167,9 @@ struct LexArgs {
   uint32_t *tile_counter;     // [1] dynamic count-tile index
   uint64_t *st_count;         // [num_ctiles] look-back words of the count scan
   uint32_t *result;           // [0] accept, [1] tokens, [2] timeout flag
+  uint32_t *clear;            // the 16 words (counter, results, parser flags) that lex_reduce clears
+  uint32_t timeout0;          // what it sets the timeout flag to (testing hook)
+  uint32_t *host_result;      // when set: pinned host copy of result
   // chunked mode (the reference's chunk loop, lexer.fut:144-172): `in` is the virtual string in
   // which every chunk [j*chunk, min(j*chunk + chunk + 1, n_orig)) is laid end to end, so the byte
   // shared by two neighbouring chunks appears twice.
@@ -362,6 +365,10 @@ lex_reduce(LexArgs p) {
   const int lane = threadIdx.x & (WAVE - 1);
   const uint32_t wpb = blockDim.x / WAVE;
   const uint32_t stride = gridDim.x * wpb;
+  // the words that lex_emit and the parser count in and look back at
+  const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint32_t i = gt; i < p.num_ctiles; i += gridDim.x * blockDim.x) p.st_count[i] = 0;
+  if (gt < 16) p.clear[gt] = gt == (uint32_t)(p.result + 2 - p.clear) ? p.timeout0 : 0u;
   // two tiles per iteration: their table-lookup chains are independent and overlap
   for (uint32_t t0 = blockIdx.x * wpb + threadIdx.x / WAVE; t0 < p.num_tiles; t0 += 2 * stride) {
     uint32_t tile[2] = {t0, t0 + stride};
@@ -585,6 +592,8 @@ __global__ void lex_tile_docs(LexArgs p) {
     const_cast<uint4 *>(p.tile_rec)[doc.tile_base + i] =
         make_uint4((uint32_t)doc.offset, (uint32_t)(doc.offset >> 32), (uint32_t)doc.len, i);
   }
+  // its result, which an empty document keeps
+  if (threadIdx.x < 2) p.doc_res[2 * blockIdx.x + threadIdx.x] = 0;
   // and the document's scan chunks (first wave tile, tile count)
   for (uint32_t c = threadIdx.x; c < doc.nchunks; c += blockDim.x)
     const_cast<uint2 *>(p.chunks)[doc.chunk_base + c] =
@@ -623,7 +632,10 @@ __device__ void lookback_count(const LexArgs &p, uint32_t tile, int lane, uint32
         __builtin_amdgcn_s_sleep(2);
       }
       if (given_up) {
-        if (lane == 0) st_relaxed(p.result + 2, 1u);
+        if (lane == 0) {
+          st_relaxed(p.result + 2, 1u);
+          if (p.host_result) p.host_result[2] = 1u;
+        }
         cnt = 0;
         last = -1;
         return;
@@ -1013,6 +1025,10 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     } else {
       p.result[1] = total;
       p.result[0] = acc_end;
+      if (p.host_result) {
+        p.host_result[1] = total;
+        p.host_result[0] = acc_end;
+      }
     }
   }
 }
@@ -1495,7 +1511,8 @@ struct PArgs {
   PTup *tiles;             // [ntiles] tile totals
   PTup *pre;               // [ntiles] exclusive prefixes (parse_pscan)
   PTup *total;             // [1]
-  uint32_t *flags;         // [0] reject
+  uint32_t *flags;         // [0] reject, [1] overflow, [2] misplaced ends, [3] build the tree
+  uint32_t *hw;            // single document by the tree parser: pinned host words (tree_verdict)
   uint64_t ntiles;
   int subst;               // single document: terminal productions pair up with the tokens
   uint32_t tshift;         // log2 of the positions per tile: 10 (PK_TILE) or 8 (FT_TILE)
@@ -1525,6 +1542,11 @@ struct PArgs {
   uint64_t bcap, ncap;
 };
 
+// The tiles the tree kernels process: none when the batch, or the document's open ends, exceed the
+// scratch, or when the document is rejected already.
+template <bool BATCH>
+__device__ __forceinline__ uint64_t tree_tiles(const PArgs &a);
+
 // Batched mode: the brackets / productions the element kernels process: the grand totals, or
 // none when they exceed the scratch capacities (then nothing is written).
 __device__ __forceinline__ bool batch_elems_fit(const PArgs &a) {
@@ -1533,6 +1555,17 @@ __device__ __forceinline__ bool batch_elems_fit(const PArgs &a) {
          (uint64_t)t.np <= a.ncap;
 }
 
+
+template <>
+__device__ __forceinline__ uint64_t tree_tiles<true>(const PArgs &a) {
+  return batch_elems_fit(a) ? *a.ntiles_dev : 0;
+}
+template <>
+__device__ __forceinline__ uint64_t tree_tiles<false>(const PArgs &a) {
+  if (!a.flags[3] || (uint64_t)(uint32_t)a.total->nb > a.bcap) return 0;
+  const uint64_t P = a.T_dev ? std::min<uint64_t>(*a.T_dev, a.T) + 2 : a.P;
+  return (P + (1ull << a.tshift) - 1) >> a.tshift;
+}
 
 struct PDoc {
   uint64_t tok_base;    // first token slot of the document (batched lexer layout)
@@ -2034,6 +2067,31 @@ __global__ void __launch_bounds__(PSB) pscan_reduce(PArgs a, SegTup *btot) {
   if (threadIdx.x == 0) btot[blockIdx.x] = total;
 }
 
+// What a single document's tree kernels go by, written where the grand total is: whether the tree is
+// to be built at all (lexer verdict, missing pairs, misplaced end terminals, the depth check of
+// depths, parser.fut:153-166), and the words the host decides by, straight to pinned host memory:
+// [0] lexer verdict, [1] tokens, [2] time-out, [4] missing pair, [5] overflow, [6] misplaced ends,
+// [8..13] grand total ([7], a bracket mismatch, comes from the tree kernels).
+__device__ __forceinline__ void tree_verdict(const PArgs &a, const PTup &t, bool over) {
+  a.flags[1] = over ? 1u : 0u;
+  if (!a.hw) return;
+  const uint32_t acc = a.T_dev ? a.T_dev[-1] : 1u, tmo = a.T_dev ? ld_relaxed(a.T_dev + 1) : 0u;
+  const uint32_t miss = ld_relaxed(a.flags), odd = ld_relaxed(a.flags + 2);
+  a.flags[3] = acc && !tmo && !miss && !odd && !over && t.mind >= 0 && t.dd == 0 ? 1u : 0u;
+  a.hw[0] = acc;
+  a.hw[1] = a.T_dev ? a.T_dev[0] : 0u;
+  a.hw[2] = tmo;
+  a.hw[4] = miss;
+  a.hw[5] = over ? 1u : 0u;
+  a.hw[6] = odd;
+  a.hw[8] = (uint32_t)t.nb;
+  a.hw[9] = (uint32_t)t.np;
+  a.hw[10] = (uint32_t)t.dd;
+  a.hw[11] = (uint32_t)t.mind;
+  a.hw[12] = (uint32_t)t.ds;
+  a.hw[13] = (uint32_t)t.nt;
+}
+
 __global__ void __launch_bounds__(PSB) pscan_top(PArgs a, SegTup *btot, uint64_t nblocks_max) {
   __shared__ SegTup s_w[PSB / WAVE];
   __shared__ SegTup s_carry;
@@ -2075,7 +2133,7 @@ __global__ void __launch_bounds__(PSB) pscan_top(PArgs a, SegTup *btot, uint64_t
   __syncthreads();
   if (threadIdx.x == 0) {
     *a.total = s_carry.t;
-    if (s_elems[0] >= (1ull << 31) || s_elems[1] >= (1ull << 31)) a.flags[1] = 1u;
+    tree_verdict(a, s_carry.t, s_elems[0] >= (1ull << 31) || s_elems[1] >= (1ull << 31));
   }
 }
 
@@ -2100,6 +2158,62 @@ __global__ void __launch_bounds__(PSB) pscan_down(PArgs a, const SegTup *bpre) {
     const int32_t low64 = wave_min_i32(low);
     if ((threadIdx.x & (WAVE - 1)) == 0) a.tile_low1[t / WAVE] = low64;
   }
+}
+
+// The tile scan in one workgroup, each thread over a run of consecutive tiles: in place of
+// pscan_reduce, pscan_top and pscan_down where the tiles are few (up to PSCAN_ONE_MAX), whose time is
+// their launches.
+constexpr uint64_t PSCAN_ONE_MAX = 16 * PSB;
+
+template <bool BATCH>
+__global__ void __launch_bounds__(PSB) pscan_one(PArgs a) {
+  __shared__ SegTup s_w[PSB / WAVE];
+  __shared__ unsigned long long s_elems[2];
+  const uint64_t ntiles = pk_ntiles<BATCH>(a);
+  const uint64_t run = (ntiles + PSB - 1) / PSB;
+  const uint64_t lo = std::min<uint64_t>(ntiles, threadIdx.x * run);
+  const uint64_t hi = std::min<uint64_t>(ntiles, lo + run);
+  if (threadIdx.x < 2) s_elems[threadIdx.x] = 0ull;
+  SegTup acc{ptup_id(), 0};
+  unsigned long long mine_b = 0ull, mine_p = 0ull;
+  for (uint64_t t = lo; t < hi; ++t) {
+    const SegTup v{a.tiles[t], tile_reset<BATCH>(a, t)};
+    mine_b += (uint32_t)v.t.nb;
+    mine_p += (uint32_t)v.t.np;
+    acc = seg_op(acc, v);
+  }
+  SegTup total;
+  SegTup ex = seg_block_excl(acc, s_w, total);
+  for (uint64_t t = lo; t < hi; ++t) {
+    const SegTup v{a.tiles[t], tile_reset<BATCH>(a, t)};
+    PTup out = ex.t;
+    if (v.f) out = PTup{ex.t.nb, ex.t.np, 0, INT32_MAX, 0, 0};
+    a.pre[t] = out;
+    if (a.tile_low) a.tile_low[t] = out.dd + v.t.mind;
+    ex = seg_op(ex, v);
+  }
+  // a total of brackets or productions of 2^31 or more, as in pscan_top
+#pragma unroll
+  for (int d = WAVE / 2; d >= 1; d >>= 1) {
+    mine_b += __shfl_xor(mine_b, d, WAVE);
+    mine_p += __shfl_xor(mine_p, d, WAVE);
+  }
+  if ((threadIdx.x & (WAVE - 1)) == 0) {
+    atomicAdd(&s_elems[0], mine_b);
+    atomicAdd(&s_elems[1], mine_p);
+  }
+  __threadfence_block();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *a.total = total.t;
+    tree_verdict(a, total.t, s_elems[0] >= (1ull << 31) || s_elems[1] >= (1ull << 31));
+  }
+  if (a.tile_low)
+    for (uint64_t g = threadIdx.x / WAVE; g * WAVE < ntiles; g += PSB / WAVE) {
+      const uint64_t t = g * WAVE + (threadIdx.x & (WAVE - 1));
+      const int32_t m = wave_min_i32(t < ntiles ? a.tile_low[t] : INT32_MAX);
+      if ((threadIdx.x & (WAVE - 1)) == 0) a.tile_low1[g] = m;
+    }
 }
 
 // position tiles of a document of T tokens
@@ -2773,8 +2887,7 @@ __device__ __forceinline__ void ft_load_doc(const PArgs &a, FtTile<ET> &t) {
 // dependent load after the other.
 template <typename S, bool BATCH, typename ET, bool ROWS>
 __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, const S *ends,
-                                                  uint32_t *node, S *span, uint32_t *parent,
-                                                  int write_nodes) {
+                                                  uint32_t *node, S *span, uint32_t *parent) {
   extern __shared__ __align__(16) uint32_t ft_smem[];
   uint2 *const s_prod = reinterpret_cast<uint2 *>(ft_smem);
   uint32_t *const s_tab = ft_smem + 2 * ((a.nprod + 1) & ~1u);
@@ -2799,7 +2912,12 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
     for (uint32_t i = threadIdx.x; i < a.nstack; i += blockDim.x) s_br[i] = a.tbr[i];
   }
   __syncthreads();
-  const uint64_t ntiles = BATCH ? (batch_elems_fit(a) ? *a.ntiles_dev : 0) : a.ntiles;
+  const uint64_t ntiles = tree_tiles<BATCH>(a);
+  // single document: nodes go out when they fit the caller's arrays, and tokens take terminal nodes
+  // when there are as many of both
+  const bool write_nodes = BATCH || (uint64_t)(uint32_t)a.total->np <= a.ncap;
+  const int subst1 =
+      !BATCH && a.subst && (uint32_t)a.total->nt == (a.T_dev ? *a.T_dev : (uint32_t)a.T) ? 1 : 0;
   const uint64_t stride = (uint64_t)gridDim.x * wpb;
   uint64_t tile = (uint64_t)blockIdx.x * wpb + w;
   FtTile<ET> nxt;
@@ -2818,7 +2936,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
     const int32_t tlow = (int32_t)ft_word(cur, 9);            // lowest depth in it, at most 0
     uint64_t tok0 = pre_nt;                                   // the tile's first token
     uint32_t docnode0 = 0;                                    // the document's first node
-    int subst = a.subst;
+    int subst = subst1;
     if (BATCH) {
       tok0 += (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)cur.doc, 0) |
               ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)cur.doc, 1) << 32);
@@ -3001,7 +3119,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
     }
     if (__ballot(mism) != 0ull && lane == 0) {
       if (BATCH) atomicOr(a.doc_flags + (ft_word(cur, 12) & 0x7FFFFFFFu), 2u);
-      else atomicOr(a.flags, 1u);
+      else a.hw[7] = 1u;
     }
     wave_lds_sync();
     if (!write_nodes) continue;
@@ -3032,10 +3150,11 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
 // of them ending far away, which is what the many wavefronts per group are for.
 constexpr int LINK_THREADS = 512;
 template <bool BATCH>
-__global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv, uint32_t *parent,
-                                                           int write_nodes) {
+__global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv,
+                                                           uint32_t *parent) {
   const int lane = threadIdx.x & (WAVE - 1);
-  const uint64_t ntiles = BATCH ? (batch_elems_fit(a) ? *a.ntiles_dev : 0) : a.ntiles;
+  const uint64_t ntiles = tree_tiles<BATCH>(a);
+  const bool write_nodes = BATCH || (uint64_t)(uint32_t)a.total->np <= a.ncap;
   const uint64_t ngroups = (ntiles + WAVE - 1) / WAVE;
   const int32_t w0 = (int32_t)(blockIdx.y * LINK_THREADS + threadIdx.x / WAVE * WAVE);
   const int32_t wstep = (int32_t)(gridDim.y * LINK_THREADS);
@@ -3095,7 +3214,7 @@ __global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv, u
         if (found) at = a.links[(uint64_t)soff + (uint32_t)(su + (h - slow))];
         if (at.y != me.y) {
           if (BATCH) atomicOr(a.doc_flags + qdoc, 2u);
-          else atomicOr(a.flags, 1u);
+          else a.hw[7] = 1u;
         }
         if (write_nodes && me.x != 0xFFFFFFFFu) parent[me.x] = at.x;
       }
@@ -3589,9 +3708,6 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     ctx->err = "scratch allocation failed";
     return ALPACC_ERR_HIP;
   }
-  clear_u32<<<1, 64, 0, st>>>(small, 16);
-  if (ctx->force_timeout) set_u32<<<1, 1, 0, st>>>(small + 6, 1u);
-  clear_u32<<<grid_for(2 * ctiles, 256), 256, 0, st>>>((uint32_t *)st_count, 2 * ctiles);
   LexArgs a;
   a.in = d_in;
   a.n = n;
@@ -3620,6 +3736,12 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   a.tile_counter = small;
   a.st_count = st_count;
   a.result = small + 4;
+  a.clear = small;
+  a.timeout0 = ctx->force_timeout ? 1u : 0u;
+  // the verdict goes straight to pinned host words: a copy queued behind the kernels is one more
+  // launch and about 8 us
+  a.host_result = sync ? ctx->h_small : nullptr;
+  ctx->h_small[2] = a.timeout0;
   a.chunk = (uint32_t)chunk;
   a.nchunks = (uint32_t)K;
   a.n_orig = n_orig;
@@ -3652,10 +3774,9 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     launch_lex_emit<false, false>(ctx->dfa_lds, (unsigned)ctiles, a, st);
   }
   ctx->prof_end(S_LEX_EMIT, st);
-  ctx->launches += 7;
+  ctx->launches += 5;
   CK(hipGetLastError());
   if (!sync) return ALPACC_ACCEPT;
-  CK(hipMemcpyAsync(ctx->h_small, small + 4, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
   CK(hipStreamSynchronize(st));
   if (ctx->h_small[2]) {
     ctx->err = "lexer look-back did not complete";
@@ -3764,6 +3885,8 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
   a.num_ctiles = (uint32_t)ctiles;
   a.tile_counter = pl.small;
   a.result = pl.small + 4;
+  a.clear = pl.small;
+  a.timeout0 = ctx->force_timeout ? 1u : 0u;
   a.docs = pl.d_docs;
   a.ndocs = ndocs;
   a.doc_res = doc_res;
@@ -3775,13 +3898,15 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
 
 void enqueue_lex_batch(alpacc_ctx *ctx, const LexBatchPlan &pl, hipStream_t st) {
   (void)hipMemcpyAsync(pl.d_docs, pl.h_docs, pl.ndocs * sizeof(LexDoc), hipMemcpyHostToDevice, st);
-  clear_u32<<<grid_for(2 * (uint64_t)pl.ndocs, 256), 256, 0, st>>>(pl.doc_res, 2 * (uint64_t)pl.ndocs);
-  clear_u32<<<1, 64, 0, st>>>(pl.small, 16);
-  if (pl.force_timeout) set_u32<<<1, 1, 0, st>>>(pl.small + 6, 1u);
-  ctx->launches += 2;
-  if (pl.tiles == 0) return;
+  if (pl.tiles == 0) {
+    clear_u32<<<grid_for(2 * (uint64_t)pl.ndocs, 256), 256, 0, st>>>(pl.doc_res,
+                                                                     2 * (uint64_t)pl.ndocs);
+    clear_u32<<<1, 64, 0, st>>>(pl.small, 16);
+    if (pl.force_timeout) set_u32<<<1, 1, 0, st>>>(pl.small + 6, 1u);
+    ctx->launches += 2;
+    return;
+  }
   const LexArgs &a = pl.a;
-  clear_u32<<<grid_for(2 * pl.ctiles, 256), 256, 0, st>>>((uint32_t *)a.st_count, 2 * pl.ctiles);
   lex_tile_docs<<<pl.ndocs, 256, 0, st>>>(a);
   ctx->prof_begin(S_LEX_REDUCE, st);
   launch_lex_reduce<true>(pl.lex_tab, pl.lex_blocks, pl.lex_lds, a, st);
@@ -3794,7 +3919,7 @@ void enqueue_lex_batch(alpacc_ctx *ctx, const LexBatchPlan &pl, hipStream_t st) 
   ctx->prof_begin(S_LEX_EMIT, st);
   launch_lex_emit<false, true>(pl.dfa_lds != 0, (unsigned)pl.ctiles, a, st);
   ctx->prof_end(S_LEX_EMIT, st);
-  ctx->launches += 7;
+  ctx->launches += 6;
 }
 
 // The batched lexer queued on `st` (descriptors through the context's pinned staging);
@@ -3899,13 +4024,12 @@ void launch_keys_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles_max, hipS
 // 586 and 426 us with once (the wavefronts then write and compute in step).
 template <typename S, bool BATCH>
 void launch_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const S *starts, const S *ends,
-                 uint32_t *node, S *span, uint32_t *parent, int write_nodes, hipStream_t st) {
+                 uint32_t *node, S *span, uint32_t *parent, hipStream_t st) {
   const uint64_t wpb = ctx->tree_threads / WAVE;
   const unsigned g = (unsigned)std::max<uint64_t>(
       1, std::min<uint64_t>((ntiles + wpb - 1) / wpb, (uint64_t)std::max(1, ctx->cus) * ctx->tree_bpc * TREE_WAVES));
   auto run = [&](auto kernel) {
-    kernel<<<g, ctx->tree_threads, ctx->tree_lds, st>>>(a, starts, ends, node, span, parent,
-                                                        write_nodes);
+    kernel<<<g, ctx->tree_threads, ctx->tree_lds, st>>>(a, starts, ends, node, span, parent);
   };
   if (ctx->E < 255 && ctx->d_trow) run(parse_tree<S, BATCH, uint8_t, true>);
   else if (ctx->E < 255) run(parse_tree<S, BATCH, uint8_t, false>);
@@ -3916,14 +4040,14 @@ void launch_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const S *star
 // The links between the tiles of a tree (lv: the min hierarchy over the tiles' lowest depths).
 template <bool BATCH>
 int launch_links(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const Levels &lv,
-                 uint32_t *parent, int write_nodes, hipStream_t st) {
+                 uint32_t *parent, hipStream_t st) {
   Levels none;
   none.nlev = 0;
   const int rc = fill_levels(ctx, lv, none, st);
   if (rc) return rc;
   const unsigned groups = grid_for(ntiles, WAVE, 1u << 14);
   const dim3 grid(groups, std::min(32u, std::max(1u, 1024u / groups)));
-  link_tiles<BATCH><<<grid, LINK_THREADS, 0, st>>>(a, lv, parent, write_nodes);
+  link_tiles<BATCH><<<grid, LINK_THREADS, 0, st>>>(a, lv, parent);
   ctx->launches++;
   return 0;
 }
@@ -3931,7 +4055,7 @@ int launch_links(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const Levels 
 // keys, tile totals and the tile scan (ntiles_max: tiles to cover, the device count in batch)
 template <bool BATCH>
 int parse_phase1(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max, hipStream_t st,
-                 SegTup *btot = nullptr) {
+                 SegTup *btot = nullptr, uint64_t ntiles_est = ~0ull) {
   ctx->prof_begin(S_PARSE_KEYS, st);
   const uint64_t nsuper = (ntiles_max + PKK_TILES - 1) / PKK_TILES;
   const unsigned kgrid =
@@ -3947,6 +4071,13 @@ int parse_phase1(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max, hipStream_t st,
     parse_keys2<false, BATCH, 4><<<kgrid, PKK_THREADS, 0, st>>>(a);
   else
     parse_keys2<false, BATCH, PK_MAXW><<<kgrid, PKK_THREADS, 0, st>>>(a);
+  if (std::min(ntiles_est, ntiles_max) <= PSCAN_ONE_MAX) {
+    pscan_one<BATCH><<<1, PSB, 0, st>>>(a);
+    ctx->prof_end(S_PARSE_KEYS, st);
+    ctx->launches += 2;
+    CK(hipGetLastError());
+    return 0;
+  }
   const uint64_t nb = std::max<uint64_t>(1, (ntiles_max + PSB - 1) / PSB);
   if (!btot) btot = (SegTup *)ctx->buf(B_BTOT, (nb + 1) * sizeof(SegTup));
   if (!btot) {
@@ -4014,6 +4145,140 @@ int run_search(alpacc_ctx *ctx, const PArgs &a, const ElemBufs &e, uint64_t B, u
   return 0;
 }
 
+template <typename S>
+int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *ends,
+                     uint64_t T, uint32_t *parent, uint32_t *node, S *span, uint64_t cap,
+                     uint64_t *num_nodes, hipStream_t st, bool productions_only = false,
+                     bool lexed = false, const uint8_t *kinds8 = nullptr, bool may_tree = true);
+
+// run_parse_tokens for the tree parser: one queue, with one host synchronisation at its end. The
+// kernels size themselves by the device's counts (tree_verdict), the records of open ends by an
+// estimate from T (b_per_byte, grown to what calls needed): a call that needs more runs the tree
+// kernels again. The synchronisation in the middle that sized the element scratch cost about 25 us.
+template <typename S>
+int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *ends, uint64_t T,
+             uint32_t *parent, uint32_t *node, S *span, uint64_t cap, uint64_t *num_nodes,
+             hipStream_t st, bool productions_only, bool lexed, const uint8_t *kinds8) {
+  *num_nodes = 0;
+  uint64_t P = T + 2;
+  const uint64_t elem_max = (uint64_t)std::max(ctx->max_nb, ctx->max_np);
+  if (!lexed && P * elem_max >= (1ull << 31)) {
+    ctx->err = "token stream too long for 32-bit element counts";
+    return ALPACC_ERR_ARG;
+  }
+  // tiles: the bound, and (T a bound: bytes) the estimate that the grids are sized by
+  const uint64_t tiles_max = tile_count(true, P);
+  const uint64_t tiles_est =
+      lexed ? std::min<uint64_t>(tiles_max, (uint64_t)(ctx->p_per_byte * (double)T) / FT_TILE + 1)
+            : tiles_max;
+  uint64_t bcap = std::min<uint64_t>(P * std::max<uint32_t>(ctx->max_nb, 1),
+                                     std::max<uint64_t>(256, (uint64_t)(ctx->b_per_byte * (double)T)));
+  uint32_t *small = (uint32_t *)ctx->buf(B_SMALL, 64 * sizeof(uint32_t));
+  uint16_t *ent = (uint16_t *)ctx->buf(B_ENT, ctx->E < 255 ? tiles_max * FT_TILE + 16
+                                                           : (tiles_max * FT_TILE + 8) * sizeof(uint16_t));
+  PTup *tiles = (PTup *)ctx->buf(B_PTILES, (tiles_max + 1) * sizeof(PTup));
+  PTup *pre = (PTup *)ctx->buf(B_PPRE, (tiles_max + 1) * sizeof(PTup));
+  uint2 *links = (uint2 *)ctx->buf(B_LINKS, (bcap + 16) * sizeof(uint2));
+  PArgs a;
+  parse_args_init(ctx, a);
+  if (!small || !ent || !tiles || !pre || !links || !parse_args_tree(ctx, a, tiles_max)) {
+    ctx->err = "scratch allocation failed";
+    return ALPACC_ERR_HIP;
+  }
+  volatile uint32_t *hw = ctx->h_small;
+  a.kinds = kinds;
+  a.kinds8 = kinds8;
+  a.T = T;
+  a.P = P;
+  a.T_dev = lexed ? small + 5 : nullptr;  // the lexer's result words: verdict, count, time-out
+  a.ent = ent;
+  a.tiles = tiles;
+  a.pre = pre;
+  a.total = reinterpret_cast<PTup *>(small + 16);
+  a.flags = small + 8;  // (cleared with the lexer's words)
+  a.hw = ctx->h_small;
+  a.ntiles = tiles_max;
+  a.links = links;
+  a.bcap = bcap;
+  a.ncap = std::min<uint64_t>(cap, 1ull << 31);
+  a.subst = productions_only ? 0 : 1;
+  Levels lv;
+  int rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, lv, B_LEVELS);
+  if (rc) return rc;
+  hw[7] = 0;
+  ctx->prof_begin(S_PARSE, st);
+  if (!lexed) {
+    clear_u32<<<1, 64, 0, st>>>(a.flags, 4);
+    ctx->launches++;
+  }
+  rc = parse_phase1<false>(ctx, a, tiles_max, st, nullptr, tiles_est);
+  if (rc) return rc;
+  for (int attempt = 0;; ++attempt) {
+    ctx->prof_begin(S_PARSE_TREE, st);
+    launch_tree<S, false>(ctx, a, tiles_est, starts, ends, node, span, parent, st);
+    ctx->prof_end(S_PARSE_TREE, st);
+    ctx->launches++;
+    ctx->prof_begin(S_LINK_TILES, st);
+    rc = launch_links<false>(ctx, a, tiles_est, lv, parent, st);
+    ctx->prof_end(S_LINK_TILES, st);
+    if (rc) return rc;
+    ctx->prof_end(S_PARSE, st);
+    CK(hipGetLastError());
+    CK(hipStreamSynchronize(st));
+    if (lexed) {
+      if (hw[2]) {
+        ctx->err = "lexer look-back did not complete";
+        return ALPACC_ERR_TIMEOUT;
+      }
+      if (!hw[0]) return ALPACC_REJECT;  // the lexer rejected the input
+      T = hw[1];
+      P = T + 2;
+      if (P * elem_max >= (1ull << 31)) {
+        ctx->err = "token stream too long for 32-bit element counts";
+        return ALPACC_ERR_ARG;
+      }
+    }
+    if (hw[6]) {  // start or end terminals among the tokens: the element-level kernels take them
+      ctx->prof_drop(S_PARSE);
+      return run_parse_tokens<S>(ctx, kinds, starts, ends, T, parent, node, span, cap, num_nodes, st,
+                                 productions_only, false, kinds8, false);
+    }
+    if (hw[4]) return ALPACC_REJECT;  // a missing pair (to_keys, parser.fut:235-240)
+    // depths (parser.fut:153-166): a prefix below zero, or a non-zero end
+    if ((int32_t)hw[11] < 0 || hw[10] != 0) return ALPACC_REJECT;
+    const uint64_t B = hw[8], N = hw[9];
+    ctx->last_counts[0] = T;
+    ctx->last_counts[1] = P;
+    ctx->last_counts[2] = B;
+    ctx->last_counts[3] = N;
+    *num_nodes = N;
+    if (lexed && tile_count(true, P) > tiles_est)  // widen the estimate the grids are sized by
+      ctx->p_per_byte =
+          std::min(4.0, std::max(ctx->p_per_byte, 1.25 * (double)P / (double)std::max<uint64_t>(a.T, 1)));
+    if (B > bcap) {  // more open ends than records: the tree kernels wrote nothing
+      if (attempt > 0) {
+        ctx->err = "link scratch sizing did not converge";
+        return ALPACC_ERR_HIP;
+      }
+      bcap = B + B / 8 + 256;
+      if (a.T) ctx->b_per_byte = std::max(ctx->b_per_byte, (double)bcap / (double)a.T);
+      a.bcap = bcap;
+      a.links = (uint2 *)ctx->buf(B_LINKS, (bcap + 16) * sizeof(uint2));
+      if (!a.links) {
+        ctx->err = "scratch allocation failed";
+        return ALPACC_ERR_HIP;
+      }
+      continue;
+    }
+    if (hw[7]) return ALPACC_REJECT;  // brackets_matches (parser.fut:174-184)
+    if (N > cap) {
+      ctx->err = "output capacity too small";
+      return ALPACC_ERR_CAPACITY;
+    }
+    return ALPACC_ACCEPT;
+  }
+}
+
 // The parser on a token stream of T tokens, with one host synchronisation after the tile scan,
 // which sizes the element scratch (so that parse_expand2 runs one workgroup per actual tile) and
 // decides the missing-pair and depth checks.
@@ -4024,8 +4289,11 @@ int run_search(alpacc_ctx *ctx, const PArgs &a, const ElemBufs &e, uint64_t B, u
 template <typename S>
 int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *ends,
                      uint64_t T, uint32_t *parent, uint32_t *node, S *span, uint64_t cap,
-                     uint64_t *num_nodes, hipStream_t st, bool productions_only = false,
-                     bool lexed = false, const uint8_t *kinds8 = nullptr, bool may_tree = true) {
+                     uint64_t *num_nodes, hipStream_t st, bool productions_only, bool lexed,
+                     const uint8_t *kinds8, bool may_tree) {
+  if (may_tree && ctx->tree_ok)
+    return run_tree<S>(ctx, kinds, starts, ends, T, parent, node, span, cap, num_nodes, st,
+                       productions_only, lexed, kinds8);
   if (!ctx->has_parser) {
     ctx->err = "bundle has no parser";
     return ALPACC_ERR_NO_PARSER;
@@ -4037,12 +4305,9 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
     ctx->err = "token stream too long for 32-bit element counts";
     return ALPACC_ERR_ARG;
   }
-  const bool tree = may_tree && ctx->tree_ok;
-  uint64_t ntiles = tile_count(tree, P);
+  uint64_t ntiles = tile_count(false, P);
   uint32_t *small = (uint32_t *)ctx->buf(B_SMALL, 64 * sizeof(uint32_t));
-  uint16_t *ent = (uint16_t *)ctx->buf(
-      B_ENT, tree && ctx->E < 255 ? ntiles * FT_TILE + 16
-                                  : (ntiles * (tree ? FT_TILE : PK_TILE) + 8) * sizeof(uint16_t));
+  uint16_t *ent = (uint16_t *)ctx->buf(B_ENT, (ntiles * PK_TILE + 8) * sizeof(uint16_t));
   PTup *tiles = (PTup *)ctx->buf(B_PTILES, (ntiles + 1) * sizeof(PTup));
   PTup *pre = (PTup *)ctx->buf(B_PPRE, (ntiles + 1) * sizeof(PTup));
   if (!small || !ent || !tiles || !pre) {
@@ -4064,10 +4329,6 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
   a.total = total;
   a.flags = flags;
   a.ntiles = ntiles;
-  if (tree && !parse_args_tree(ctx, a, ntiles)) {
-    ctx->err = "scratch allocation failed";
-    return ALPACC_ERR_HIP;
-  }
   ctx->prof_begin(S_PARSE, st);
   clear_u32<<<1, 64, 0, st>>>(flags, 4);
   ctx->launches++;
@@ -4090,16 +4351,13 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
       ctx->err = "token stream too long for 32-bit element counts";
       return ALPACC_ERR_ARG;
     }
-    ntiles = tile_count(tree, P);
+    ntiles = tile_count(false, P);
     a.T = T;
     a.P = P;
     a.ntiles = ntiles;
     a.T_dev = nullptr;  // from here on the counts are known on the host
   }
   const uint32_t *hs = ctx->h_small + sh;
-  if (tree && hs[2])  // start or end terminals among the tokens: the tree parser does not take them
-    return run_parse_tokens<S>(ctx, kinds, starts, ends, T, parent, node, span, cap, num_nodes, st,
-                               productions_only, false, kinds8, false);
   if (hs[0]) return ALPACC_REJECT;  // a missing pair (to_keys, parser.fut:235-240)
   PTup tot;
   memcpy(&tot, hs + 8, sizeof(PTup));
@@ -4114,36 +4372,17 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
   ctx->last_counts[3] = N;
   *num_nodes = N;
   const int write_nodes = N <= cap ? 1 : 0;
-  if (tree) {
-    a.links = (uint2 *)ctx->buf(B_LINKS, (B + 16) * sizeof(uint2));
-    if (!a.links) {
-      ctx->err = "scratch allocation failed";
-      return ALPACC_ERR_HIP;
-    }
-    Levels lv;
-    rc = plan_levels(ctx, a.tile_low, a.tile_low1, ntiles, lv, B_LEVELS);
-    if (rc) return rc;
-    ctx->prof_begin(S_PARSE_TREE, st);
-    launch_tree<S, false>(ctx, a, ntiles, starts, ends, node, span, parent, write_nodes, st);
-    ctx->prof_end(S_PARSE_TREE, st);
-    ctx->launches++;
-    ctx->prof_begin(S_LINK_TILES, st);
-    rc = launch_links<false>(ctx, a, ntiles, lv, parent, write_nodes, st);
-    ctx->prof_end(S_LINK_TILES, st);
-    CK(hipGetLastError());
-  } else {
-    ElemBufs e;
-    rc = elem_bufs(ctx, B, N, e, st);
-    if (rc) return rc;
-    const size_t xlds = px_lds_bytes(ctx->nstackw, ctx->nprodw, ctx->E);
-    ctx->prof_begin(S_PARSE_EXPAND, st);
-    parse_expand2<S, false><<<(unsigned)ntiles, PK_THREADS, xlds, st>>>(
-        a, starts, ends, e.depth, e.br, e.dl1, e.sx, e.sl1, node, span, write_nodes);
-    ctx->prof_end(S_PARSE_EXPAND, st);
-    ctx->launches++;
-    CK(hipGetLastError());
-    rc = run_search<false>(ctx, a, e, B, write_nodes ? N : 0, parent, flags, st);
-  }
+  ElemBufs e;
+  rc = elem_bufs(ctx, B, N, e, st);
+  if (rc) return rc;
+  const size_t xlds = px_lds_bytes(ctx->nstackw, ctx->nprodw, ctx->E);
+  ctx->prof_begin(S_PARSE_EXPAND, st);
+  parse_expand2<S, false><<<(unsigned)ntiles, PK_THREADS, xlds, st>>>(
+      a, starts, ends, e.depth, e.br, e.dl1, e.sx, e.sl1, node, span, write_nodes);
+  ctx->prof_end(S_PARSE_EXPAND, st);
+  ctx->launches++;
+  CK(hipGetLastError());
+  rc = run_search<false>(ctx, a, e, B, write_nodes ? N : 0, parent, flags, st);
   if (rc) return rc;
   ctx->prof_end(S_PARSE, st);
   if (!write_nodes || N == 0) {
@@ -4357,17 +4596,17 @@ void enqueue_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t 
                                       const_cast<uint64_t *>(a.ntiles_dev));
   pb_tile_docs<<<ndocs, 256, 0, st>>>(a);
   ctx->launches += 2;
-  (void)parse_phase1<true>(ctx, a, pl.tiles_max, st, pl.btot);
+  (void)parse_phase1<true>(ctx, a, pl.tiles_max, st, pl.btot, pl.tiles_est);
   pb_docs<<<(ndocs + 255) / 256, 256, 0, st>>>(a);
   if (pl.tree) {
     ctx->launches++;
     ctx->prof_begin(S_PARSE_TREE, st);
     launch_tree<uint32_t, true>(ctx, a, pl.tiles_est, pl.starts, pl.ends, pl.node, pl.span,
-                                pl.parent, 1, st);
+                                pl.parent, st);
     ctx->prof_end(S_PARSE_TREE, st);
     ctx->launches++;
     ctx->prof_begin(S_LINK_TILES, st);
-    (void)launch_links<true>(ctx, a, pl.tiles_est, pl.lvt, pl.parent, 1, st);
+    (void)launch_links<true>(ctx, a, pl.tiles_est, pl.lvt, pl.parent, st);
     ctx->prof_end(S_LINK_TILES, st);
     finish_parse_batch(ctx, pl, st);
     return;
