@@ -159,6 +159,7 @@ struct LexArgs {
   uint32_t num_tiles;         // wave tiles of LEX_TILE bytes
   uint32_t num_ctiles;        // count tiles of LEX_CT_WAVES wave tiles
   uint32_t aligned;           // input pointer is 16-byte aligned
+  uint32_t self_scan;         // lex_emit finds its tiles' start states itself (tile_start_state)
   uint16_t *lane_excl;        // [num_tiles*64] exclusive endomorphism of each lane in its wave tile
   uint16_t *tile_agg;         // [num_tiles] endomorphism of each wave tile
   uint16_t *tile_excl;        // [num_tiles] exclusive endomorphism within its scan block
@@ -658,6 +659,53 @@ __device__ __forceinline__ uint64_t pack_count(uint32_t cnt, int32_t last, uint6
   return flag | ((uint64_t)(uint32_t)(last + 1) << 31) | (uint64_t)cnt;
 }
 
+// The lexer state at the start of wave tile LEX_CT_WAVES * ct + w of a document of at most
+// LEX_SELF_TILES wave tiles, found by the count tile's workgroup itself: the tiles before it are
+// composed by a tree over its threads, its own 16 by a scan. That is 12 dependent look-ups, where
+// lex_scan_tiles, lex_scan_blocks and lex_tile_states are 22 and three launches: lex_emit takes
+// 3-5 us longer on a short document and the call 12 us less. Longer documents keep the scan kernels.
+// s_tmp: LDS of 2 * LEX_CT_WAVES words. All threads of the workgroup take part.
+constexpr uint32_t LEX_SELF_TILES = LEX_BLOCK;
+__device__ uint32_t tile_start_state(const LexArgs &p, uint32_t ct, int w, int lane, uint32_t *s_tmp) {
+  const uint32_t first = ct * LEX_CT_WAVES;
+  if ((uint32_t)w * WAVE < first) {
+    uint32_t v = threadIdx.x < first ? p.tile_agg[threadIdx.x] : 0u;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+      const uint32_t left = __shfl(v, (lane - d) & (WAVE - 1), WAVE);
+      if (((lane + 1) & (2 * d - 1)) == 0) v = comp_lookup(p.endo_comp, p.e, left, v);
+    }
+    if (lane == WAVE - 1) s_tmp[w] = v;
+  } else if (lane == 0) {
+    s_tmp[w] = 0;
+  }
+  __syncthreads();
+  if (w == 0) {
+    // lanes 0-15: the count tile's own tiles; lanes 16-31: the wavefronts' totals of earlier ones
+    uint32_t v = 0;
+    if (lane < LEX_CT_WAVES) v = first + lane < p.num_tiles ? p.tile_agg[first + lane] : 0u;
+    else if (lane < 2 * LEX_CT_WAVES) v = s_tmp[lane - LEX_CT_WAVES];
+#define LEX_COMP_STEP(CTRL, D)                                            \
+    {                                                                     \
+      const uint32_t o = (uint32_t)dpp_i32<CTRL>(0, (int32_t)v);          \
+      if ((lane & 15) >= D) v = comp_lookup(p.endo_comp, p.e, o, v);      \
+    }
+    LEX_COMP_STEP(DPP_ROW_SHR1, 1)
+    LEX_COMP_STEP(DPP_ROW_SHR2, 2)
+    LEX_COMP_STEP(DPP_ROW_SHR4, 4)
+    LEX_COMP_STEP(DPP_ROW_SHR8, 8)
+#undef LEX_COMP_STEP
+    const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)v, 2 * LEX_CT_WAVES - 1);
+    const uint32_t ex = (uint32_t)dpp_i32<DPP_ROW_SHR1>(0, (int32_t)v);  // lane 0: the identity
+    if (lane < LEX_CT_WAVES) {
+      const uint32_t pre = comp_lookup(p.endo_comp, p.e, before, ex);
+      s_tmp[LEX_CT_WAVES + lane] = p.endo_apply[pre * p.m1 + p.init];
+    }
+  }
+  __syncthreads();
+  return s_tmp[LEX_CT_WAVES + w];
+}
+
 // K3: walk the lexer DFA from the known lane start states, count token ends / find token starts,
 // scan them across the count tile (16 wave tiles) and across count tiles (decoupled look-back),
 // then write (kind, start, end) of every token. CHUNKED: the input is the virtual string of the
@@ -711,8 +759,10 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
   uint32_t cls[LEX_IPT / 4];
   load_classes(tv.ptr, tv.aligned, s_cls, base, valid, cls, tv.n);
   uint32_t s_lane = 0;
+  uint32_t s_tile = 0;
+  if (!BATCH && p.self_scan) s_tile = tile_start_state(p, ct, w, lane, &s_stage[0][0][0]);
   if (tile < p.num_tiles) {
-    const uint32_t s_tile = p.tile_state[tile];
+    if (BATCH || !p.self_scan) s_tile = p.tile_state[tile];
     const uint32_t ex = p.lane_excl[(uint64_t)tile * WAVE + lane];
     s_lane = p.endo_apply[ex * p.m1 + s_tile];
   }
@@ -3728,6 +3778,7 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   a.num_tiles = (uint32_t)tiles;
   a.num_ctiles = (uint32_t)ctiles;
   a.aligned = ((uintptr_t)d_in & 15) == 0 ? 1u : 0u;
+  a.self_scan = tiles <= LEX_SELF_TILES ? 1u : 0u;
   a.lane_excl = lane_excl;
   a.tile_agg = tile_agg;
   a.tile_excl = tile_excl;
@@ -3761,9 +3812,12 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   launch_lex_reduce<false>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
   ctx->prof_end(S_LEX_REDUCE, st);
   ctx->prof_begin(S_LEX_SCAN, st);
-  lex_scan_tiles<<<(unsigned)sblocks, LEX_SCAN_BLOCK, 0, st>>>(a);
-  lex_scan_blocks<<<1, LEX_SCAN_BLOCK, 0, st>>>(a, (uint32_t)sblocks);
-  lex_tile_states<<<grid_for(tiles, 256), 256, 0, st>>>(a);
+  if (!a.self_scan) {
+    lex_scan_tiles<<<(unsigned)sblocks, LEX_SCAN_BLOCK, 0, st>>>(a);
+    lex_scan_blocks<<<1, LEX_SCAN_BLOCK, 0, st>>>(a, (uint32_t)sblocks);
+    lex_tile_states<<<grid_for(tiles, 256), 256, 0, st>>>(a);
+    ctx->launches += 3;
+  }
   ctx->prof_end(S_LEX_SCAN, st);
   ctx->prof_begin(S_LEX_EMIT, st);
   if (chunk > 0) {
@@ -3774,7 +3828,7 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     launch_lex_emit<false, false>(ctx->dfa_lds, (unsigned)ctiles, a, st);
   }
   ctx->prof_end(S_LEX_EMIT, st);
-  ctx->launches += 5;
+  ctx->launches += 2;
   CK(hipGetLastError());
   if (!sync) return ALPACC_ACCEPT;
   CK(hipStreamSynchronize(st));
