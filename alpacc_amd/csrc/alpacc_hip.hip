@@ -5947,6 +5947,20 @@ int alpacc_copy_to_host(void *dst, const void *src, uint64_t bytes, void *stream
   return hipStreamSynchronize(st) == hipSuccess ? 0 : -1;
 }
 
+int alpacc_copy_to_device_async(void *dst, const void *src, uint64_t bytes, void *stream) {
+  if (bytes == 0) return 0;
+  return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, (hipStream_t)stream) == hipSuccess
+             ? 0
+             : -1;
+}
+
+int alpacc_copy_to_host_async(void *dst, const void *src, uint64_t bytes, void *stream) {
+  if (bytes == 0) return 0;
+  return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, (hipStream_t)stream) == hipSuccess
+             ? 0
+             : -1;
+}
+
 int alpacc_copy_device(void *dst, const void *src, uint64_t bytes, void *stream) {
   if (bytes == 0) return 0;
   return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream) == hipSuccess

@@ -261,6 +261,10 @@ void *alpacc_host_alloc(uint64_t bytes); /* pinned host memory */
 void alpacc_host_free(void *ptr);
 int alpacc_copy_to_device(void *dst, const void *src, uint64_t bytes, void *stream);
 int alpacc_copy_to_host(void *dst, const void *src, uint64_t bytes, void *stream);
+/* the same, only queued: the host side is pinned memory (alpacc_host_alloc) that stays as it is until
+ * the stream has been waited for */
+int alpacc_copy_to_device_async(void *dst, const void *src, uint64_t bytes, void *stream);
+int alpacc_copy_to_host_async(void *dst, const void *src, uint64_t bytes, void *stream);
 int alpacc_copy_device(void *dst, const void *src, uint64_t bytes, void *stream); /* async */
 int alpacc_device_memset(void *dst, int value, uint64_t bytes, void *stream);
 void *alpacc_stream_create(void);
