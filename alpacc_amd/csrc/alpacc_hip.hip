@@ -185,6 +185,8 @@ struct LexArgs {
   // numbered through the documents in order), the DFA starts afresh and token positions restart
   // at 0 in every document, and document d's tokens go to slots [tok_base, tok_base + len + 1).
   const struct LexDoc *docs;  // [ndocs]
+  const struct LexDoc *host_docs;  // when set: pinned host copy that lex_tile_docs brings in
+  uint32_t one_chunk;         // every document is at most one scan chunk
   const uint32_t *tile_doc;   // [num_tiles] document of every wave tile
   const uint4 *tile_rec;      // [num_tiles] the document's byte offset (x, y), length, tile in it
   const uint2 *chunks;        // [nchunks] first wave tile, tile count of every scan chunk
@@ -540,21 +542,24 @@ __global__ void __launch_bounds__(LEX_SCAN_BLOCK) lex_scan_chunks(LexArgs p) {
   const bool in = i < ch.y;
   s[i] = in ? p.tile_agg[ch.x + i] : 0;  // 0: the identity
   __syncthreads();
-  for (uint32_t d = 1; d < LEX_SCAN_BLOCK; d <<= 1) {
+  // a tree over the tiles the chunk has, not the most it can have
+  uint32_t n = 1;
+  while (n < ch.y) n <<= 1;
+  for (uint32_t d = 1; d < n; d <<= 1) {
     uint32_t nv = 0;
-    const bool act = ((i + 1) & (2 * d - 1)) == 0;
+    const bool act = i < n && ((i + 1) & (2 * d - 1)) == 0;
     if (act) nv = comp_lookup(p.endo_comp, p.e, s[i - d], s[i]);
     __syncthreads();
     if (act) s[i] = (uint16_t)nv;
     __syncthreads();
   }
-  if (i == LEX_SCAN_BLOCK - 1) {
+  if (i == n - 1) {
     p.block_agg[blockIdx.x] = s[i];
     s[i] = 0;
   }
   __syncthreads();
-  for (uint32_t d = LEX_SCAN_BLOCK / 2; d >= 1; d >>= 1) {
-    const bool right = ((i + 1) & (2 * d - 1)) == 0;
+  for (uint32_t d = n / 2; d >= 1; d >>= 1) {
+    const bool right = i < n && ((i + 1) & (2 * d - 1)) == 0;
     uint32_t l = 0, r = 0;
     if (right) {
       l = s[i - d];
@@ -567,7 +572,11 @@ __global__ void __launch_bounds__(LEX_SCAN_BLOCK) lex_scan_chunks(LexArgs p) {
     }
     __syncthreads();
   }
-  if (in) p.tile_excl[ch.x + i] = s[i];
+  if (!in) return;
+  if (p.one_chunk)  // the whole document: its tiles' start states, and the two kernels below are not run
+    p.tile_state[ch.x + i] = p.endo_apply[s[i] * p.m1 + p.init];
+  else
+    p.tile_excl[ch.x + i] = s[i];
 }
 
 __global__ void __launch_bounds__(LEX_SCAN_BLOCK) lex_scan_doc_chunks(LexArgs p) {
@@ -587,7 +596,8 @@ __global__ void __launch_bounds__(LEX_SCAN_BLOCK) lex_chunk_states(LexArgs p) {
 
 // Batched mode: the document of every wave tile, and the record its input loads start from.
 __global__ void lex_tile_docs(LexArgs p) {
-  const LexDoc doc = p.docs[blockIdx.x];
+  const LexDoc doc = (p.host_docs ? p.host_docs : p.docs)[blockIdx.x];
+  if (p.host_docs && threadIdx.x == 0) const_cast<LexDoc *>(p.docs)[blockIdx.x] = doc;
   for (uint32_t i = threadIdx.x; i < doc.ntiles; i += blockDim.x) {
     const_cast<uint32_t *>(p.tile_doc)[doc.tile_base + i] = blockIdx.x;
     const_cast<uint4 *>(p.tile_rec)[doc.tile_base + i] =
@@ -1582,6 +1592,7 @@ struct PArgs {
   const uint32_t *ptile_doc; // [tiles] document of every position tile
   const uint64_t *ntiles_dev;
   uint32_t ndocs;
+  uint32_t setup_tiles;      // documents of few tiles: pb_setup fills ptile_doc itself
   uint32_t *doc_flags;       // [ndocs] bit 0: missing pair, bit 1: bracket mismatch
   uint32_t *chunk_doc;       // [N / 64] document of the first production of every 64-chunk
   uint32_t *chunk_base;      // [N / 64] first node of that document; bit 31: a later document
@@ -2210,6 +2221,34 @@ __global__ void __launch_bounds__(PSB) pscan_down(PArgs a, const SegTup *bpre) {
   }
 }
 
+// Batched parser: per document element ranges, the depth check (depths, parser.fut:153-166) and
+// whether the terminal productions pair up with the tokens (safe_zip, :300-303).
+__device__ void pb_doc(const PArgs &a, uint32_t d) {
+  PDoc pd = a.pdocs[d];
+  if (pd.ptiles == 0) {
+    // no positions: the offsets where the document's elements would start keep them monotone
+    const uint64_t ntiles = *a.ntiles_dev;
+    const PTup at = pd.ptile_base < ntiles ? a.pre[pd.ptile_base] : *a.total;
+    pd.br_off = (uint32_t)at.nb;
+    pd.node_off = (uint32_t)at.np;
+    pd.status = 0;
+    a.pdocs[d] = pd;
+    return;
+  }
+  const uint32_t f = pd.ptile_base, l = f + pd.ptiles - 1;
+  const PTup first = a.pre[f];
+  PTup inc = ptup_op(a.pre[l], a.tiles[l]);
+  pd.br_off = (uint32_t)first.nb;
+  pd.node_off = (uint32_t)first.np;
+  pd.B = (uint32_t)(inc.nb - first.nb);
+  pd.N = (uint32_t)(inc.np - first.np);
+  bool ok = pd.lex_ok && (a.doc_flags[d] & 1u) == 0;
+  if (inc.mind < 0 || inc.dd != 0) ok = false;  // B counts the brackets left after cancellation
+  pd.status = ok ? 1u : 0u;
+  pd.subst = (uint32_t)inc.nt == pd.T ? 1u : 0u;
+  a.pdocs[d] = pd;
+}
+
 // The tile scan in one workgroup, each thread over a run of consecutive tiles: in place of
 // pscan_reduce, pscan_top and pscan_down where the tiles are few (up to PSCAN_ONE_MAX), whose time is
 // their launches.
@@ -2252,12 +2291,13 @@ __global__ void __launch_bounds__(PSB) pscan_one(PArgs a) {
     atomicAdd(&s_elems[0], mine_b);
     atomicAdd(&s_elems[1], mine_p);
   }
+  if (threadIdx.x == 0) *a.total = total.t;
   __threadfence_block();
   __syncthreads();
-  if (threadIdx.x == 0) {
-    *a.total = total.t;
+  if (threadIdx.x == 0)
     tree_verdict(a, total.t, s_elems[0] >= (1ull << 31) || s_elems[1] >= (1ull << 31));
-  }
+  if (BATCH)  // (a launch of pb_docs less)
+    for (uint32_t d = threadIdx.x; d < a.ndocs; d += PSB) pb_doc(a, d);
   if (a.tile_low)
     for (uint64_t g = threadIdx.x / WAVE; g * WAVE < ntiles; g += PSB / WAVE) {
       const uint64_t t = g * WAVE + (threadIdx.x & (WAVE - 1));
@@ -2308,6 +2348,9 @@ __global__ void __launch_bounds__(PS_THREADS) pb_setup(PArgs a, const LexDoc *ld
     pd.subst = 0;
     a.pdocs[d] = pd;
     a.doc_flags[d] = 0;
+    if (a.setup_tiles)  // (else by pb_tile_docs)
+      for (uint32_t i = 0; i < pd.ptiles; ++i)
+        const_cast<uint32_t *>(a.ptile_doc)[base + i] = d | (i == 0 ? 0x80000000u : 0u);
     base += pd.ptiles;
   }
   if (threadIdx.x == PS_THREADS - 1) *ntiles_out = base;
@@ -2320,34 +2363,9 @@ __global__ void pb_tile_docs(PArgs a) {
     const_cast<uint32_t *>(a.ptile_doc)[doc.ptile_base + i] = blockIdx.x | (i == 0 ? 0x80000000u : 0u);
 }
 
-// Batched parser: per document element ranges, the depth check (depths, parser.fut:153-166) and
-// whether the terminal productions pair up with the tokens (safe_zip, :300-303).
 __global__ void pb_docs(PArgs a) {
   const uint32_t d = blockIdx.x * blockDim.x + threadIdx.x;
-  if (d >= a.ndocs) return;
-  PDoc pd = a.pdocs[d];
-  if (pd.ptiles == 0) {
-    // no positions: the offsets where the document's elements would start keep them monotone
-    const uint64_t ntiles = *a.ntiles_dev;
-    const PTup at = pd.ptile_base < ntiles ? a.pre[pd.ptile_base] : *a.total;
-    pd.br_off = (uint32_t)at.nb;
-    pd.node_off = (uint32_t)at.np;
-    pd.status = 0;
-    a.pdocs[d] = pd;
-    return;
-  }
-  const uint32_t f = pd.ptile_base, l = f + pd.ptiles - 1;
-  const PTup first = a.pre[f];
-  PTup inc = ptup_op(a.pre[l], a.tiles[l]);
-  pd.br_off = (uint32_t)first.nb;
-  pd.node_off = (uint32_t)first.np;
-  pd.B = (uint32_t)(inc.nb - first.nb);
-  pd.N = (uint32_t)(inc.np - first.np);
-  bool ok = pd.lex_ok && (a.doc_flags[d] & 1u) == 0;
-  if (inc.mind < 0 || inc.dd != 0) ok = false;  // B counts the brackets left after cancellation
-  pd.status = ok ? 1u : 0u;
-  pd.subst = (uint32_t)inc.nt == pd.T ? 1u : 0u;
-  a.pdocs[d] = pd;
+  if (d < a.ndocs) pb_doc(a, d);
 }
 
 constexpr int PX_STAGE = 256;  // element slots per wavefront and round
@@ -3555,12 +3573,11 @@ T *upload(const T *h, size_t count, std::string &err) {
     }                                                                   \
   } while (0)
 
-// reduce-then-scan of n int2 values from `src` into `sink`; the grand total goes to *total
-// (copied to the host when total is not NULL).
-// buf_id: the scratch arena of the upper levels; hierarchies in use at the same time need their own
 // Lays out the 64-ary min levels above level 1 (l1, written by parse_expand2) in the arena
-// buf_id; fill_levels computes them.
-int plan_levels(alpacc_ctx *ctx, int32_t *base, int32_t *l1, uint64_t n, Levels &lv, int buf_id) {
+// buf_id (hierarchies in use at the same time need their own); fill_levels computes them.
+// top: entries of the highest level (searched one after the other).
+int plan_levels(alpacc_ctx *ctx, int32_t *base, int32_t *l1, uint64_t n, Levels &lv, int buf_id,
+                uint64_t top = 64) {
   lv.nlev = 1;
   lv.L[0] = base;
   lv.len[0] = n;
@@ -3570,7 +3587,7 @@ int plan_levels(alpacc_ctx *ctx, int32_t *base, int32_t *l1, uint64_t n, Levels 
   lv.len[1] = len;
   lv.nlev = 2;
   uint64_t total = 0, l = len;
-  while (l > 64) {
+  while (l > top) {
     l = (l + 63) / 64;
     total += ((l + 3) & ~3ull) + 16;
   }
@@ -3580,7 +3597,7 @@ int plan_levels(alpacc_ctx *ctx, int32_t *base, int32_t *l1, uint64_t n, Levels 
     return ALPACC_ERR_HIP;
   }
   uint64_t off = 0;
-  while (len > 64) {
+  while (len > top) {
     if (lv.nlev >= MAX_LEVELS) {
       ctx->err = "input too large for the min levels";
       return ALPACC_ERR_ARG;
@@ -3857,6 +3874,8 @@ struct LexBatchPlan {
   size_t lex_lds;
 };
 
+constexpr uint32_t LEX_HOST_DOCS = 1024;
+
 // Documents (offset, length) of d_in, each lexed on its own; document d's tokens go to slots
 // [tok_base_d, tok_base_d + len_d + 1) of kinds/starts/ends (tok_base = exclusive sum of len + 1),
 // its (accept, token count) to doc_res[2d], [2d+1] (device). h_docs: pinned, ndocs entries.
@@ -3868,7 +3887,7 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
     ctx->err = "bundle has no lexer";
     return ALPACC_ERR_ARG;
   }
-  uint64_t tiles = 0, toks = 0, chunks = 0;
+  uint64_t tiles = 0, toks = 0, chunks = 0, max_tiles = 0;
   for (uint32_t d = 0; d < ndocs; ++d) {
     if (lengths[d] >= (1ull << 31) - 2) {
       ctx->err = "documents must be shorter than 2^31 - 2 bytes";
@@ -3879,6 +3898,7 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
     h_docs[d] = LexDoc{offsets[d], lengths[d], toks, (uint32_t)tiles, (uint32_t)nt,
                        (uint32_t)chunks, (uint32_t)nch};
     tiles += nt;
+    max_tiles = std::max(max_tiles, nt);
     chunks += nch;
     toks += lengths[d] + 1;
     if (tiles >= (1ull << 31) / LEX_TILE * 2) {
@@ -3942,6 +3962,10 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
   a.clear = pl.small;
   a.timeout0 = ctx->force_timeout ? 1u : 0u;
   a.docs = pl.d_docs;
+  // few descriptors are read over the bus by the first kernel itself (one queued copy less, 6 us);
+  // many are left to the copy engine
+  a.host_docs = ndocs <= LEX_HOST_DOCS ? h_docs : nullptr;
+  a.one_chunk = chunks <= ndocs && max_tiles <= LEX_SCAN_BLOCK ? 1u : 0u;
   a.ndocs = ndocs;
   a.doc_res = doc_res;
   const uint64_t wpb = LEX_BLOCK / WAVE;
@@ -3951,7 +3975,8 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
 }
 
 void enqueue_lex_batch(alpacc_ctx *ctx, const LexBatchPlan &pl, hipStream_t st) {
-  (void)hipMemcpyAsync(pl.d_docs, pl.h_docs, pl.ndocs * sizeof(LexDoc), hipMemcpyHostToDevice, st);
+  if (!pl.a.host_docs || pl.tiles == 0)
+    (void)hipMemcpyAsync(pl.d_docs, pl.h_docs, pl.ndocs * sizeof(LexDoc), hipMemcpyHostToDevice, st);
   if (pl.tiles == 0) {
     clear_u32<<<grid_for(2 * (uint64_t)pl.ndocs, 256), 256, 0, st>>>(pl.doc_res,
                                                                      2 * (uint64_t)pl.ndocs);
@@ -3967,13 +3992,16 @@ void enqueue_lex_batch(alpacc_ctx *ctx, const LexBatchPlan &pl, hipStream_t st) 
   ctx->prof_end(S_LEX_REDUCE, st);
   ctx->prof_begin(S_LEX_SCAN, st);
   lex_scan_chunks<<<(unsigned)pl.nchunks, LEX_SCAN_BLOCK, 0, st>>>(a);
-  lex_scan_doc_chunks<<<pl.ndocs, LEX_SCAN_BLOCK, 0, st>>>(a);
-  lex_chunk_states<<<(unsigned)pl.nchunks, LEX_SCAN_BLOCK, 0, st>>>(a);
+  if (!a.one_chunk) {
+    lex_scan_doc_chunks<<<pl.ndocs, LEX_SCAN_BLOCK, 0, st>>>(a);
+    lex_chunk_states<<<(unsigned)pl.nchunks, LEX_SCAN_BLOCK, 0, st>>>(a);
+    ctx->launches += 2;
+  }
   ctx->prof_end(S_LEX_SCAN, st);
   ctx->prof_begin(S_LEX_EMIT, st);
   launch_lex_emit<false, true>(pl.dfa_lds != 0, (unsigned)pl.ctiles, a, st);
   ctx->prof_end(S_LEX_EMIT, st);
-  ctx->launches += 6;
+  ctx->launches += 4;
 }
 
 // The batched lexer queued on `st` (descriptors through the context's pinned staging);
@@ -4044,6 +4072,9 @@ bool parse_args_tree(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max) {
 }
 
 constexpr unsigned TREE_WAVES = 16;
+// highest level of the tiles' min hierarchy: up to 16384 tiles (of the bound) have no level above the
+// one that the tile scan writes, which saves a launch; only pops that end far away search it
+constexpr uint64_t TILE_TOP = 256;
 
 // tiles of `positions` key positions, of the tree parser or the element-level one
 inline uint64_t tile_count(bool tree, uint64_t positions) {
@@ -4257,7 +4288,7 @@ int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *e
   a.ncap = std::min<uint64_t>(cap, 1ull << 31);
   a.subst = productions_only ? 0 : 1;
   Levels lv;
-  int rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, lv, B_LEVELS);
+  int rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, lv, B_LEVELS, TILE_TOP);
   if (rc) return rc;
   hw[7] = 0;
   ctx->prof_begin(S_PARSE, st);
@@ -4456,8 +4487,10 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
 }
 
 // Final per-document results of the batched parser.
-__global__ void pb_finish(PArgs a, alpacc_doc_result *out) {
+// out, words: pinned host memory, so that no copy is queued behind it; words gets the 32 result words.
+__global__ void pb_finish(PArgs a, alpacc_doc_result *out, const uint32_t *small, uint32_t *words) {
   const uint32_t d = blockIdx.x * blockDim.x + threadIdx.x;
+  if (d < 32) words[d] = small[d];
   if (d >= a.ndocs) return;
   const PDoc pd = a.pdocs[d];
   alpacc_doc_result r;
@@ -4497,7 +4530,7 @@ struct ParseBatchPlan {
   Levels lvb, lvs;
   uint32_t *parent, *node, *span;
   const uint32_t *starts, *ends;
-  alpacc_doc_result *d_results, *h_results;
+  alpacc_doc_result *h_results;
   uint32_t *h_words;  // pinned copy of the result words small[0 .. 32)
   size_t xlds;
   unsigned search_bs, search_cap;
@@ -4510,9 +4543,10 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
                      uint32_t *span, uint64_t cap, uint64_t bcap, ParseBatchPlan &pl,
                      hipStream_t st) {
   memset(&pl, 0, sizeof(pl));
-  uint64_t nbytes = 0, tiles_max = 0;
+  uint64_t nbytes = 0, tiles_max = 0, max_len = 0;
   for (uint32_t d = 0; d < ndocs; ++d) {
     nbytes += lengths[d];
+    max_len = std::max(max_len, lengths[d]);
     tiles_max += tile_count(ctx->tree_ok, lengths[d] + 3);
   }
   pl.tree = ctx->tree_ok ? 1 : 0;
@@ -4544,7 +4578,6 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
                                      : (tiles_max * tpos + 8) * sizeof(uint16_t));
   PTup *tiles = (PTup *)ctx->buf(B_PTILES, (tiles_max + 1) * sizeof(PTup));
   PTup *pre = (PTup *)ctx->buf(B_PPRE, (tiles_max + 1) * sizeof(PTup));
-  pl.d_results = (alpacc_doc_result *)ctx->buf(B_RESULTS, (ndocs + 1) * sizeof(alpacc_doc_result));
   const uint64_t nbs = std::max<uint64_t>(1, (tiles_max + PSB - 1) / PSB);
   pl.btot = (SegTup *)ctx->buf(B_BTOT, (nbs + 1) * sizeof(SegTup));
   uint32_t *chunk_doc = nullptr, *chunk_base = nullptr;
@@ -4567,7 +4600,7 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   const size_t res_bytes = ((ndocs + 1) * sizeof(alpacc_doc_result) + 255) & ~(size_t)255;
   uint8_t *stg = ctx->stage(docs_bytes + res_bytes + 256, st);
   if (!kinds || !starts || !ends || !doc_res || !pdocs || !doc_flags || !ptile_doc || !ent ||
-      !tiles || !pre || !pl.d_results || !pl.btot || !elems || !stg) {
+      !tiles || !pre || !pl.btot || !elems || !stg) {
     ctx->err = "scratch allocation failed";
     return ALPACC_ERR_HIP;
   }
@@ -4597,6 +4630,8 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   a.bcap = bcap;
   a.ncap = ncap;
   a.links = links;
+  // pb_setup writes a document's tiles one after the other: short documents only
+  a.setup_tiles = max_len <= (256u << 10) ? 1u : 0u;
   if (pl.tree && !parse_args_tree(ctx, a, tiles_max)) {
     ctx->err = "scratch allocation failed";
     return ALPACC_ERR_HIP;
@@ -4618,7 +4653,7 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   pl.ends = ends;
   pl.lvb.nlev = pl.lvs.nlev = 0;
   if (pl.tree)
-    rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, pl.lvt, B_LEVELS);
+    rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, pl.lvt, B_LEVELS, TILE_TOP);
   else if (bcap > 0)
     rc = plan_levels(ctx, pl.e.depth, pl.e.dl1, bcap, pl.lvb, B_LEVELS);
   if (!rc && ncap > 0 && !pl.tree) rc = plan_levels(ctx, pl.e.sx, pl.e.sl1, ncap, pl.lvs, B_LEVELS_S);
@@ -4632,12 +4667,9 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
 // The end of a planned call: the documents' results, and their copies to the host.
 void finish_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t st) {
   const uint32_t ndocs = pl.lx.ndocs;
-  pb_finish<<<(ndocs + 255) / 256, 256, 0, st>>>(pl.a, pl.d_results);
+  pb_finish<<<(ndocs + 255) / 256, 256, 0, st>>>(pl.a, pl.h_results, pl.lx.small, pl.h_words);
   ctx->launches++;
   ctx->prof_end(S_PARSE, st);
-  (void)hipMemcpyAsync(pl.h_results, pl.d_results, ndocs * sizeof(alpacc_doc_result),
-                       hipMemcpyDeviceToHost, st);
-  (void)hipMemcpyAsync(pl.h_words, pl.lx.small, 32 * sizeof(uint32_t), hipMemcpyDeviceToHost, st);
 }
 
 // Queues the planned call on `st`: copies and kernels only (no allocation, no synchronisation).
@@ -4648,12 +4680,14 @@ void enqueue_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t 
   ctx->prof_begin(S_PARSE, st);
   pb_setup<<<1, PS_THREADS, 0, st>>>(a, pl.lx.d_docs, pl.lx.doc_res,
                                       const_cast<uint64_t *>(a.ntiles_dev));
-  pb_tile_docs<<<ndocs, 256, 0, st>>>(a);
-  ctx->launches += 2;
+  if (!a.setup_tiles) pb_tile_docs<<<ndocs, 256, 0, st>>>(a);
+  ctx->launches += a.setup_tiles ? 1 : 2;
   (void)parse_phase1<true>(ctx, a, pl.tiles_max, st, pl.btot, pl.tiles_est);
-  pb_docs<<<(ndocs + 255) / 256, 256, 0, st>>>(a);
-  if (pl.tree) {
+  if (std::min(pl.tiles_est, pl.tiles_max) > PSCAN_ONE_MAX) {
+    pb_docs<<<(ndocs + 255) / 256, 256, 0, st>>>(a);
     ctx->launches++;
+  }
+  if (pl.tree) {
     ctx->prof_begin(S_PARSE_TREE, st);
     launch_tree<uint32_t, true>(ctx, a, pl.tiles_est, pl.starts, pl.ends, pl.node, pl.span,
                                 pl.parent, st);
@@ -4667,7 +4701,7 @@ void enqueue_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t 
   }
   elem_init<<<grid_for(std::max(pl.nbc, pl.npc) + 16, 256, 4096), 256, 0, st>>>(
       pl.e.dl1, pl.nbc + 16, pl.e.sl1, pl.npc + 16);
-  ctx->launches += 2;
+  ctx->launches++;
   if (pl.tiles_max > 0) {
     ctx->prof_begin(S_PARSE_EXPAND, st);
     parse_expand2<uint32_t, true><<<(unsigned)std::max<uint64_t>(1, pl.tiles_est), PK_THREADS,
