@@ -345,6 +345,46 @@ __device__ __forceinline__ void load_classes(const uint8_t *in, bool aligned, co
   }
 }
 
+// The wave-exclusive composition of the lanes' endomorphisms v (Blelloch up- and down-sweep over
+// the (endo x endo) table) in v; returns the wavefront's total.
+__device__ __forceinline__ uint32_t lex_lane_scan(const uint16_t *comp_tab, uint32_t e, int lane,
+                                                  uint32_t &v) {
+#pragma unroll
+  for (int d = 1; d < WAVE; d <<= 1) {
+    const uint32_t left = __shfl(v, (lane - d) & (WAVE - 1), WAVE);
+    if (((lane + 1) & (2 * d - 1)) == 0) v = comp_lookup(comp_tab, e, left, v);
+  }
+  const uint32_t total = __shfl(v, WAVE - 1, WAVE);
+  if (lane == WAVE - 1) v = 0;
+#pragma unroll
+  for (int d = WAVE / 2; d >= 1; d >>= 1) {
+    const uint32_t left = __shfl(v, (lane - d) & (WAVE - 1), WAVE);
+    const uint32_t right = __shfl(v, (lane + d) & (WAVE - 1), WAVE);
+    if (((lane + 1) & (2 * d - 1)) == 0)
+      v = comp_lookup(comp_tab, e, v, left);
+    else if (((lane + 1 + d) & (2 * d - 1)) == 0)
+      v = right;
+  }
+  return total;
+}
+
+// Exclusive composition inside every row of 16 lanes (four look-ups); incl: the inclusive one.
+__device__ __forceinline__ uint32_t lex_row_scan(const LexArgs &p, int lane, uint32_t v,
+                                                 uint32_t &incl) {
+#define LEX_COMP_STEP(CTRL, D)                                            \
+  {                                                                       \
+    const uint32_t o = (uint32_t)dpp_i32<CTRL>(0, (int32_t)v);            \
+    if ((lane & 15) >= D) v = comp_lookup(p.endo_comp, p.e, o, v);        \
+  }
+  LEX_COMP_STEP(DPP_ROW_SHR1, 1)
+  LEX_COMP_STEP(DPP_ROW_SHR2, 2)
+  LEX_COMP_STEP(DPP_ROW_SHR4, 4)
+  LEX_COMP_STEP(DPP_ROW_SHR8, 8)
+#undef LEX_COMP_STEP
+  incl = v;
+  return (uint32_t)dpp_i32<DPP_ROW_SHR1>(0, (int32_t)v);  // the row's first lane: the identity
+}
+
 // K1: per wave tile, the endomorphism of every lane's bytes (serial walk through the
 // (endo x class) table) and their wave-exclusive composition (Blelloch up/down sweep with the
 // (endo x endo) table, 126 lookups per wave). Persistent, grid-stride over wave tiles.
@@ -695,18 +735,9 @@ __device__ uint32_t tile_start_state(const LexArgs &p, uint32_t ct, int w, int l
     uint32_t v = 0;
     if (lane < LEX_CT_WAVES) v = first + lane < p.num_tiles ? p.tile_agg[first + lane] : 0u;
     else if (lane < 2 * LEX_CT_WAVES) v = s_tmp[lane - LEX_CT_WAVES];
-#define LEX_COMP_STEP(CTRL, D)                                            \
-    {                                                                     \
-      const uint32_t o = (uint32_t)dpp_i32<CTRL>(0, (int32_t)v);          \
-      if ((lane & 15) >= D) v = comp_lookup(p.endo_comp, p.e, o, v);      \
-    }
-    LEX_COMP_STEP(DPP_ROW_SHR1, 1)
-    LEX_COMP_STEP(DPP_ROW_SHR2, 2)
-    LEX_COMP_STEP(DPP_ROW_SHR4, 4)
-    LEX_COMP_STEP(DPP_ROW_SHR8, 8)
-#undef LEX_COMP_STEP
-    const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)v, 2 * LEX_CT_WAVES - 1);
-    const uint32_t ex = (uint32_t)dpp_i32<DPP_ROW_SHR1>(0, (int32_t)v);  // lane 0: the identity
+    uint32_t incl;
+    const uint32_t ex = lex_row_scan(p, lane, v, incl);
+    const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)incl, 2 * LEX_CT_WAVES - 1);
     if (lane < LEX_CT_WAVES) {
       const uint32_t pre = comp_lookup(p.endo_comp, p.e, before, ex);
       s_tmp[LEX_CT_WAVES + lane] = p.endo_apply[pre * p.m1 + p.init];
@@ -723,7 +754,9 @@ __device__ uint32_t tile_start_state(const LexArgs &p, uint32_t ct, int w, int l
 // lex_step, lexer.fut:104-107), spans are shifted as lex_step does, and every chunk's last
 // element is recorded in chunk_info for lex_chunk_fixup.
 // DFA_LDS: the walk words (dfa_walk, (m + 1) x C) are copied to LDS; else they are read from L2.
-template <bool CHUNKED, bool BATCH, bool DFA_LDS>
+// SHORT: the whole document is this one count tile, and the workgroup does lex_reduce's part too
+// (with the (endo x class) table in dynamic LDS): lex 4 KB 28 -> 23.5 us, two launches as one.
+template <bool CHUNKED, bool BATCH, bool DFA_LDS, bool SHORT = false>
 __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
   __shared__ uint32_t s_dfa[LEX_MAX_DFA];
   __shared__ uint8_t s_cls[256];
@@ -743,9 +776,18 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
 #define LEX_WALK(ROW4, CL) (*reinterpret_cast<const uint32_t *>(dfa + (ROW4) + ((CL) << 2)))
   const uint32_t C4 = C << 2;
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_cls[i] = p.byte_class[i];
-  if (threadIdx.x == 0) s_ctile = atomicAdd(p.tile_counter, 1u);
+  extern __shared__ __align__(16) uint8_t smem[];
+  const uint16_t *s_step = reinterpret_cast<const uint16_t *>(smem);
+  if (SHORT) {
+    table_to_lds(smem, p.endo_step, 2 * p.e * C);
+    // the words that the parser counts in; the verdict and the count are written below
+    if (threadIdx.x < 16 && p.clear + threadIdx.x != p.result && p.clear + threadIdx.x != p.result + 1)
+      p.clear[threadIdx.x] = p.clear + threadIdx.x == p.result + 2 ? p.timeout0 : 0u;
+  } else if (threadIdx.x == 0) {
+    s_ctile = atomicAdd(p.tile_counter, 1u);
+  }
   __syncthreads();
-  const uint32_t ct = s_ctile;
+  const uint32_t ct = SHORT ? 0u : s_ctile;
   const int lane = threadIdx.x & (WAVE - 1);
   const int w = threadIdx.x / WAVE;
   const uint32_t tile = ct * LEX_CT_WAVES + w;
@@ -770,8 +812,25 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
   load_classes(tv.ptr, tv.aligned, s_cls, base, valid, cls, tv.n);
   uint32_t s_lane = 0;
   uint32_t s_tile = 0;
-  if (!BATCH && p.self_scan) s_tile = tile_start_state(p, ct, w, lane, &s_stage[0][0][0]);
-  if (tile < p.num_tiles) {
+  if (SHORT) {
+    // lex_reduce's walk and scan of this wavefront's tile, then the tiles before it
+    uint32_t x = 0;
+#pragma unroll
+    for (int j = 0; j < LEX_IPT; ++j)
+      if (j < valid) x = s_step[__umul24(x, C) + LEX_CLS(j)];
+    uint32_t total = lex_lane_scan(p.endo_comp, p.e, lane, x);
+    uint32_t *s_tmp = &s_stage[0][0][0];
+    if (lane == 0) s_tmp[w] = total;
+    __syncthreads();
+    if (w == 0) {
+      const uint32_t ex = lex_row_scan(p, lane, lane < LEX_CT_WAVES ? s_tmp[lane] : 0u, total);
+      if (lane < LEX_CT_WAVES) s_tmp[LEX_CT_WAVES + lane] = p.endo_apply[ex * p.m1 + p.init];
+    }
+    __syncthreads();
+    s_lane = p.endo_apply[x * p.m1 + s_tmp[LEX_CT_WAVES + w]];
+  }
+  if (!SHORT && !BATCH && p.self_scan) s_tile = tile_start_state(p, ct, w, lane, &s_stage[0][0][0]);
+  if (!SHORT && tile < p.num_tiles) {
     if (BATCH || !p.self_scan) s_tile = p.tile_state[tile];
     const uint32_t ex = p.lane_excl[(uint64_t)tile * WAVE + lane];
     s_lane = p.endo_apply[ex * p.m1 + s_tile];
@@ -890,7 +949,7 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     const int32_t ltot = __builtin_amdgcn_readlane(wli, LEX_CT_WAVES - 1);
     const bool ftot = __builtin_amdgcn_readlane(wfi, LEX_CT_WAVES - 1) != 0;
     // a count tile holding a document start already has its (post-reset) inclusive value
-    if (lane == 0) st_relaxed64(p.st_count + ct, pack_count(ctot, ltot, ftot ? CT_INC : CT_AGG));
+    if (!SHORT && lane == 0) st_relaxed64(p.st_count + ct, pack_count(ctot, ltot, ftot ? CT_INC : CT_AGG));
     ct_tot = ctot;
     ct_last = ltot;
     ct_reset = ftot;
@@ -1943,11 +2002,10 @@ __device__ __forceinline__ int32_t ft_pushes(uint32_t f) { return (int32_t)((f >
 // no LDS exchange stand between the lookups and the tile's totals. ET: the entry ids' type (u8 with
 // 0xFF for none below 255 entries, else u16). Tile totals in PTup: nb = records the tile leaves
 // open (pops and pushes), np, dd, mind (at most 0), nt.
+// blk of nblk: this workgroup's share of the tiles. pk_smem: dynamic LDS of the pair index; s_ent: LDS.
 template <bool IDX8, bool BATCH, int KW, typename ET>
-__global__ void __launch_bounds__(PKK_THREADS) __attribute__((amdgpu_waves_per_eu(KW == 4 ? 8 : 1)))
-parse_keys_tree(PArgs a) {
-  extern __shared__ __align__(16) uint8_t pk_smem[];
-  __shared__ uint32_t s_ent[256];
+__device__ __forceinline__ void keys_tree_run(const PArgs &a, uint8_t *pk_smem, uint32_t *s_ent,
+                                              uint32_t blk, uint32_t nblk) {
   if (IDX8) {
     table_to_lds(pk_smem, a.index8, a.index_len);
     for (uint32_t i = threadIdx.x; i < a.E; i += blockDim.x) s_ent[i] = a.tent[i].x;
@@ -1958,13 +2016,13 @@ parse_keys_tree(PArgs a) {
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const uint32_t W = a.q + a.k;
   const uint64_t ntiles = pk_ntiles<BATCH>(a);
-  const uint64_t stride = (uint64_t)gridDim.x * (PKK_THREADS / WAVE);
+  const uint64_t stride = (uint64_t)nblk * (PKK_THREADS / WAVE);
   bool miss = false, odd = false;
   PosView npv;
   uint32_t nsym[PK_IPT + KW - 1];
   bool nraw = false;
   uint32_t noff = 0;
-  uint64_t tile = (uint64_t)blockIdx.x * (PKK_THREADS / WAVE) + w;
+  uint64_t tile = (uint64_t)blk * (PKK_THREADS / WAVE) + w;
   if (tile < ntiles)
     keys_window<BATCH, KW, FT_TILE>(a, tile, ntiles, W, npv, nsym, nraw, noff);
   for (; tile < ntiles; tile += stride) {
@@ -2052,6 +2110,14 @@ parse_keys_tree(PArgs a) {
     if (__ballot(miss) != 0ull && lane == 0) atomicOr(a.flags, 1u);
     if (__ballot(odd) != 0ull && lane == 0) atomicOr(a.flags + 2, 1u);
   }
+}
+
+template <bool IDX8, bool BATCH, int KW, typename ET>
+__global__ void __launch_bounds__(PKK_THREADS) __attribute__((amdgpu_waves_per_eu(KW == 4 ? 8 : 1)))
+parse_keys_tree(PArgs a) {
+  extern __shared__ __align__(16) uint8_t pk_smem[];
+  __shared__ uint32_t s_ent[256];
+  keys_tree_run<IDX8, BATCH, KW, ET>(a, pk_smem, s_ent, blockIdx.x, gridDim.x);
 }
 
 // Segmented tile totals: element counts (nb, np) run through all tiles, the other fields restart
@@ -2255,9 +2321,8 @@ __device__ void pb_doc(const PArgs &a, uint32_t d) {
 constexpr uint64_t PSCAN_ONE_MAX = 16 * PSB;
 
 template <bool BATCH>
-__global__ void __launch_bounds__(PSB) pscan_one(PArgs a) {
-  __shared__ SegTup s_w[PSB / WAVE];
-  __shared__ unsigned long long s_elems[2];
+__device__ __forceinline__ void pscan_one_run(const PArgs &a, SegTup *s_w,
+                                              unsigned long long *s_elems) {
   const uint64_t ntiles = pk_ntiles<BATCH>(a);
   const uint64_t run = (ntiles + PSB - 1) / PSB;
   const uint64_t lo = std::min<uint64_t>(ntiles, threadIdx.x * run);
@@ -2304,6 +2369,30 @@ __global__ void __launch_bounds__(PSB) pscan_one(PArgs a) {
       const int32_t m = wave_min_i32(t < ntiles ? a.tile_low[t] : INT32_MAX);
       if ((threadIdx.x & (WAVE - 1)) == 0) a.tile_low1[g] = m;
     }
+}
+
+template <bool BATCH>
+__global__ void __launch_bounds__(PSB) pscan_one(PArgs a) {
+  __shared__ SegTup s_w[PSB / WAVE];
+  __shared__ unsigned long long s_elems[2];
+  pscan_one_run<BATCH>(a, s_w, s_elems);
+}
+
+// Short single documents (an estimate of at most KEYS_SCAN_MAX tiles, four rounds of one
+// workgroup's wavefronts): the key look-ups and the tile scan in one workgroup, a launch less.
+constexpr uint64_t KEYS_SCAN_MAX = 4 * (PKK_THREADS / WAVE);
+
+template <bool IDX8, int KW, typename ET>
+__global__ void __launch_bounds__(PKK_THREADS) keys_scan_tree(PArgs a) {
+  extern __shared__ __align__(16) uint8_t pk_smem[];
+  __shared__ uint32_t s_ent[256];
+  __shared__ SegTup s_w[PSB / WAVE];
+  __shared__ unsigned long long s_elems[2];
+  static_assert(PKK_THREADS == PSB, "one workgroup runs both");
+  keys_tree_run<IDX8, false, KW, ET>(a, pk_smem, s_ent, 0, 1);
+  __threadfence_block();
+  __syncthreads();  // the tiles' totals and the flags are out
+  pscan_one_run<false>(a, s_w, s_elems);
 }
 
 // position tiles of a document of T tokens
@@ -2806,6 +2895,93 @@ __device__ void parents_run(uint64_t N, const Levels &lv, uint32_t *parent, cons
   }
 }
 
+// The open pops of every tile (links[pre.nb ..), the k-th one at the k-th height below the tile's
+// start) against the open pushes of earlier tiles (behind the pops, upwards from the tile's lowest
+// height): the match is in the last earlier tile whose lowest height is at most the pop's. One
+// workgroup (a column of them where there are few groups) per 64 tiles, its wavefronts taking turns
+// at their pops, 64 at a time: binary lifting over the 64 lowest heights, and a climb of the 64-ary
+// min hierarchy over all tiles for those that leave them. Documents as they come leave 6 pops open
+// per tile and nearly all end inside the 64 tiles; deep nesting leaves up to some 500 per tile, most
+// of them ending far away, which is what the many wavefronts per group are for.
+constexpr int LINK_THREADS = 512;
+template <bool BATCH>
+__device__ __forceinline__ void link_run(const PArgs &a, const Levels &lv, uint32_t *parent,
+                                         uint64_t grp0, uint64_t gstep, int32_t w0, int32_t wstep) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  const uint64_t ntiles = tree_tiles<BATCH>(a);
+  const bool write_nodes = BATCH || (uint64_t)(uint32_t)a.total->np <= a.ncap;
+  const uint64_t ngroups = (ntiles + WAVE - 1) / WAVE;
+  for (uint64_t grp = grp0; grp < ngroups; grp += gstep) {
+    const uint64_t t = grp * WAVE + lane;
+    int32_t d0 = 0, low = INT32_MAX, u = 0, v = 0, off = 0;
+    uint32_t doc = 0;
+    if (t < ntiles) {
+      const PTup pre = a.pre[t], tot = a.tiles[t];
+      d0 = pre.dd;
+      u = -tot.mind;
+      low = d0 - u;
+      v = tot.dd + u;
+      off = pre.nb;
+      if (BATCH) doc = a.ptile_doc[t] & 0x7FFFFFFFu;
+    }
+    int32_t M[6];
+    lift_build(low, M);
+    const int32_t uincl = wave_incl_i32(u, 0, OpAdd());
+    const int32_t total = __builtin_amdgcn_readlane(uincl, WAVE - 1);
+    for (int32_t q0 = w0; q0 < total; q0 += wstep) {
+      const int32_t q = q0 + lane;
+      const bool pop = q < total;
+      // the tile of pop q: the number of tiles whose pops all come before it
+      int l4 = 0;
+#pragma unroll
+      for (int step = WAVE / 2; step >= 1; step >>= 1)
+        if (__builtin_amdgcn_ds_bpermute(l4 + 4 * (step - 1), uincl) <= q) l4 += 4 * step;
+      if (!pop) l4 = 0;
+      const int l = l4 >> 2;
+      const int32_t k = q - (__builtin_amdgcn_ds_bpermute(l4, uincl) - __builtin_amdgcn_ds_bpermute(l4, u));
+      const int32_t h = __builtin_amdgcn_ds_bpermute(l4, d0) - 1 - k;
+      const uint32_t lnk = (uint32_t)__builtin_amdgcn_ds_bpermute(l4, off) + (uint32_t)k;
+      const int p = lift_query(M, l, h);
+      const int s4 = (p - 1) << 2;
+      uint32_t soff = (uint32_t)__builtin_amdgcn_ds_bpermute(s4, off);
+      int32_t su = __builtin_amdgcn_ds_bpermute(s4, u), sv = __builtin_amdgcn_ds_bpermute(s4, v);
+      int32_t slow = __builtin_amdgcn_ds_bpermute(s4, low);
+      const uint32_t qdoc = BATCH ? (uint32_t)__builtin_amdgcn_ds_bpermute(l4, (int)doc) : 0u;
+      if (pop) {
+        const uint2 me = a.links[lnk];
+        bool found = p > 0;
+        if (!found) {
+          const int64_t far = prev_le_far(lv, grp, h);
+          if (far >= 0) {
+            const PTup pre = a.pre[far], tot = a.tiles[far];
+            su = -tot.mind;
+            sv = tot.dd + su;
+            slow = pre.dd - su;
+            soff = (uint32_t)pre.nb;
+            found = true;
+          }
+        }
+        // (in a rejected document the found tile may be another document's: no push at h then)
+        found = found && h - slow < sv;
+        uint2 at = make_uint2(0u, 0xFFFFFFFFu);
+        if (found) at = a.links[(uint64_t)soff + (uint32_t)(su + (h - slow))];
+        if (at.y != me.y) {
+          if (BATCH) atomicOr(a.doc_flags + qdoc, 2u);
+          else a.hw[7] = 1u;
+        }
+        if (write_nodes && me.x != 0xFFFFFFFFu) parent[me.x] = at.x;
+      }
+    }
+  }
+}
+
+template <bool BATCH>
+__global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv, uint32_t *parent) {
+  link_run<BATCH>(a, lv, parent, blockIdx.x, gridDim.x,
+                  (int32_t)(blockIdx.y * LINK_THREADS + threadIdx.x / WAVE * WAVE),
+                  (int32_t)(gridDim.y * LINK_THREADS));
+}
+
 // An entry of at most 3 pops, 4 pushes and 4 productions as one row of three 16-byte words: its
 // word x, its pops, its pushes, its productions' records; row E is empty, for positions without an
 // entry.
@@ -2953,7 +3129,8 @@ __device__ __forceinline__ void ft_load_doc(const PArgs &a, FtTile<ET> &t) {
 // every load issued before the first is used (an operation that a position does not have goes to
 // the lane's padding word); else (larger entries) it loops over each position's own counts, one
 // dependent load after the other.
-template <typename S, bool BATCH, typename ET, bool ROWS>
+// LINK: one workgroup does the whole (short) document, and then link_tiles' part too.
+template <typename S, bool BATCH, typename ET, bool ROWS, bool LINK = false>
 __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, const S *ends,
                                                   uint32_t *node, S *span, uint32_t *parent) {
   extern __shared__ __align__(16) uint32_t ft_smem[];
@@ -3206,87 +3383,12 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
                                starts + tok0, ends + tok0, parent, node, span);
     wave_lds_sync();  // the next tile writes the records again
   }
-}
-
-// The open pops of every tile (links[pre.nb ..), the k-th one at the k-th height below the tile's
-// start) against the open pushes of earlier tiles (behind the pops, upwards from the tile's lowest
-// height): the match is in the last earlier tile whose lowest height is at most the pop's. One
-// workgroup (a column of them where there are few groups) per 64 tiles, its wavefronts taking turns
-// at their pops, 64 at a time: binary lifting over the 64 lowest heights, and a climb of the 64-ary
-// min hierarchy over all tiles for those that leave them. Documents as they come leave 6 pops open
-// per tile and nearly all end inside the 64 tiles; deep nesting leaves up to some 500 per tile, most
-// of them ending far away, which is what the many wavefronts per group are for.
-constexpr int LINK_THREADS = 512;
-template <bool BATCH>
-__global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv,
-                                                           uint32_t *parent) {
-  const int lane = threadIdx.x & (WAVE - 1);
-  const uint64_t ntiles = tree_tiles<BATCH>(a);
-  const bool write_nodes = BATCH || (uint64_t)(uint32_t)a.total->np <= a.ncap;
-  const uint64_t ngroups = (ntiles + WAVE - 1) / WAVE;
-  const int32_t w0 = (int32_t)(blockIdx.y * LINK_THREADS + threadIdx.x / WAVE * WAVE);
-  const int32_t wstep = (int32_t)(gridDim.y * LINK_THREADS);
-  for (uint64_t grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
-    const uint64_t t = grp * WAVE + lane;
-    int32_t d0 = 0, low = INT32_MAX, u = 0, v = 0, off = 0;
-    uint32_t doc = 0;
-    if (t < ntiles) {
-      const PTup pre = a.pre[t], tot = a.tiles[t];
-      d0 = pre.dd;
-      u = -tot.mind;
-      low = d0 - u;
-      v = tot.dd + u;
-      off = pre.nb;
-      if (BATCH) doc = a.ptile_doc[t] & 0x7FFFFFFFu;
-    }
-    int32_t M[6];
-    lift_build(low, M);
-    const int32_t uincl = wave_incl_i32(u, 0, OpAdd());
-    const int32_t total = __builtin_amdgcn_readlane(uincl, WAVE - 1);
-    for (int32_t q0 = w0; q0 < total; q0 += wstep) {
-      const int32_t q = q0 + lane;
-      const bool pop = q < total;
-      // the tile of pop q: the number of tiles whose pops all come before it
-      int l4 = 0;
-#pragma unroll
-      for (int step = WAVE / 2; step >= 1; step >>= 1)
-        if (__builtin_amdgcn_ds_bpermute(l4 + 4 * (step - 1), uincl) <= q) l4 += 4 * step;
-      if (!pop) l4 = 0;
-      const int l = l4 >> 2;
-      const int32_t k = q - (__builtin_amdgcn_ds_bpermute(l4, uincl) - __builtin_amdgcn_ds_bpermute(l4, u));
-      const int32_t h = __builtin_amdgcn_ds_bpermute(l4, d0) - 1 - k;
-      const uint32_t lnk = (uint32_t)__builtin_amdgcn_ds_bpermute(l4, off) + (uint32_t)k;
-      const int p = lift_query(M, l, h);
-      const int s4 = (p - 1) << 2;
-      uint32_t soff = (uint32_t)__builtin_amdgcn_ds_bpermute(s4, off);
-      int32_t su = __builtin_amdgcn_ds_bpermute(s4, u), sv = __builtin_amdgcn_ds_bpermute(s4, v);
-      int32_t slow = __builtin_amdgcn_ds_bpermute(s4, low);
-      const uint32_t qdoc = BATCH ? (uint32_t)__builtin_amdgcn_ds_bpermute(l4, (int)doc) : 0u;
-      if (pop) {
-        const uint2 me = a.links[lnk];
-        bool found = p > 0;
-        if (!found) {
-          const int64_t far = prev_le_far(lv, grp, h);
-          if (far >= 0) {
-            const PTup pre = a.pre[far], tot = a.tiles[far];
-            su = -tot.mind;
-            sv = tot.dd + su;
-            slow = pre.dd - su;
-            soff = (uint32_t)pre.nb;
-            found = true;
-          }
-        }
-        // (in a rejected document the found tile may be another document's: no push at h then)
-        found = found && h - slow < sv;
-        uint2 at = make_uint2(0u, 0xFFFFFFFFu);
-        if (found) at = a.links[(uint64_t)soff + (uint32_t)(su + (h - slow))];
-        if (at.y != me.y) {
-          if (BATCH) atomicOr(a.doc_flags + qdoc, 2u);
-          else a.hw[7] = 1u;
-        }
-        if (write_nodes && me.x != 0xFFFFFFFFu) parent[me.x] = at.x;
-      }
-    }
+  if (LINK) {
+    __threadfence_block();
+    __syncthreads();  // every tile's links and parents are out
+    Levels lv;
+    lv.nlev = 0;  // (64 tiles at most)
+    link_run<BATCH>(a, lv, parent, 0, 1, (int32_t)(w * WAVE), (int32_t)blockDim.x);
   }
 }
 
@@ -3387,6 +3489,7 @@ struct alpacc_ctx {
   bool dfa_lds = true;   // lex_emit's DFA table in LDS
   size_t lex_lds = 0;    // lex_reduce's dynamic LDS
   int lex_tables_lds = 1;  // tuning: 0 keeps every lexer table in L2
+  bool lex_short = false;  // short documents lexed by one workgroup: the tables fit its LDS
   // parser tables
   bool has_parser = false;
   uint32_t q = 0, k = 0, nT = 0, start_t = 0, end_t = 0, empty_t = 0, E = 0;
@@ -3701,6 +3804,18 @@ void *noalloc_scratch_setup(int device) {
   return g_noalloc_ptr[device];
 }
 
+// Waits for a lexer call and reads its verdict from the pinned words.
+int lex_verdict(alpacc_ctx *ctx, uint64_t *num_tokens, hipStream_t st) {
+  CK(hipStreamSynchronize(st));
+  const volatile uint32_t *hw = ctx->h_small;
+  if (hw[2]) {
+    ctx->err = "lexer look-back did not complete";
+    return ALPACC_ERR_TIMEOUT;
+  }
+  *num_tokens = hw[1];
+  return hw[0] ? ALPACC_ACCEPT : ALPACC_REJECT;
+}
+
 // The lexer. chunk == 0: unchunked (kinds/starts/ends as u32). chunk > 0: the reference's chunk
 // loop with chunks of `chunk` bytes (kinds, starts64/ends64).
 // sync = false (unchunked only): return ALPACC_ACCEPT once the kernels are queued; the verdict,
@@ -3825,6 +3940,14 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   const uint64_t wpb = LEX_BLOCK / WAVE;
   uint64_t blocks = (tiles + wpb - 1) / wpb;
   blocks = std::min<uint64_t>(blocks, (uint64_t)std::max(1, ctx->cus) * ctx->lex_bpc);
+  if (chunk == 0 && ctiles == 1 && ctx->lex_short) {
+    ctx->prof_begin(S_LEX_EMIT, st);
+    lex_emit<false, false, true, true><<<1, LEX_BLOCK, 2 * ctx->e * ctx->C, st>>>(a);
+    ctx->prof_end(S_LEX_EMIT, st);
+    ctx->launches++;
+    CK(hipGetLastError());
+    return sync ? lex_verdict(ctx, num_tokens, st) : ALPACC_ACCEPT;
+  }
   ctx->prof_begin(S_LEX_REDUCE, st);
   launch_lex_reduce<false>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
   ctx->prof_end(S_LEX_REDUCE, st);
@@ -3847,14 +3970,7 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   ctx->prof_end(S_LEX_EMIT, st);
   ctx->launches += 2;
   CK(hipGetLastError());
-  if (!sync) return ALPACC_ACCEPT;
-  CK(hipStreamSynchronize(st));
-  if (ctx->h_small[2]) {
-    ctx->err = "lexer look-back did not complete";
-    return ALPACC_ERR_TIMEOUT;
-  }
-  *num_tokens = ctx->h_small[1];
-  return ctx->h_small[0] ? ALPACC_ACCEPT : ALPACC_REJECT;
+  return sync ? lex_verdict(ctx, num_tokens, st) : ALPACC_ACCEPT;
 }
 
 // A batched lexer pass planned on the host: every buffer sized and allocated, the document
@@ -4072,6 +4188,9 @@ bool parse_args_tree(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max) {
 }
 
 constexpr unsigned TREE_WAVES = 16;
+// a document of at most so many tiles (by the estimate) has its tree built and linked by one
+// workgroup, two rounds of its wavefronts, a launch less
+constexpr uint64_t TREE_LINK_MAX = 8;
 // highest level of the tiles' min hierarchy: up to 16384 tiles (of the bound) have no level above the
 // one that the tile scan writes, which saves a launch; only pops that end far away search it
 constexpr uint64_t TILE_TOP = 256;
@@ -4081,42 +4200,55 @@ inline uint64_t tile_count(bool tree, uint64_t positions) {
   return tree ? (positions + FT_TILE - 1) / FT_TILE : (positions + PK_TILE - 1) / PK_TILE;
 }
 
-// The key lookups of the tree parser.
+// The key lookups of the tree parser; with_scan: and the tile scan, in one workgroup.
 template <bool BATCH>
-void launch_keys_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles_max, hipStream_t st) {
+void launch_keys_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles_max, bool with_scan,
+                      hipStream_t st) {
   constexpr uint64_t wpb = PKK_THREADS / WAVE;
   const unsigned g = (unsigned)std::max<uint64_t>(
       1, std::min<uint64_t>((ntiles_max + wpb - 1) / wpb,
                             (uint64_t)std::max(1, ctx->cus) * ctx->keys_bpc));
   const bool small_w = ctx->q + ctx->k <= 4, ent8 = ctx->E < 255;
-  if (ctx->d_index8 && small_w)
-    parse_keys_tree<true, BATCH, 4, uint8_t><<<g, PKK_THREADS, ctx->index_len, st>>>(a);
-  else if (ctx->d_index8)
-    parse_keys_tree<true, BATCH, PK_MAXW, uint8_t><<<g, PKK_THREADS, ctx->index_len, st>>>(a);
-  else if (small_w && ent8)
-    parse_keys_tree<false, BATCH, 4, uint8_t><<<g, PKK_THREADS, 0, st>>>(a);
-  else if (ent8)
-    parse_keys_tree<false, BATCH, PK_MAXW, uint8_t><<<g, PKK_THREADS, 0, st>>>(a);
-  else if (small_w)
-    parse_keys_tree<false, BATCH, 4, uint16_t><<<g, PKK_THREADS, 0, st>>>(a);
+  const size_t lds = ctx->d_index8 ? ctx->index_len : 0;
+  // (IDX8, KW, entry type) of the grammar
+  auto pick = [&](auto run) {
+    using std::integral_constant;
+    if (ctx->d_index8 && small_w) run(std::true_type(), integral_constant<int, 4>(), uint8_t());
+    else if (ctx->d_index8) run(std::true_type(), integral_constant<int, PK_MAXW>(), uint8_t());
+    else if (small_w && ent8) run(std::false_type(), integral_constant<int, 4>(), uint8_t());
+    else if (ent8) run(std::false_type(), integral_constant<int, PK_MAXW>(), uint8_t());
+    else if (small_w) run(std::false_type(), integral_constant<int, 4>(), uint16_t());
+    else run(std::false_type(), integral_constant<int, PK_MAXW>(), uint16_t());
+  };
+  if (with_scan)
+    pick([&](auto idx8, auto kw, auto et) {
+      keys_scan_tree<decltype(idx8)::value, decltype(kw)::value, decltype(et)>
+          <<<1, PKK_THREADS, lds, st>>>(a);
+    });
   else
-    parse_keys_tree<false, BATCH, PK_MAXW, uint16_t><<<g, PKK_THREADS, 0, st>>>(a);
+    pick([&](auto idx8, auto kw, auto et) {
+      parse_keys_tree<decltype(idx8)::value, BATCH, decltype(kw)::value, decltype(et)>
+          <<<g, PKK_THREADS, lds, st>>>(a);
+    });
 }
 
+// link: one workgroup, which links the tiles as well (entry rows, byte entry ids).
 // The tree of about ntiles tiles by workgroups striding over them (each wavefront loads its next
 // tile's words while it works on one): up to TREE_WAVES times as many as the GPU holds at once, which
 // measured 510 us on a 256 MiB batch of sexp documents and 416 us on a 256 MiB JSON document against
 // 586 and 426 us with once (the wavefronts then write and compute in step).
 template <typename S, bool BATCH>
 void launch_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const S *starts, const S *ends,
-                 uint32_t *node, S *span, uint32_t *parent, hipStream_t st) {
+                 uint32_t *node, S *span, uint32_t *parent, bool link, hipStream_t st) {
   const uint64_t wpb = ctx->tree_threads / WAVE;
   const unsigned g = (unsigned)std::max<uint64_t>(
-      1, std::min<uint64_t>((ntiles + wpb - 1) / wpb, (uint64_t)std::max(1, ctx->cus) * ctx->tree_bpc * TREE_WAVES));
+      1, std::min<uint64_t>((ntiles + wpb - 1) / wpb,
+                            link ? 1 : (uint64_t)std::max(1, ctx->cus) * ctx->tree_bpc * TREE_WAVES));
   auto run = [&](auto kernel) {
     kernel<<<g, ctx->tree_threads, ctx->tree_lds, st>>>(a, starts, ends, node, span, parent);
   };
-  if (ctx->E < 255 && ctx->d_trow) run(parse_tree<S, BATCH, uint8_t, true>);
+  if (link) run(parse_tree<S, false, uint8_t, true, true>);
+  else if (ctx->E < 255 && ctx->d_trow) run(parse_tree<S, BATCH, uint8_t, true>);
   else if (ctx->E < 255) run(parse_tree<S, BATCH, uint8_t, false>);
   else if (ctx->d_trow) run(parse_tree<S, BATCH, uint16_t, true>);
   else run(parse_tree<S, BATCH, uint16_t, false>);
@@ -4146,8 +4278,15 @@ int parse_phase1(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max, hipStream_t st,
   const unsigned kgrid =
       (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(nsuper, (uint64_t)std::max(1, ctx->cus) * ctx->keys_bpc));
   const bool small_w = ctx->q + ctx->k <= 4;
+  if (!BATCH && a.tshift == 8 && std::min(ntiles_est, ntiles_max) <= KEYS_SCAN_MAX) {
+    launch_keys_tree<BATCH>(ctx, a, ntiles_max, true, st);
+    ctx->prof_end(S_PARSE_KEYS, st);
+    ctx->launches++;
+    CK(hipGetLastError());
+    return 0;
+  }
   if (a.tshift == 8)
-    launch_keys_tree<BATCH>(ctx, a, ntiles_max, st);
+    launch_keys_tree<BATCH>(ctx, a, ntiles_max, false, st);
   else if (ctx->d_index8 && small_w)
     parse_keys2<true, BATCH, 4><<<kgrid, PKK_THREADS, ctx->index_len, st>>>(a);
   else if (ctx->d_index8)
@@ -4290,6 +4429,8 @@ int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *e
   Levels lv;
   int rc = plan_levels(ctx, a.tile_low, a.tile_low1, tiles_max, lv, B_LEVELS, TILE_TOP);
   if (rc) return rc;
+  // (the bound, which the kernel relies on, and the estimate, which makes it worth while)
+  const bool link = tiles_max <= WAVE && tiles_est <= TREE_LINK_MAX && ctx->d_trow && ctx->E < 255;
   hw[7] = 0;
   ctx->prof_begin(S_PARSE, st);
   if (!lexed) {
@@ -4300,13 +4441,15 @@ int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *e
   if (rc) return rc;
   for (int attempt = 0;; ++attempt) {
     ctx->prof_begin(S_PARSE_TREE, st);
-    launch_tree<S, false>(ctx, a, tiles_est, starts, ends, node, span, parent, st);
+    launch_tree<S, false>(ctx, a, tiles_est, starts, ends, node, span, parent, link, st);
     ctx->prof_end(S_PARSE_TREE, st);
     ctx->launches++;
-    ctx->prof_begin(S_LINK_TILES, st);
-    rc = launch_links<false>(ctx, a, tiles_est, lv, parent, st);
-    ctx->prof_end(S_LINK_TILES, st);
-    if (rc) return rc;
+    if (!link) {
+      ctx->prof_begin(S_LINK_TILES, st);
+      rc = launch_links<false>(ctx, a, tiles_est, lv, parent, st);
+      ctx->prof_end(S_LINK_TILES, st);
+      if (rc) return rc;
+    }
     ctx->prof_end(S_PARSE, st);
     CK(hipGetLastError());
     CK(hipStreamSynchronize(st));
@@ -4690,7 +4833,7 @@ void enqueue_parse_batch(alpacc_ctx *ctx, const ParseBatchPlan &pl, hipStream_t 
   if (pl.tree) {
     ctx->prof_begin(S_PARSE_TREE, st);
     launch_tree<uint32_t, true>(ctx, a, pl.tiles_est, pl.starts, pl.ends, pl.node, pl.span,
-                                pl.parent, st);
+                                pl.parent, false, st);
     ctx->prof_end(S_PARSE_TREE, st);
     ctx->launches++;
     ctx->prof_begin(S_LINK_TILES, st);
@@ -4875,6 +5018,15 @@ int place_lexer_tables(alpacc_ctx *ctx, std::string &err) {
     lds = 256;
   }
   ctx->dfa_lds = ctx->lex_tables_lds && (size_t)ctx->m1 * ctx->C <= (size_t)LEX_MAX_DFA;
+  // lex_emit's own LDS is 72 KB
+  const size_t step = (size_t)2 * ctx->e * ctx->C;
+  ctx->lex_short = ctx->lex_tab >= 1 && ctx->dfa_lds && step <= 80 * 1024;
+  if (ctx->lex_short &&
+      hipFuncSetAttribute((const void *)lex_emit<false, false, true, true>,
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)step) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->lex_short = false;
+  }
   if (lds > 64 * 1024) {
     const int want = (int)lds;
     if (hipFuncSetAttribute((const void *)lex_reduce<1, false>,
