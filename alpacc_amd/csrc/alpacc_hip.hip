@@ -50,7 +50,7 @@ constexpr uint32_t ST_INC = 2u << 30;
 constexpr uint64_t CT_AGG = 1ull << 62;
 constexpr uint64_t CT_INC = 2ull << 62;
 constexpr uint32_t SPIN_LIMIT = 1u << 22;        // bounded waits: a stuck look-back ends the kernel
-constexpr int LEX_CT_WAVES = LEX_BLOCK / WAVE;   // wave tiles per count tile (one block)
+constexpr int LEX_CT_WAVES = 16;                 // wave tiles per count tile (one lex_emit block)
 constexpr int LEX_SCAN_BLOCK = 1024;             // wave tiles per K2a scan block
 constexpr int LEX_MAX_DFA = 4096;                // max (m+1)*C entries of the DFA table in LDS
 constexpr int LEX_STAGE = 384;                   // tokens staged per wavefront and round
@@ -129,6 +129,13 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// look-back words of a number of count tiles: theirs, their groups', then the ticket counter on a
+// cache line of its own (LB_TICKET words before the end)
+constexpr uint64_t LB_TICKET = 32;
+__host__ __device__ constexpr uint64_t lb_words(uint64_t ctiles) {
+  return ctiles + (ctiles + WAVE - 1) / WAVE + 16 + LB_TICKET;
+}
+
 // A table of `bytes` bytes from global memory into LDS (both 16-byte aligned) by the whole
 // workgroup, 16 bytes per load: a short document's kernels are mostly this copy, and a load per
 // element took json's 54 KB (endomorphism x class) table 27 rounds and its 50 KB pair index 50
@@ -167,8 +174,9 @@ struct LexArgs {
   uint8_t *tile_state;        // [num_tiles] lexer DFA state at the start of each wave tile
   uint32_t *tile_counter;     // [1] dynamic count-tile index
   uint64_t *st_count;         // [num_ctiles] look-back words of the count scan
+  uint64_t *st_group;         // [num_ctiles / 64] the same of groups of 64 count tiles (behind st_count)
   uint32_t *result;           // [0] accept, [1] tokens, [2] timeout flag
-  uint32_t *clear;            // the 16 words (counter, results, parser flags) that lex_reduce clears
+  uint32_t *clear;            // the 16 words (results, parser flags) that lex_reduce clears
   uint32_t timeout0;          // what it sets the timeout flag to (testing hook)
   uint32_t *host_result;      // when set: pinned host copy of result
   // chunked mode (the reference's chunk loop, lexer.fut:144-172): `in` is the virtual string in
@@ -345,6 +353,41 @@ __device__ __forceinline__ void load_classes(const uint8_t *in, bool aligned, co
   }
 }
 
+// The bytes in[base .. base + 32) of one lane, four to a word; past the document's end (valid < 32)
+// the words hold any bytes of the aligned 16-byte words around (as load_classes, which see).
+__device__ __forceinline__ void load_words(const uint8_t *in, bool aligned, uint64_t base, int valid,
+                                           uint64_t n, uint32_t (&wds)[LEX_IPT / 4]) {
+  if (valid == LEX_IPT && aligned) {
+    const uint4 a = *reinterpret_cast<const uint4 *>(in + base);
+    const uint4 b = *reinterpret_cast<const uint4 *>(in + base + 16);
+    wds[0] = a.x; wds[1] = a.y; wds[2] = a.z; wds[3] = a.w;
+    wds[4] = b.x; wds[5] = b.y; wds[6] = b.z; wds[7] = b.w;
+  } else if (valid > 0) {
+    const uint8_t *q = in + base;
+    const uint32_t off = (uint32_t)((uintptr_t)q & 15);
+    const uint4 *a4 = reinterpret_cast<const uint4 *>(q - off);
+    // index (from a4) of the word holding the document's last byte; q is inside the document
+    const uint32_t lw = (uint32_t)(((uintptr_t)(in + n - 1) >> 4) - ((uintptr_t)q >> 4));
+    const uint4 x0 = a4[0], x1 = a4[min(1u, lw)], x2 = a4[min(2u, lw)];
+    const uint32_t w[12] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w,
+                            x2.x, x2.y, x2.z, x2.w};
+    const uint32_t sh = off & 3;
+#define LEX_ALIGN_CASE(W0)                                                              \
+  _Pragma("unroll") for (int r = 0; r < 8; ++r) wds[r] =                                \
+      __builtin_amdgcn_alignbyte(w[(W0) + r + 1], w[(W0) + r], sh);
+    switch (off >> 2) {
+      case 0: LEX_ALIGN_CASE(0) break;
+      case 1: LEX_ALIGN_CASE(1) break;
+      case 2: LEX_ALIGN_CASE(2) break;
+      default: LEX_ALIGN_CASE(3) break;
+    }
+#undef LEX_ALIGN_CASE
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) wds[q] = 0u;
+  }
+}
+
 // The wave-exclusive composition of the lanes' endomorphisms v (Blelloch up- and down-sweep over
 // the (endo x endo) table) in v; returns the wavefront's total.
 __device__ __forceinline__ uint32_t lex_lane_scan(const uint16_t *comp_tab, uint32_t e, int lane,
@@ -410,7 +453,7 @@ lex_reduce(LexArgs p) {
   const uint32_t stride = gridDim.x * wpb;
   // the words that lex_emit and the parser count in and look back at
   const uint32_t gt = blockIdx.x * blockDim.x + threadIdx.x;
-  for (uint32_t i = gt; i < p.num_ctiles; i += gridDim.x * blockDim.x) p.st_count[i] = 0;
+  for (uint32_t i = gt; i < lb_words(p.num_ctiles); i += gridDim.x * blockDim.x) p.st_count[i] = 0;
   if (gt < 16) p.clear[gt] = gt == (uint32_t)(p.result + 2 - p.clear) ? p.timeout0 : 0u;
   // two tiles per iteration: their table-lookup chains are independent and overlap
   for (uint32_t t0 = blockIdx.x * wpb + threadIdx.x / WAVE; t0 < p.num_tiles; t0 += 2 * stride) {
@@ -651,62 +694,91 @@ __global__ void lex_tile_docs(LexArgs p) {
         make_uint2(doc.tile_base + c * LEX_SCAN_BLOCK, min((uint32_t)LEX_SCAN_BLOCK, doc.ntiles - c * LEX_SCAN_BLOCK));
 }
 
-// Exclusive (token count, last token start) of a count tile: decoupled look-back; the two
-// components combine by + and max, so the window reduces with plain wave reductions.
-__device__ void lookback_count(const LexArgs &p, uint32_t tile, int lane, uint32_t &cnt,
-                               int32_t &last) {
-  uint32_t csum = 0;
-  int32_t lmax = -1;
-  int64_t j = (int64_t)tile - 1;
+__device__ __forceinline__ uint64_t pack_count(uint32_t cnt, int32_t last, uint64_t flag) {
+  return flag | ((uint64_t)(uint32_t)(last + 1) << 31) | (uint64_t)cnt;
+}
+
+// One window of a look-back: lane l holds word base[at - l] (lanes of `none`: no word). Adds the
+// words back to the nearest inclusive one (or all) to (csum, lmax) and returns true when there is an
+// inclusive one; a word not yet published is waited for, one load per poll (every waiting workgroup
+// reading its whole window, and the shared timeout word, at each poll slows the loads of those still
+// walking). given_up: the bounded wait ended without it.
+__device__ bool lookback_window(const LexArgs &p, const uint64_t *base, int64_t at, bool none, int lane,
+                                uint64_t w, uint32_t &csum, int32_t &lmax, bool &given_up) {
   uint32_t spins = 0;
   while (true) {
-    const int64_t idx = j - lane;
-    const uint64_t w = idx >= 0 ? ld_relaxed64(p.st_count + idx) : CT_INC;
-    const uint32_t flag = (uint32_t)(w >> 62);
+    const uint32_t flag = none ? 1u : (uint32_t)(w >> 62);
     const uint64_t incm = __ballot(flag == 2);
-    const uint64_t zerom = __ballot(flag == 0);
     const uint64_t upto = incm ? (((incm & (~incm + 1)) << 1) - 1) : ~0ull;
-    if (zerom & upto) {
-      // wait on the nearest count tile not yet published, one word per poll, then read the
-      // window again: every waiting count tile reading its whole window (and the shared timeout
-      // word) at each poll piles requests onto the few lines that hold the recent words, and the
-      // loads of the tiles still walking slow down behind them
-      const int zl = __ffsll((unsigned long long)(zerom & upto)) - 1;
-      const uint64_t *zw = p.st_count + (j - zl);
-      bool given_up = false;
-      while ((ld_relaxed64(zw) >> 62) == 0) {
-        ++spins;
-        if (spins > SPIN_LIMIT || ((spins & 63) == 1 && ld_relaxed(p.result + 2) != 0)) {
-          given_up = true;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-      }
-      if (given_up) {
+    const uint64_t zerom = __ballot(flag == 0) & upto;
+    if (!zerom) {
+      const bool in = !none && ((upto >> lane) & 1ull);
+      csum += wave_sum_u32(in ? (uint32_t)(w & 0x7FFFFFFFull) : 0u);
+      lmax = max(lmax, wave_max_i32(in ? (int32_t)((w >> 31) & 0x7FFFFFFFull) - 1 : -1));
+      return incm != 0;
+    }
+    const uint64_t *zw = base + (at - (__ffsll((unsigned long long)zerom) - 1));
+    while ((ld_relaxed64(zw) >> 62) == 0) {
+      ++spins;
+      if (spins > SPIN_LIMIT || ((spins & 63) == 1 && ld_relaxed(p.result + 2) != 0)) {
         if (lane == 0) {
           st_relaxed(p.result + 2, 1u);
           if (p.host_result) p.host_result[2] = 1u;
         }
-        cnt = 0;
-        last = -1;
-        return;
+        given_up = true;
+        return true;
       }
-      continue;
+      __builtin_amdgcn_s_sleep(2);
     }
-    const bool in = (upto >> lane) & 1ull;
-    uint32_t c = in ? (uint32_t)(w & 0x7FFFFFFFull) : 0u;
-    int32_t l = in ? (int32_t)((w >> 31) & 0x7FFFFFFFull) - 1 : -1;
-    csum += wave_sum_u32(c);
-    lmax = max(lmax, wave_max_i32(l));
-    if (incm) break;
-    j -= WAVE;
+    if (!none) w = ld_relaxed64(base + (at - lane));
   }
-  cnt = csum;
-  last = lmax;
 }
 
-__device__ __forceinline__ uint64_t pack_count(uint32_t cnt, int32_t last, uint64_t flag) {
-  return flag | ((uint64_t)(uint32_t)(last + 1) << 31) | (uint64_t)cnt;
+// Exclusive (token count, last token start) of count tile ct, whose own total is (tot, tlast): the
+// words of the earlier tiles of its group of 64 and of the LB_GROUPS groups before, then the words of
+// the groups before those, 64 to a window, back to an inclusive one. A group's word is published by
+// its last tile, as soon as it has seen the group's other tiles, and again as inclusive once it knows
+// its own prefix. So a tile waits for the totals of earlier tiles, never for their prefixes: with one
+// level of words that turn inclusive one after the other the prefix advances 64 tiles per round trip
+// of 2.5 us, and once the tiles' own work had got shorter than that (256 MiB of JSON without any
+// look-back: 186 us) it bound the kernel at 321 us; now 227, and 259 before the shorter walk and
+// staging. The ticket counter's own cache line is part of it: on the line of the time-out word that
+// waiting tiles look at, the 8192 tickets kept the kernel at 364 us.
+// The two components combine by + and max, so the windows reduce with plain wave reductions.
+constexpr int LB_GROUPS = 1;
+__device__ void lookback_count(const LexArgs &p, uint32_t ct, int lane, uint32_t tot, int32_t tlast,
+                               bool reset, uint32_t &cnt, int32_t &last) {
+  const int64_t g = (int64_t)(ct / WAVE), r = (int64_t)(ct % WAVE);
+  // the first windows in one round trip
+  uint64_t w[LB_GROUPS + 1];
+#pragma unroll
+  for (int k = 0; k <= LB_GROUPS; ++k) {
+    const int64_t at = k == 0 ? (int64_t)ct - 1 : (g - k) * WAVE + WAVE - 1;
+    w[k] = (k == 0 ? lane >= r : at < 0) ? 0ull : ld_relaxed64(p.st_count + (at - lane));
+  }
+  int64_t at = g - 1 - LB_GROUPS;
+  uint64_t wg = at - lane >= 0 ? ld_relaxed64(p.st_group + (at - lane)) : 0ull;
+  uint32_t csum = 0;
+  int32_t lmax = -1;
+  bool given_up = false;
+  bool done = lookback_window(p, p.st_count, (int64_t)ct - 1, lane >= r, lane, w[0], csum, lmax, given_up);
+  const bool ends_group = r == WAVE - 1 && !reset && lane == 0;
+  if (ends_group)
+    st_relaxed64(p.st_group + g, pack_count(csum + tot, max(lmax, tlast), done ? CT_INC : CT_AGG));
+#pragma unroll
+  for (int k = 1; k <= LB_GROUPS; ++k)
+    if (!done && g >= k)
+      done = lookback_window(p, p.st_count, (g - k) * WAVE + WAVE - 1, false, lane, w[k], csum, lmax,
+                             given_up);
+  for (; !done && at >= 0; at -= WAVE) {
+    const bool none = at - lane < 0;
+    done = lookback_window(p, p.st_group, at, none, lane, wg, csum, lmax, given_up);
+    if (!done && at >= WAVE)
+      wg = at - WAVE - lane >= 0 ? ld_relaxed64(p.st_group + (at - WAVE - lane)) : 0ull;
+  }
+  if (ends_group) st_relaxed64(p.st_group + g, pack_count(csum + tot, max(lmax, tlast), CT_INC));
+  cnt = given_up ? 0u : csum;
+  last = given_up ? -1 : lmax;
 }
 
 // The lexer state at the start of wave tile LEX_CT_WAVES * ct + w of a document of at most
@@ -715,7 +787,7 @@ __device__ __forceinline__ uint64_t pack_count(uint32_t cnt, int32_t last, uint6
 // lex_scan_tiles, lex_scan_blocks and lex_tile_states are 22 and three launches: lex_emit takes
 // 3-5 us longer on a short document and the call 12 us less. Longer documents keep the scan kernels.
 // s_tmp: LDS of 2 * LEX_CT_WAVES words. All threads of the workgroup take part.
-constexpr uint32_t LEX_SELF_TILES = LEX_BLOCK;
+constexpr uint32_t LEX_SELF_TILES = LEX_CT_WAVES * WAVE;
 __device__ uint32_t tile_start_state(const LexArgs &p, uint32_t ct, int w, int lane, uint32_t *s_tmp) {
   const uint32_t first = ct * LEX_CT_WAVES;
   if ((uint32_t)w * WAVE < first) {
@@ -757,29 +829,37 @@ __device__ uint32_t tile_start_state(const LexArgs &p, uint32_t ct, int w, int l
 // SHORT: the whole document is this one count tile, and the workgroup does lex_reduce's part too
 // (with the (endo x class) table in dynamic LDS): lex 4 KB 28 -> 23.5 us, two launches as one.
 template <bool CHUNKED, bool BATCH, bool DFA_LDS, bool SHORT = false>
-__global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
-  __shared__ uint32_t s_dfa[LEX_MAX_DFA];
-  __shared__ uint8_t s_cls[256];
+__global__ void __launch_bounds__(LEX_CT_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(SHORT ? 4 : 8)))
+lex_emit(LexArgs p) {
+  __shared__ uint8_t s_cls[256];  // one word per bank: look-ups never conflict
   __shared__ uint32_t s_wcnt[LEX_CT_WAVES];
   __shared__ int32_t s_wlast[LEX_CT_WAVES];
   __shared__ uint32_t s_wreset[LEX_CT_WAVES];
   __shared__ uint32_t s_ctile;
   __shared__ uint32_t s_cpre;  // the count tile's look-back prefix (count, last start)
   __shared__ int32_t s_lpre;
-  __shared__ uint32_t s_stage[LEX_CT_WAVES][2][LEX_STAGE];  // starts, ends
-  __shared__ uint8_t s_kind[LEX_CT_WAVES][LEX_STAGE];
+  __shared__ __align__(16) uint32_t s_lab[LEX_CT_WAVES][LEX_TILE / 4];  // label after every byte
+  __shared__ uint32_t s_stage[LEX_CT_WAVES][LEX_STAGE];  // last byte | start << 16, from the tile
+  extern __shared__ __align__(16) uint8_t smem[];  // the walk words, then (SHORT) endo_step
+  uint32_t *const s_dfa = reinterpret_cast<uint32_t *>(smem);
   const uint32_t C = p.C;
-  if (DFA_LDS)
-    for (uint32_t i = threadIdx.x; i < p.m1 * C; i += blockDim.x) s_dfa[i] = p.dfa_walk[i];
-  // walk words (the next state's row as a byte offset, kept / boundary / accept bits, label)
-  const uint8_t *dfa = reinterpret_cast<const uint8_t *>(DFA_LDS ? s_dfa : p.dfa_walk);
-#define LEX_WALK(ROW4, CL) (*reinterpret_cast<const uint32_t *>(dfa + (ROW4) + ((CL) << 2)))
-  const uint32_t C4 = C << 2;
+  if (DFA_LDS)  // rows as byte offsets
+    for (uint32_t i = threadIdx.x; i < p.m1 * C; i += blockDim.x) {
+      const uint32_t x = p.dfa_walk[i];
+      s_dfa[i] = x + (x & 0xFFFF0000u) * 3u;
+    }
   for (uint32_t i = threadIdx.x; i < 256; i += blockDim.x) s_cls[i] = p.byte_class[i];
-  extern __shared__ __align__(16) uint8_t smem[];
-  const uint16_t *s_step = reinterpret_cast<const uint16_t *>(smem);
+  // The walk word of the state whose row is `row` (in bytes in LDS, else in words) for class c.
+  auto walk = [&](uint32_t row, uint32_t c) -> uint32_t {
+    if (DFA_LDS)
+      return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(s_dfa) + row +
+                                                 (c << 2));
+    return p.dfa_walk[row + c];
+  };
+  const uint32_t dfa_bytes = DFA_LDS ? (4 * p.m1 * C + 15) & ~15u : 0u;
+  const uint16_t *s_step = reinterpret_cast<const uint16_t *>(smem + dfa_bytes);
   if (SHORT) {
-    table_to_lds(smem, p.endo_step, 2 * p.e * C);
+    table_to_lds(smem + dfa_bytes, p.endo_step, 2 * p.e * C);
     // the words that the parser counts in; the verdict and the count are written below
     if (threadIdx.x < 16 && p.clear + threadIdx.x != p.result && p.clear + threadIdx.x != p.result + 1)
       p.clear[threadIdx.x] = p.clear + threadIdx.x == p.result + 2 ? p.timeout0 : 0u;
@@ -808,8 +888,10 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
   const uint64_t tbase = (uint64_t)tv.ltile * LEX_TILE;
   const uint64_t base = tbase + (uint64_t)lane * LEX_IPT;
   const int valid = (tile >= p.num_tiles || base >= n) ? 0 : (int)min((uint64_t)LEX_IPT, n - base);
-  uint32_t cls[LEX_IPT / 4];
-  load_classes(tv.ptr, tv.aligned, s_cls, base, valid, cls, tv.n);
+  uint32_t wds[LEX_IPT / 4];
+  load_words(tv.ptr, tv.aligned, base, valid, n, wds);
+  // class of the lane's byte j (j a constant)
+#define LEX_C(j) ((uint32_t)s_cls[(wds[(j) >> 2] >> (8 * ((j)&3))) & 0xFFu])
   uint32_t s_lane = 0;
   uint32_t s_tile = 0;
   if (SHORT) {
@@ -817,9 +899,9 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     uint32_t x = 0;
 #pragma unroll
     for (int j = 0; j < LEX_IPT; ++j)
-      if (j < valid) x = s_step[__umul24(x, C) + LEX_CLS(j)];
+      if (j < valid) x = s_step[__umul24(x, C) + LEX_C(j)];
     uint32_t total = lex_lane_scan(p.endo_comp, p.e, lane, x);
-    uint32_t *s_tmp = &s_stage[0][0][0];
+    uint32_t *s_tmp = &s_stage[0][0];
     if (lane == 0) s_tmp[w] = total;
     __syncthreads();
     if (w == 0) {
@@ -829,74 +911,80 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     __syncthreads();
     s_lane = p.endo_apply[x * p.m1 + s_tmp[LEX_CT_WAVES + w]];
   }
-  if (!SHORT && !BATCH && p.self_scan) s_tile = tile_start_state(p, ct, w, lane, &s_stage[0][0][0]);
+  if (!SHORT && !BATCH && p.self_scan) s_tile = tile_start_state(p, ct, w, lane, &s_stage[0][0]);
   if (!SHORT && tile < p.num_tiles) {
     if (BATCH || !p.self_scan) s_tile = p.tile_state[tile];
     const uint32_t ex = p.lane_excl[(uint64_t)tile * WAVE + lane];
     s_lane = p.endo_apply[ex * p.m1 + s_tile];
   }
-  uint32_t c_next = __shfl_down(LEX_CLS(0), 1, WAVE);
-  if (lane == WAVE - 1) {
-    const uint64_t nb = tbase + LEX_TILE;
-    c_next = nb < n ? s_cls[tv.ptr[nb]] : 0u;
-  }
+  // the byte after the lane's (any byte past the document's end)
+  uint32_t b_next = (uint32_t)dpp_i32<DPP_WAVE_SHL1>(0, (int32_t)(wds[0] & 0xFFu));
+  if (lane == WAVE - 1 && tbase + LEX_TILE < n) b_next = tv.ptr[tbase + LEX_TILE];
 
   // ---- one walk: token-end mask, token-start mask and the label after every byte
   uint32_t endm = 0, startm = 0;
-  uint32_t labs[LEX_IPT / 4] = {0, 0, 0, 0, 0, 0, 0, 0};
   uint32_t acc_end = 0;  // whether the state after the document's last byte accepts
   uint32_t lab_end = 0;
+  const uint8_t *lab8 = reinterpret_cast<const uint8_t *>(s_lab[w]);  // by position in the tile
   // the lane holding its document's last byte (no byte follows it)
   const bool doc_last = valid > 0 && base + (uint64_t)valid == n;
+  const uint32_t row0 = __umul24(s_lane, DFA_LDS ? C << 2 : C);
   if (valid > 0) {
-    // every lane walks all its 32 classes, a document's last lane too (class 0 past the end, and
-    // c_next is 0 there), so that no wave runs a second, bounds-checked walk for one lane; the
-    // marks past the document's end are cleared below. x_j, the word that took byte j, gives the
-    // label of byte j (bits 24-30) and whether it is kept (bit 18); x_{j+1} whether a token
-    // boundary follows byte j (bit 19). A token ends at j where a boundary follows a kept byte and
-    // starts at j + 1 where a boundary precedes a kept byte: two bit masks, ANDed after the walk.
-    uint32_t x = LEX_WALK(__umul24(s_lane, C4), LEX_CLS(0));
-    const uint32_t start0 = (x >> 19) & (x >> 18) & 1u;
-    uint32_t pm = 0, km = 0;
+    // every lane walks all its 32 bytes, a document's last lane too, so that no wave runs a second,
+    // bounds-checked walk for one lane; the marks past the document's end are cleared below. x_j,
+    // the word that took byte j, tells whether a token boundary falls before byte j (bit 0), and the
+    // label of byte j and whether it is kept (byte 1 and its top bit). A token ends at j where a
+    // boundary follows a kept byte and starts at j where a boundary precedes one. Per byte that is
+    // the class address, the row address and one v_alignbit_b32 that shifts bit 0 into the boundary
+    // mask; labels are packed four at a time and their top bits gathered by v_dot4_u32_u8.
+    // (902 -> 623 VALU and 488 -> 176 scalar instructions per wavefront with the staging below.)
+    uint32_t row = row0, bm = 0, km = 0;
+    uint32_t labs[LEX_IPT / 4];
     uint32_t xs[4];
+    // the classes of eight bytes are read while the eight before them are walked: read in between the
+    // steps they would lengthen each step's wait (LDS answers in order)
+    uint32_t cl[2][8];
 #pragma unroll
-    for (int j = 0; j < LEX_IPT; ++j) {
-      km |= ((x >> 18) & 1u) << j;
-      xs[j & 3] = x;
-      if ((j & 3) == 3) {
-        // the labels of bytes j-3 .. j: byte 3 of their four words
-        const uint32_t t01 = __builtin_amdgcn_perm(xs[1], xs[0], 0x0c0c0703u);
-        const uint32_t t23 = __builtin_amdgcn_perm(xs[3], xs[2], 0x0c0c0703u);
-        labs[j >> 2] = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
+    for (int j = 0; j < 8; ++j) cl[0][j] = LEX_C(j);
+#pragma unroll
+    for (int g = 0; g < LEX_IPT / 8; ++g) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (g + 1 < LEX_IPT / 8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) cl[(g + 1) & 1][j] = LEX_C((8 * (g + 1) + j) & (LEX_IPT - 1));
       }
-      const uint32_t cn = j + 1 < LEX_IPT ? LEX_CLS((j + 1) & (LEX_IPT - 1)) : c_next;
-      const uint32_t x2 = LEX_WALK(x & 0x3FFFFu, cn);
-      pm |= ((x2 >> 19) & 1u) << j;
-      if (j + 1 < LEX_IPT) x = x2;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int j = 8 * g + k;
+        const uint32_t x = walk(row, cl[g & 1][k]);
+        row = x >> 16;
+        bm = __builtin_amdgcn_alignbit(x, bm, 1);
+        xs[j & 3] = x;
+        if ((j & 3) == 3) {
+          const uint32_t t01 = __builtin_amdgcn_perm(xs[1], xs[0], 0x0c0c0501u);
+          const uint32_t t23 = __builtin_amdgcn_perm(xs[3], xs[2], 0x0c0c0501u);
+          const uint32_t t = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
+          km |= __builtin_amdgcn_udot4((t >> 7) & 0x01010101u, 0x08040201u, 0u, false) << (j - 3);
+          labs[j >> 2] = t & 0x7F7F7F7Fu;
+        }
+      }
     }
-    endm = pm & km;
-    startm = start0 | ((pm << 1) & km);
-    acc_end = (x >> 20) & 1u;
-    lab_end = x >> 24;
+    acc_end = (xs[3] >> 1) & 1u;
+    const uint32_t after = walk(row, s_cls[b_next]) & 1u;
+    endm = ((bm >> 1) | (after << 31)) & km;
+    startm = bm & km;
+    uint4 *lab4 = reinterpret_cast<uint4 *>(s_lab[w]) + 2 * lane;
+    lab4[0] = make_uint4(labs[0], labs[1], labs[2], labs[3]);
+    lab4[1] = make_uint4(labs[4], labs[5], labs[6], labs[7]);
     if (doc_last) {
       // tokens start only inside the document, and its last byte ends no token here (the final
-      // token is appended below); its label is the one after byte valid - 1. Whether the state
-      // after that byte accepts is walked again once the count tile's total is out (below).
+      // token is appended below). Whether the state after that byte accepts is walked again once the
+      // count tile's total is out (below).
       const uint32_t keep = valid == LEX_IPT ? 0xFFFFFFFFu : (1u << valid) - 1u;
       startm &= keep;
       endm &= keep >> 1;
-      uint32_t lw;
-      switch ((valid - 1) >> 2) {  // a register array takes constant indexes only
-        case 0: lw = labs[0]; break;
-        case 1: lw = labs[1]; break;
-        case 2: lw = labs[2]; break;
-        case 3: lw = labs[3]; break;
-        case 4: lw = labs[4]; break;
-        case 5: lw = labs[5]; break;
-        case 6: lw = labs[6]; break;
-        default: lw = labs[7]; break;
-      }
-      lab_end = (lw >> (8 * ((valid - 1) & 3))) & 0xFFu;
+      lab_end = lab8[lane * LEX_IPT + valid - 1];
     }
   }
   uint32_t lastm = 0;  // CHUNKED: chunk-last positions of this lane
@@ -907,14 +995,15 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     endm &= ~lastm;
   }
   const uint32_t cnt = __popc(endm);
-  const int32_t last = startm ? (int32_t)(base + 31 - __clz(startm)) : -1;
+  // last token start of the lane, from the tile's first byte
+  const int32_t last = startm ? (int32_t)(lane * LEX_IPT + 31 - __clz(startm)) : -1;
 
   // ---- scans: wave, count tile, across count tiles
   const uint32_t cincl = (uint32_t)wave_incl_i32((int32_t)cnt, 0, OpAdd());
   const int32_t lincl = wave_incl_i32(last, -1, OpMax());
   if (lane == WAVE - 1) {
     s_wcnt[w] = cincl;
-    s_wlast[w] = lincl;
+    s_wlast[w] = lincl < 0 ? -1 : (int32_t)tbase + lincl;
     // a wave tile that starts a document restarts the count and the last start
     s_wreset[w] = (tile < p.num_tiles && tv.ltile == 0) ? 1u : 0u;
   }
@@ -949,7 +1038,12 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     const int32_t ltot = __builtin_amdgcn_readlane(wli, LEX_CT_WAVES - 1);
     const bool ftot = __builtin_amdgcn_readlane(wfi, LEX_CT_WAVES - 1) != 0;
     // a count tile holding a document start already has its (post-reset) inclusive value
-    if (!SHORT && lane == 0) st_relaxed64(p.st_count + ct, pack_count(ctot, ltot, ftot ? CT_INC : CT_AGG));
+    if (!SHORT && lane == 0) {
+      st_relaxed64(p.st_count + ct, pack_count(ctot, ltot, ftot ? CT_INC : CT_AGG));
+      // its group's word too, when the group's last tile needs no other for it
+      if (ftot && ct % WAVE == WAVE - 1)
+        st_relaxed64(p.st_group + ct / WAVE, pack_count(ctot, ltot, CT_INC));
+    }
     ct_tot = ctot;
     ct_last = ltot;
     ct_reset = ftot;
@@ -972,31 +1066,28 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
   // a document's last lane ending inside its 32 bytes: whether the state after its last byte
   // accepts (the walk above went on over class 0), walked now that the count tile's total is out
   if (doc_last && valid < LEX_IPT) {
-    uint32_t x = LEX_WALK(__umul24(s_lane, C4), LEX_CLS(0));
+    uint32_t x = walk(row0, LEX_C(0));
 #pragma unroll
     for (int j = 1; j < LEX_IPT - 1; ++j)
-      if (j < valid) x = LEX_WALK(x & 0x3FFFFu, LEX_CLS(j));
-    acc_end = (x >> 20) & 1u;
+      if (j < valid) x = walk(x >> 16, LEX_C(j));
+    acc_end = (x >> 1) & 1u;
   }
   __syncthreads();
 
   // ---- write tokens: stage in LDS by wave-local index, copy out coalesced, in rounds. The first
-  // round is staged before the look-back, so that its wait overlaps the staging; a lane whose
-  // first token began before the count tile stages START_PENDING and the copy takes the
-  // look-back's last start instead.
-  constexpr uint32_t START_PENDING = 0xFFFFFFFFu;  // positions stay below 2^31
+  // round is staged before the look-back, so that its wait overlaps the staging. A staged token is its
+  // last byte and its start, both from the tile's first byte (LEX_BEFORE: a token of the wavefront's
+  // first one that began before the tile; the copy takes the start that the count tile, or the
+  // look-back, knows); its kind is the label after its last byte.
+  constexpr uint32_t LEX_BEFORE = 0xFFFFu;
   const bool takes_prefix = s_wreset[w] != 0;
   const uint32_t wtotal = (uint32_t)__builtin_amdgcn_readlane((int32_t)cincl, WAVE - 1);
   const uint32_t lofs = cincl - cnt;                // wave-local index of this lane's first token
   const int32_t lexcl = wave_prev_i32(lincl, -1);
-  const int32_t last_in_tile = max(s_wlast[w], lexcl);
-  uint32_t start_in = last_in_tile >= 0 ? (uint32_t)last_in_tile
-                                        : (takes_prefix ? START_PENDING : 0u);
-  uint32_t pending_start = 0;
-  uint32_t wout = 0;  // slot of the wave's first token
-  uint8_t *stk = s_kind[w];
-  uint32_t *sts = s_stage[w][0];
-  uint32_t *ste = s_stage[w][1];
+  const uint32_t start_in = lexcl >= 0 ? (uint32_t)lexcl : LEX_BEFORE;
+  uint32_t before = 0;  // start of a token that began before the tile
+  uint32_t wout = 0;    // slot of the wave's first token
+  uint32_t *stage = s_stage[w];
   for (uint32_t r0 = 0;; r0 += LEX_STAGE) {
     const bool any = r0 < wtotal;  // uniform in the wave
     if (any) {
@@ -1009,25 +1100,11 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
         k += skip;
       }
       while (em && k < r0 + LEX_STAGE) {
-        const int j = __ffs(em) - 1;
+        const uint32_t j = (uint32_t)__builtin_ctz(em);
         em &= em - 1;
-        const uint32_t sm = startm & (j == 31 ? 0xFFFFFFFFu : ((2u << j) - 1u));
-        const uint32_t cur = sm ? (uint32_t)(base + 31 - __clz(sm)) : start_in;
-        uint32_t lw;
-        switch (j >> 2) {
-          case 0: lw = labs[0]; break;
-          case 1: lw = labs[1]; break;
-          case 2: lw = labs[2]; break;
-          case 3: lw = labs[3]; break;
-          case 4: lw = labs[4]; break;
-          case 5: lw = labs[5]; break;
-          case 6: lw = labs[6]; break;
-          default: lw = labs[7]; break;
-        }
-        const uint32_t o = k - r0;
-        stk[o] = (uint8_t)(lw >> (8 * (j & 3)));
-        sts[o] = cur;
-        ste[o] = (uint32_t)(base + j + (CHUNKED ? 0 : 1));
+        const uint32_t sm = startm << (31 - j);  // the starts up to byte j, the last one on top
+        const uint32_t st = sm ? (uint32_t)lane * LEX_IPT + j - (uint32_t)__builtin_clz(sm) : start_in;
+        stage[k - r0] = ((uint32_t)lane * LEX_IPT + j) | (st << 16);
         ++k;
       }
     }
@@ -1036,11 +1113,7 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
       if (w == 0) {
         uint32_t cpre = 0;
         int32_t lpre = -1;
-        if (need_lb) {
-          lookback_count(p, ct, lane, cpre, lpre);
-          if (lane == 0 && !ct_reset)
-            st_relaxed64(p.st_count + ct, pack_count(cpre + ct_tot, max(lpre, ct_last), CT_INC));
-        }
+        if (need_lb) lookback_count(p, ct, lane, ct_tot, ct_last, ct_reset, cpre, lpre);
         if (lane == 0) {
           s_cpre = cpre;
           s_lpre = lpre;
@@ -1050,34 +1123,33 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
       const uint32_t cpre = takes_prefix ? s_cpre : 0u;
       const int32_t lpre = takes_prefix ? s_lpre : -1;
       wout = (uint32_t)tv.tok_base + s_wcnt[w] + cpre;
-      pending_start = (uint32_t)max(lpre, 0);
-      if (start_in == START_PENDING) start_in = pending_start;
+      before = (uint32_t)max(s_wlast[w] >= 0 ? s_wlast[w] : lpre, 0);
     }
     if (!any) break;
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
     const uint32_t m = min((uint32_t)LEX_STAGE, wtotal - r0);
     for (uint32_t i = lane; i < m; i += WAVE) {
       const uint64_t g = (uint64_t)wout + r0 + i;
-      uint32_t sv = sts[i];
-      if (sv == START_PENDING) sv = pending_start;
-      if (!CHUNKED && p.kinds8) p.kinds8[g] = stk[i];
-      else p.kinds[g] = stk[i];
+      const uint32_t tk = stage[i];
+      const uint32_t at = tk & 0xFFFFu;
+      const uint32_t sv = (tk >> 16) == LEX_BEFORE ? before : (uint32_t)tbase + (tk >> 16);
+      const uint32_t kind = lab8[at];
+      if (!CHUNKED && p.kinds8) p.kinds8[g] = (uint8_t)kind;
+      else p.kinds[g] = kind;
       if (CHUNKED) {
         uint64_t cs, ce;
-        chunk_span(p, sv, ste[i], cs, ce);
+        chunk_span(p, sv, (uint32_t)tbase + at, cs, ce);
         p.starts64[g] = cs;
         p.ends64[g] = ce;
       } else {
         p.starts[g] = sv;
-        p.ends[g] = ste[i];
+        p.ends[g] = (uint32_t)tbase + at + 1;
       }
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
   }
+  // the start of a token that began before this lane
+  const uint32_t cur_in = lexcl >= 0 ? (uint32_t)tbase + (uint32_t)lexcl : before;
   // ---- CHUNKED: the last element of every chunk that ends in this lane
   if (CHUNKED) {
     uint32_t lm = lastm;
@@ -1086,24 +1158,13 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
       lm &= lm - 1;
       const uint32_t le = j == 31 ? 0xFFFFFFFFu : ((2u << j) - 1u);
       const uint32_t sm = startm & le;
-      const uint32_t cur = sm ? (uint32_t)(base + 31 - __clz(sm)) : (uint32_t)start_in;
-      uint32_t lw;
-      switch (j >> 2) {
-        case 0: lw = labs[0]; break;
-        case 1: lw = labs[1]; break;
-        case 2: lw = labs[2]; break;
-        case 3: lw = labs[3]; break;
-        case 4: lw = labs[4]; break;
-        case 5: lw = labs[5]; break;
-        case 6: lw = labs[6]; break;
-        default: lw = labs[7]; break;
-      }
+      const uint32_t cur = sm ? (uint32_t)(base + 31 - __clz(sm)) : cur_in;
       const uint32_t v = (uint32_t)(base + j);
       uint64_t cs, ce;
       chunk_span(p, cur, v, cs, ce);
       uint64_t *ci = p.chunk_info + 4ull * (v / (p.chunk + 1));
       ci[0] = (uint64_t)wout + lofs + __popc(endm & le);
-      ci[1] = (lw >> (8 * (j & 3))) & 0xFFu;
+      ci[1] = lab8[lane * LEX_IPT + j];
       ci[2] = cs;
       ci[3] = ce;
     }
@@ -1111,7 +1172,7 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
   // ---- the lane holding the last byte appends the final token and decides acceptance
   if (valid > 0 && base + (uint64_t)valid == n) {
     const uint32_t out = wout + wtotal;
-    int32_t cur = start_in;
+    int32_t cur = (int32_t)cur_in;
     if (startm) cur = (int32_t)(base + 31 - __clz(startm));
     uint32_t total = out;
     if (CHUNKED) {
@@ -1151,7 +1212,7 @@ __global__ void __launch_bounds__(LEX_BLOCK) lex_emit(LexArgs p) {
     }
   }
 }
-#undef LEX_WALK
+#undef LEX_C
 
 // Chunked mode: in lex_step every element that ends no token is scattered to prev_size - 1
 // (lexer.fut:108-111, 131-132), the last token of the chunks before; with several such elements
@@ -3406,10 +3467,15 @@ void launch_lex_reduce(int tab, unsigned blocks, size_t lds, const LexArgs &a, h
   else lex_reduce<0, BATCH><<<blocks, LEX_BLOCK, lds, st>>>(a);
 }
 
+// dynamic LDS of lex_emit's walk words
+inline size_t lex_dfa_lds(uint32_t m1, uint32_t C) { return (4 * (size_t)m1 * C + 15) & ~(size_t)15; }
+
 template <bool CHUNKED, bool BATCH>
 void launch_lex_emit(bool dfa_lds, unsigned grid, const LexArgs &a, hipStream_t st) {
-  if (dfa_lds) lex_emit<CHUNKED, BATCH, true><<<grid, LEX_BLOCK, 0, st>>>(a);
-  else lex_emit<CHUNKED, BATCH, false><<<grid, LEX_BLOCK, 0, st>>>(a);
+  const size_t lds = lex_dfa_lds(a.m1, a.C);
+  constexpr unsigned threads = LEX_CT_WAVES * WAVE;
+  if (dfa_lds) lex_emit<CHUNKED, BATCH, true><<<grid, threads, lds, st>>>(a);
+  else lex_emit<CHUNKED, BATCH, false><<<grid, threads, 0, st>>>(a);
 }
 
 // BS: workgroup size (one 64-element chunk per wavefront and iteration, whatever the size)
@@ -3734,7 +3800,7 @@ int fill_levels(alpacc_ctx *ctx, const Levels &la, const Levels &lb, hipStream_t
 // endomorphisms, the tile and scan-block endomorphisms, the tile start states and the look-back
 // words of the count scan.
 struct LexScratch {
-  uint32_t *small;       // 16 words: [0] count-tile counter, [4..6] accept, tokens, time-out
+  uint32_t *small;       // 16 words: [4..6] accept, tokens, time-out, [8..11] the parser's flags
   uint16_t *lane_excl;   // [tiles * 64]
   uint16_t *tile_agg;    // [tiles]
   uint16_t *tile_excl;   // [tiles]
@@ -3752,7 +3818,7 @@ constexpr uint64_t lex_scratch_bytes(uint64_t n) {
          2 * align256(((n + LEX_TILE - 1) / LEX_TILE) * 2) +
          align256((((n + LEX_TILE - 1) / LEX_TILE + LEX_SCAN_BLOCK - 1) / LEX_SCAN_BLOCK) * 2) +
          align256((n + LEX_TILE - 1) / LEX_TILE) +
-         align256((((n + LEX_TILE - 1) / LEX_TILE + LEX_CT_WAVES - 1) / LEX_CT_WAVES) * 8);
+         align256(lb_words(((n + LEX_TILE - 1) / LEX_TILE + LEX_CT_WAVES - 1) / LEX_CT_WAVES) * 8);
 }
 
 void lex_scratch_carve(uint8_t *base, uint64_t n, LexScratch &s) {
@@ -3771,7 +3837,7 @@ void lex_scratch_carve(uint8_t *base, uint64_t n, LexScratch &s) {
   s.tile_excl = (uint16_t *)take(tiles * 2);
   s.block_agg = (uint16_t *)take(sblocks * 2);
   s.tile_state = take(tiles);
-  s.st_count = (uint64_t *)take(ctiles * 8);
+  s.st_count = (uint64_t *)take(lb_words(ctiles) * 8);
 }
 
 }  // namespace
@@ -3879,7 +3945,7 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     sc.tile_excl = (uint16_t *)ctx->buf(B_TILE_EXCL, tiles * sizeof(uint16_t));
     sc.block_agg = (uint16_t *)ctx->buf(B_BLOCK_AGG, sblocks * sizeof(uint16_t));
     sc.tile_state = (uint8_t *)ctx->buf(B_TILE_STATE, tiles);
-    sc.st_count = (uint64_t *)ctx->buf(B_ST_COUNT, ctiles * sizeof(uint64_t));
+    sc.st_count = (uint64_t *)ctx->buf(B_ST_COUNT, lb_words(ctiles) * sizeof(uint64_t));
   }
   uint32_t *small = sc.small;
   uint16_t *lane_excl = sc.lane_excl, *tile_agg = sc.tile_agg, *tile_excl = sc.tile_excl;
@@ -3916,8 +3982,9 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   a.tile_excl = tile_excl;
   a.block_agg = block_agg;
   a.tile_state = tile_state;
-  a.tile_counter = small;
+  a.tile_counter = (uint32_t *)(st_count + lb_words(ctiles) - LB_TICKET);
   a.st_count = st_count;
+  a.st_group = st_count + ctiles;
   a.result = small + 4;
   a.clear = small;
   a.timeout0 = ctx->force_timeout ? 1u : 0u;
@@ -3940,9 +4007,10 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   const uint64_t wpb = LEX_BLOCK / WAVE;
   uint64_t blocks = (tiles + wpb - 1) / wpb;
   blocks = std::min<uint64_t>(blocks, (uint64_t)std::max(1, ctx->cus) * ctx->lex_bpc);
-  if (chunk == 0 && ctiles == 1 && ctx->lex_short) {
+  if (chunk == 0 && tiles <= LEX_CT_WAVES && ctx->lex_short) {
     ctx->prof_begin(S_LEX_EMIT, st);
-    lex_emit<false, false, true, true><<<1, LEX_BLOCK, 2 * ctx->e * ctx->C, st>>>(a);
+    lex_emit<false, false, true, true>
+        <<<1, LEX_CT_WAVES * WAVE, lex_dfa_lds(ctx->m1, ctx->C) + 2 * ctx->e * ctx->C, st>>>(a);
     ctx->prof_end(S_LEX_EMIT, st);
     ctx->launches++;
     CK(hipGetLastError());
@@ -4044,7 +4112,8 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
   a.lane_excl = (uint16_t *)ctx->buf(B_LANE_EXCL, tiles * WAVE * sizeof(uint16_t));
   a.tile_agg = (uint16_t *)ctx->buf(B_TILE_AGG, tiles * sizeof(uint16_t));
   a.tile_state = (uint8_t *)ctx->buf(B_TILE_STATE, tiles);
-  a.st_count = (uint64_t *)ctx->buf(B_ST_COUNT, ctiles * sizeof(uint64_t));
+  a.st_count = (uint64_t *)ctx->buf(B_ST_COUNT, lb_words(ctiles) * sizeof(uint64_t));
+  a.st_group = a.st_count + ctiles;
   a.tile_doc = (uint32_t *)ctx->buf(B_TILE_DOC, tiles * sizeof(uint32_t));
   a.tile_rec = (uint4 *)ctx->buf(B_TILE_REC, tiles * sizeof(uint4));
   a.chunks = (uint2 *)ctx->buf(B_CHUNKS, chunks * sizeof(uint2));
@@ -4073,7 +4142,7 @@ int plan_lex_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offsets
   a.ignore = ctx->ignore;
   a.num_tiles = (uint32_t)tiles;
   a.num_ctiles = (uint32_t)ctiles;
-  a.tile_counter = pl.small;
+  a.tile_counter = (uint32_t *)(a.st_count + lb_words(ctiles) - LB_TICKET);
   a.result = pl.small + 4;
   a.clear = pl.small;
   a.timeout0 = ctx->force_timeout ? 1u : 0u;
@@ -5018,9 +5087,9 @@ int place_lexer_tables(alpacc_ctx *ctx, std::string &err) {
     lds = 256;
   }
   ctx->dfa_lds = ctx->lex_tables_lds && (size_t)ctx->m1 * ctx->C <= (size_t)LEX_MAX_DFA;
-  // lex_emit's own LDS is 72 KB
-  const size_t step = (size_t)2 * ctx->e * ctx->C;
-  ctx->lex_short = ctx->lex_tab >= 1 && ctx->dfa_lds && step <= 80 * 1024;
+  // lex_emit's own LDS is 57 KB there
+  const size_t step = lex_dfa_lds(ctx->m1, ctx->C) + (size_t)2 * ctx->e * ctx->C;
+  ctx->lex_short = ctx->lex_tab >= 1 && ctx->dfa_lds && step <= 96 * 1024;
   if (ctx->lex_short &&
       hipFuncSetAttribute((const void *)lex_emit<false, false, true, true>,
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)step) != hipSuccess) {
@@ -5364,11 +5433,10 @@ alpacc_ctx *alpacc_create(const alpacc_tables *t, int device) {
     ctx->d_comp = upload(t->endo_comp, (size_t)ctx->e * ctx->e, err);
     ctx->d_apply = upload(t->endo_apply, (size_t)ctx->e * ctx->m1, err);
     {
-      // lex_emit's walk table, one word per (state, class) of dfa_step: the next state's row
-      // as a byte offset into this table (bits 0-17: at most 255 x 256 x 4), whether the label of
-      // the byte is kept (not the ignored terminal; bit 18), whether a token boundary falls before
-      // the byte (the produce bit; bit 19), whether the next state accepts (bit 20) and the label
-      // (bits 24-30).
+      // lex_emit's walk table, one word per (state, class) of dfa_step: whether a token boundary
+      // falls before the byte (the produce bit; bit 0), whether the next state accepts (bit 1), the
+      // label of the byte (bits 8-14) and whether it is kept (not the ignored terminal; bit 15), and
+      // the first word of the next state's row (bits 16-31: at most 255 x 256).
       const size_t nw = (size_t)ctx->m1 * ctx->C;
       std::vector<uint32_t> walk(nw);
       for (size_t i = 0; i < nw && err.empty(); ++i) {
@@ -5379,8 +5447,8 @@ alpacc_ctx *alpacc_create(const alpacc_tables *t, int device) {
           break;
         }
         const bool kept = ctx->ignore < 0 || lab != (uint32_t)ctx->ignore;
-        walk[i] = ns * ctx->C * 4u | (kept ? 1u << 18 : 0u) | prod << 19 |
-                  (t->state_accept[ns] ? 1u << 20 : 0u) | lab << 24;
+        walk[i] = prod | (t->state_accept[ns] ? 2u : 0u) | lab << 8 | (kept ? 1u << 15 : 0u) |
+                  (ns * ctx->C) << 16;
       }
       if (err.empty()) ctx->d_walk = upload(walk.data(), nw, err);
     }
