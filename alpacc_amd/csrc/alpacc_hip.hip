@@ -179,9 +179,10 @@ struct LexArgs {
   uint32_t *clear;            // the 16 words (results, parser flags) that lex_reduce clears
   uint32_t timeout0;          // what it sets the timeout flag to (testing hook)
   uint32_t *host_result;      // when set: pinned host copy of result
-  // chunked mode (the reference's chunk loop, lexer.fut:144-172): `in` is the virtual string in
-  // which every chunk [j*chunk, min(j*chunk + chunk + 1, n_orig)) is laid end to end, so the byte
-  // shared by two neighbouring chunks appears twice.
+  // chunked mode (the reference's chunk loop, lexer.fut:144-172): n and all positions are those of
+  // the virtual string in which every chunk [j*chunk, min(j*chunk + chunk + 1, n_orig)) is laid end to
+  // end, so the byte shared by two neighbouring chunks appears twice; `in` is the original string,
+  // which the loads map to (laying it out took 46 us for 48 MiB).
   uint32_t chunk;             // chunk size in bytes of the original string
   uint32_t nchunks;           // K = ceil(n_orig / chunk)
   uint64_t n_orig;
@@ -388,6 +389,31 @@ __device__ __forceinline__ void load_words(const uint8_t *in, bool aligned, uint
   }
 }
 
+// Chunked mode: the same for 32 bytes of the virtual string in which every chunk of cp1 - 1 bytes
+// is followed by the first byte of the next one, read from the original string of n bytes (virtual
+// position v is byte v - v / cp1 of it). A lane inside one chunk reads it like any document off a
+// 16-byte boundary; one that a chunk ends in gathers its bytes.
+__device__ __forceinline__ void load_words_chunked(const uint8_t *in, uint64_t n, uint32_t cp1,
+                                                   uint32_t base, int valid,
+                                                   uint32_t (&wds)[LEX_IPT / 4]) {
+  const uint32_t j0 = base / cp1;
+  const bool inside = valid > 0 && base + (uint32_t)valid - 1 - j0 * cp1 < cp1;
+  if (inside) {
+    const uint8_t *q = in + (base - j0);
+    load_words(in, valid == LEX_IPT && ((uintptr_t)q & 15) == 0, base - j0, valid, n, wds);
+  } else {
+#pragma unroll
+    for (int k = 0; k < LEX_IPT / 4; ++k) {
+      wds[k] = 0u;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const uint32_t v = base + 4 * k + b;
+        if (4 * k + b < valid) wds[k] |= (uint32_t)in[v - v / cp1] << (8 * b);
+      }
+    }
+  }
+}
+
 // The wave-exclusive composition of the lanes' endomorphisms v (Blelloch up- and down-sweep over
 // the (endo x endo) table) in v; returns the wavefront's total.
 __device__ __forceinline__ uint32_t lex_lane_scan(const uint16_t *comp_tab, uint32_t e, int lane,
@@ -433,7 +459,8 @@ __device__ __forceinline__ uint32_t lex_row_scan(const LexArgs &p, int lane, uin
 // (endo x endo) table, 126 lookups per wave). Persistent, grid-stride over wave tiles.
 // TAB: where the tables sit: 2 = both in LDS, 1 = the (endo x class) table in LDS and the
 // composition table in L2, 0 = both in L2 (an (endo x class) table larger than LDS).
-template <int TAB, bool BATCH>
+// CHUNKED: the document is the virtual string of the chunked mode (load_words_chunked).
+template <int TAB, bool BATCH, bool CHUNKED = false>
 __global__ void __launch_bounds__(LEX_BLOCK) __attribute__((amdgpu_waves_per_eu(8)))
 lex_reduce(LexArgs p) {
   extern __shared__ __align__(16) uint8_t smem[];
@@ -467,7 +494,13 @@ lex_reduce(LexArgs p) {
         const TileView tv = tile_view<BATCH>(p, tile[h]);
         const uint64_t base = (uint64_t)tv.ltile * LEX_TILE + (uint64_t)lane * LEX_IPT;
         valid = base >= tv.n ? 0 : (int)min((uint64_t)LEX_IPT, tv.n - base);
-        load_classes(tv.ptr, tv.aligned, s_cls, base, valid, cls, tv.n);
+        if (CHUNKED) {  // (bytes past the end are not walked)
+          uint32_t wds[LEX_IPT / 4];
+          load_words_chunked(p.in, p.n_orig, p.chunk + 1, (uint32_t)base, valid, wds);
+          classes_of_words(wds, s_cls, cls);
+        } else {
+          load_classes(tv.ptr, tv.aligned, s_cls, base, valid, cls, tv.n);
+        }
       }
       uint32_t x = 0;
       if (valid == LEX_IPT) {
@@ -782,16 +815,23 @@ __device__ void lookback_count(const LexArgs &p, uint32_t ct, int lane, uint32_t
 }
 
 // The lexer state at the start of wave tile LEX_CT_WAVES * ct + w of a document of at most
-// LEX_SELF_TILES wave tiles, found by the count tile's workgroup itself: the tiles before it are
-// composed by a tree over its threads, its own 16 by a scan. That is 12 dependent look-ups, where
-// lex_scan_tiles, lex_scan_blocks and lex_tile_states are 22 and three launches: lex_emit takes
-// 3-5 us longer on a short document and the call 12 us less. Longer documents keep the scan kernels.
+// LEX_SELF_TILES wave tiles (16 MiB), found by the count tile's workgroup itself: the tiles before it
+// are composed by its threads, a run of up to 8 each, then a tree, its own 16 by a scan. That is 12 to
+// 19 dependent look-ups, where lex_scan_tiles, lex_scan_blocks and lex_tile_states are 22 and three
+// launches. lex calls: 4 MiB 35 us against 47, 16 MiB 58 against 66; at 48 MiB (runs of 24) 142
+// against 109, so longer documents keep the scan kernels.
 // s_tmp: LDS of 2 * LEX_CT_WAVES words. All threads of the workgroup take part.
-constexpr uint32_t LEX_SELF_TILES = LEX_CT_WAVES * WAVE;
+constexpr uint32_t LEX_SELF_TILES = 8 * LEX_CT_WAVES * WAVE;
 __device__ uint32_t tile_start_state(const LexArgs &p, uint32_t ct, int w, int lane, uint32_t *s_tmp) {
   const uint32_t first = ct * LEX_CT_WAVES;
-  if ((uint32_t)w * WAVE < first) {
-    uint32_t v = threadIdx.x < first ? p.tile_agg[threadIdx.x] : 0u;
+  // a thread's run of consecutive earlier tiles, then the threads' compositions
+  const uint32_t run = (first + LEX_CT_WAVES * WAVE - 1) / (LEX_CT_WAVES * WAVE);
+  if ((uint32_t)w * WAVE * run < first) {
+    uint32_t v = 0;
+    for (uint32_t k = 0; k < run; ++k) {
+      const uint32_t t = threadIdx.x * run + k;
+      if (t < first) v = k == 0 ? p.tile_agg[t] : comp_lookup(p.endo_comp, p.e, v, p.tile_agg[t]);
+    }
 #pragma unroll
     for (int d = 1; d < WAVE; d <<= 1) {
       const uint32_t left = __shfl(v, (lane - d) & (WAVE - 1), WAVE);
@@ -889,7 +929,8 @@ lex_emit(LexArgs p) {
   const uint64_t base = tbase + (uint64_t)lane * LEX_IPT;
   const int valid = (tile >= p.num_tiles || base >= n) ? 0 : (int)min((uint64_t)LEX_IPT, n - base);
   uint32_t wds[LEX_IPT / 4];
-  load_words(tv.ptr, tv.aligned, base, valid, n, wds);
+  if (CHUNKED) load_words_chunked(p.in, p.n_orig, p.chunk + 1, (uint32_t)base, valid, wds);
+  else load_words(tv.ptr, tv.aligned, base, valid, n, wds);
   // class of the lane's byte j (j a constant)
 #define LEX_C(j) ((uint32_t)s_cls[(wds[(j) >> 2] >> (8 * ((j)&3))) & 0xFFu])
   uint32_t s_lane = 0;
@@ -919,7 +960,10 @@ lex_emit(LexArgs p) {
   }
   // the byte after the lane's (any byte past the document's end)
   uint32_t b_next = (uint32_t)dpp_i32<DPP_WAVE_SHL1>(0, (int32_t)(wds[0] & 0xFFu));
-  if (lane == WAVE - 1 && tbase + LEX_TILE < n) b_next = tv.ptr[tbase + LEX_TILE];
+  if (lane == WAVE - 1 && tbase + LEX_TILE < n) {
+    const uint32_t nb = (uint32_t)(tbase + LEX_TILE);
+    b_next = CHUNKED ? p.in[nb - nb / (p.chunk + 1)] : tv.ptr[nb];
+  }
 
   // ---- one walk: token-end mask, token-start mask and the label after every byte
   uint32_t endm = 0, startm = 0;
@@ -1227,16 +1271,6 @@ __global__ void lex_chunk_fixup(LexArgs p) {
     p.kinds[c - 1] = (uint32_t)p.chunk_info[4ull * j + 1];
     p.starts64[c - 1] = p.chunk_info[4ull * j + 2];
     p.ends64[c - 1] = p.chunk_info[4ull * j + 3];
-  }
-}
-
-// Chunked mode: lay the chunks [j*chunk, min(j*chunk + chunk + 1, n)) end to end.
-__global__ void lex_chunk_expand(const uint8_t *in, uint32_t chunk, uint64_t nv, uint8_t *out) {
-  const uint32_t cp1 = chunk + 1;
-  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < nv;
-       v += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t vv = (uint32_t)v;
-    out[v] = in[vv - vv / cp1];
   }
 }
 
@@ -2378,8 +2412,9 @@ __device__ void pb_doc(const PArgs &a, uint32_t d) {
 
 // The tile scan in one workgroup, each thread over a run of consecutive tiles: in place of
 // pscan_reduce, pscan_top and pscan_down where the tiles are few (up to PSCAN_ONE_MAX), whose time is
-// their launches.
-constexpr uint64_t PSCAN_ONE_MAX = 16 * PSB;
+// their launches: a 2 MiB JSON parse 68 us against 83, 6 MiB 94 against 101; at 14 MiB one workgroup
+// takes longer, 147 against 132.
+constexpr uint64_t PSCAN_ONE_MAX = 8 * PSB;
 
 template <bool BATCH>
 __device__ __forceinline__ void pscan_one_run(const PArgs &a, SegTup *s_w,
@@ -3460,11 +3495,11 @@ inline unsigned grid_for(uint64_t n, unsigned block, unsigned cap = 1u << 16) {
 }
 
 // lex_reduce / lex_emit with the table placement chosen at context creation
-template <bool BATCH>
+template <bool BATCH, bool CHUNKED>
 void launch_lex_reduce(int tab, unsigned blocks, size_t lds, const LexArgs &a, hipStream_t st) {
-  if (tab == 2) lex_reduce<2, BATCH><<<blocks, LEX_BLOCK, lds, st>>>(a);
-  else if (tab == 1) lex_reduce<1, BATCH><<<blocks, LEX_BLOCK, lds, st>>>(a);
-  else lex_reduce<0, BATCH><<<blocks, LEX_BLOCK, lds, st>>>(a);
+  if (tab == 2) lex_reduce<2, BATCH, CHUNKED><<<blocks, LEX_BLOCK, lds, st>>>(a);
+  else if (tab == 1) lex_reduce<1, BATCH, CHUNKED><<<blocks, LEX_BLOCK, lds, st>>>(a);
+  else lex_reduce<0, BATCH, CHUNKED><<<blocks, LEX_BLOCK, lds, st>>>(a);
 }
 
 // dynamic LDS of lex_emit's walk words
@@ -3696,7 +3731,6 @@ enum BufId {
   B_SX,
   B_DL1,
   B_SL1,
-  B_VIRT,
   B_CHUNK_INFO,
   B_TOK_START64,
   B_TOK_END64,
@@ -3914,16 +3948,6 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     ctx->err = "the chunked lexer has no fixed-scratch form";
     return ALPACC_ERR_ARG;
   }
-  if (chunk > 0) {
-    uint8_t *virt = (uint8_t *)ctx->buf(B_VIRT, n + 16);
-    if (!virt) {
-      ctx->err = "scratch allocation failed";
-      return ALPACC_ERR_HIP;
-    }
-    lex_chunk_expand<<<grid_for(n, 256, 1u << 14), 256, 0, st>>>(d_in, (uint32_t)chunk, n, virt);
-    ctx->launches++;
-    d_in = virt;
-  }
   uint64_t *chunk_info = nullptr;
   if (chunk > 0) {
     chunk_info = (uint64_t *)ctx->buf(B_CHUNK_INFO, K * 4 * sizeof(uint64_t));
@@ -4017,7 +4041,8 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     return sync ? lex_verdict(ctx, num_tokens, st) : ALPACC_ACCEPT;
   }
   ctx->prof_begin(S_LEX_REDUCE, st);
-  launch_lex_reduce<false>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
+  if (chunk > 0) launch_lex_reduce<false, true>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
+  else launch_lex_reduce<false, false>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
   ctx->prof_end(S_LEX_REDUCE, st);
   ctx->prof_begin(S_LEX_SCAN, st);
   if (!a.self_scan) {
@@ -4173,7 +4198,7 @@ void enqueue_lex_batch(alpacc_ctx *ctx, const LexBatchPlan &pl, hipStream_t st) 
   const LexArgs &a = pl.a;
   lex_tile_docs<<<pl.ndocs, 256, 0, st>>>(a);
   ctx->prof_begin(S_LEX_REDUCE, st);
-  launch_lex_reduce<true>(pl.lex_tab, pl.lex_blocks, pl.lex_lds, a, st);
+  launch_lex_reduce<true, false>(pl.lex_tab, pl.lex_blocks, pl.lex_lds, a, st);
   ctx->prof_end(S_LEX_REDUCE, st);
   ctx->prof_begin(S_LEX_SCAN, st);
   lex_scan_chunks<<<(unsigned)pl.nchunks, LEX_SCAN_BLOCK, 0, st>>>(a);
@@ -5099,6 +5124,8 @@ int place_lexer_tables(alpacc_ctx *ctx, std::string &err) {
   if (lds > 64 * 1024) {
     const int want = (int)lds;
     if (hipFuncSetAttribute((const void *)lex_reduce<1, false>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, want) != hipSuccess ||
+        hipFuncSetAttribute((const void *)lex_reduce<1, false, true>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, want) != hipSuccess ||
         hipFuncSetAttribute((const void *)lex_reduce<1, true>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, want) != hipSuccess) {
