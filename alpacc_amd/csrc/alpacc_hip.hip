@@ -1735,8 +1735,8 @@ struct PArgs {
   const uint32_t *tbr;     // [nstack]
   const uint2 *tprod;      // [nprod]
   const uint4 *trow;       // [3 * (E + 1)] one row per entry, when every entry fits (FT_ROW)
-  uint32_t t_rec, t_slots, t_query;  // its LDS words per wavefront: node records, slots per lane
-                                     // (a power of two), queries
+  uint32_t t_rec, t_slots;  // its LDS words per wavefront: node records and open pops; slots per
+                            // lane (a power of two)
   uint32_t t_prods, t_pops, t_pushes;  // largest counts of any entry
   uint2 *links;            // records of the tiles' open ends (see parse_tree)
   int32_t *tile_low, *tile_low1;  // lowest depth of every tile, and of every 64 tiles
@@ -2082,9 +2082,10 @@ parse_keys2(PArgs a) {
 //   link_tiles      : the open pops of all tiles against the open pushes of earlier ones
 
 constexpr int FT_TILE = WAVE * PK_IPT;  // positions per tile: one wavefront, PK_IPT per lane
-constexpr uint32_t FT_NO_NODE = 0x7FFu;      // a pop without a production (tiles have fewer nodes)
-constexpr uint32_t FT_ROOT = 0xFFFEu;        // parent of the node that fills an unowned symbol
 constexpr uint32_t FT_OPEN = 0xFFFFu;        // parent in an earlier tile
+constexpr uint32_t FT_REC_GAP = 4;           // record words behind the last node's that are written
+                                             // but not read
+constexpr uint32_t FT_REC_PAD = 8;           // the same behind all of them, for entries without nodes
 
 // Word x of a pair entry: productions | terminal productions << 4 | pops << 8 | pushes << 12. Word
 // y: first bracket | first production << 16.
@@ -3083,11 +3084,13 @@ __global__ void __launch_bounds__(LINK_THREADS) link_tiles(PArgs a, Levels lv, u
 // entry.
 constexpr uint32_t FT_ROW_POPS = 3, FT_ROW_PUSHES = 4, FT_ROW_PRODS = 4;
 
-// LDS of parse_tree, in 32-bit words: the tables, then per wavefront the node records, the slots
-// (t_slots per lane and one of padding) and the open pops.
+// LDS of parse_tree, in 32-bit words: the tables, then per wavefront the node records from the bottom
+// up and the open pops from the top down in one array (t_rec words: as many as the entries with the
+// most of both together can make), and the slots (t_slots per lane and one of padding).
 __host__ __device__ inline uint32_t ft_table_words(bool rows, uint32_t E, uint32_t nstack,
                                                    uint32_t nprod) {
-  return (rows ? 12 * (E + 1) : 2 * E + ((nstack + 1) & ~1u)) + 2 * ((nprod + 1) & ~1u);
+  return (rows ? 12 * (E + 1) : 2 * E + ((nstack + 1) & ~1u) + ((nprod + 1) & ~1u)) +
+         2 * ((nprod + 1) & ~1u);
 }
 __host__ __device__ inline uint32_t ft_slot_words(uint32_t slots) { return WAVE * (slots + 1); }
 
@@ -3102,29 +3105,31 @@ __device__ __forceinline__ void ft_write_nodes(const uint32_t *s_rec, const uint
                                                const S *ends, uint32_t *parent, uint32_t *node,
                                                S *span) {
   const int lane = threadIdx.x & (WAVE - 1);
-  const uint32_t nend = node0 + nnode;
+  if (nnode == 0) return;
   uint32_t rank = 0;  // terminal nodes of the tile before this chunk
   constexpr int NC = 4;
-  for (uint32_t c0 = node0 & ~(uint32_t)(WAVE - 1); c0 < nend; c0 += NC * WAVE) {
+  // node words with tokens (x) or without (y)
+  const uint32_t *const words = reinterpret_cast<const uint32_t *>(s_prod) + (subst ? 0 : 1);
+  const uint32_t rel0 = node0 - docnode0;
+  for (uint32_t c0 = node0 & ~(uint32_t)(WAVE - 1); c0 < node0 + nnode; c0 += NC * WAVE) {
     uint32_t rec[NC], pw[NC];
+    bool act[NC];
     S s0[NC], s1[NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-      const uint32_t g = c0 + k * WAVE + lane;
-      rec[k] = s_rec[g >= node0 && g < nend ? g - node0 : 0u];
+      const uint32_t idx = c0 + k * WAVE + lane - node0;
+      act[k] = idx < nnode;
+      rec[k] = s_rec[min(idx, nnode - 1)];
     }
 #pragma unroll
-    for (int k = 0; k < NC; ++k) pw[k] = s_prod[rec[k] & 0xFFFFu].y;
+    for (int k = 0; k < NC; ++k) pw[k] = words[2 * (rec[k] & 0xFFFFu)];
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-      const uint32_t g = c0 + k * WAVE + lane;
-      const bool term = subst && g >= node0 && g < nend && (pw[k] >> 16) != 0u;
+      const bool term = act[k] && (int32_t)pw[k] < 0;  // ALPACC_NODE_TERMINAL
       const uint64_t tm = __ballot(term);
-      const uint32_t r =
-          rank + __builtin_amdgcn_mbcnt_hi((uint32_t)(tm >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)tm, 0u));
+      const uint32_t r = __builtin_amdgcn_mbcnt_hi(
+          (uint32_t)(tm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tm, rank));
       rank += (uint32_t)__popcll(tm);
-      pw[k] = term ? (ALPACC_NODE_TERMINAL | ((pw[k] >> 16) - 1u)) : (pw[k] & 0xFFFFu);
       if (TOK) {
         const uint2 x = s_tok[term ? r : 0u];
         s0[k] = term ? (S)x.x : (S)0;
@@ -3137,20 +3142,22 @@ __device__ __forceinline__ void ft_write_nodes(const uint32_t *s_rec, const uint
         }
       }
     }
+    // (uniform bases, so that the stores take a scalar address and the lane's offset)
+    uint32_t *const cpar = parent + c0, *const cnode = node + c0;
+    S *const cspan = span + 2 * (uint64_t)c0;
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
-      const uint32_t g = c0 + k * WAVE + lane;
-      if (g >= node0 && g < nend) {
+      const uint32_t o = k * WAVE + (uint32_t)lane;
+      if (act[k]) {
         // streamed out: the tree is not read back
-        const uint32_t par = rec[k] >> 16;
-        __builtin_nontemporal_store(par == FT_ROOT ? 0u : node0 - docnode0 + par, parent + g);
-        __builtin_nontemporal_store(pw[k], node + g);
+        __builtin_nontemporal_store(rel0 + (rec[k] >> 16), cpar + o);
+        __builtin_nontemporal_store(pw[k], cnode + o);
         if (sizeof(S) == 4) {
           __builtin_nontemporal_store((uint64_t)(uint32_t)s0[k] | ((uint64_t)(uint32_t)s1[k] << 32),
-                                      reinterpret_cast<uint64_t *>(span) + g);
+                                      reinterpret_cast<uint64_t *>(cspan) + o);
         } else {
-          span[2 * (uint64_t)g] = s0[k];
-          span[2 * (uint64_t)g + 1] = s1[k];
+          cspan[2 * o] = s0[k];
+          cspan[2 * o + 1] = s1[k];
         }
       }
     }
@@ -3216,11 +3223,13 @@ __device__ __forceinline__ void ft_load_doc(const PArgs &a, FtTile<ET> &t) {
 //     64 nodes at a time, and the node, span and parent are written, coalesced.
 // The sequential walk per lane needs a few instructions per position where a cooperative search
 // over 64 elements needed 160, and the matches are read from LDS instead of written and searched.
-// 256 MiB JSON document: 415 us and link_tiles 30, against 567 + 125 + 349 us of parse_expand2,
-// bracket_match and parse_parents; 256 MiB batch of sexp documents: 510 + 41 against 805 + 105 + 588.
-// It is bound by VALU issue (about 1100 per tile, 4 wavefronts per SIMD) close to the 1.75 GB it
-// moves. On the way: entry rows and straight-line step 1 760 -> 700 us, no load among the stores
-// 700 -> 598, the next tile's words loaded ahead 598 -> 425, a larger grid 425 -> 415.
+// 256 MiB JSON document: 346 us and link_tiles 30, against 567 + 125 + 349 us of parse_expand2,
+// bracket_match and parse_parents; 256 MiB batch of sexp documents: 509 + 41 against 805 + 105 + 588.
+// What bounds it now is the 1.75 GB (sexp: 2.5 GB) it moves, at 5.0 TB/s where a large copy reaches
+// 5.2. On the way: entry rows and straight-line step 1 760 -> 700 us, no load among the stores
+// 700 -> 598, the next tile's words loaded ahead 598 -> 425, a larger grid 425 -> 415; open pops in
+// the records' array (a fourth workgroup per CU), one scan, no selects around the stores to LDS and
+// uniform store bases 415 -> 346.
 // ROWS: the entries come as rows, and step 1 runs the four positions' operations in straight line,
 // every load issued before the first is used (an operation that a position does not have goes to
 // the lane's padding word); else (larger entries) it loops over each position's own counts, one
@@ -3235,16 +3244,22 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
   const uint4 *const s_row = reinterpret_cast<const uint4 *>(s_tab);
   const uint2 *const s_ent = reinterpret_cast<const uint2 *>(s_tab);
   uint32_t *const s_br = s_tab + 2 * a.E;
+  uint32_t *const s_prec = s_br + ((a.nstack + 1) & ~1u);
   const int lane = threadIdx.x & (WAVE - 1);
   const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const uint32_t wpb = blockDim.x / WAVE;
-  const uint32_t wave_words = a.t_rec + ft_slot_words(a.t_slots) + a.t_query;
+  const uint32_t wave_words = a.t_rec + ft_slot_words(a.t_slots);
   uint32_t *const s_rec = ft_smem + ft_table_words(ROWS, a.E, a.nstack, a.nprod) + w * wave_words;
   uint32_t *const s_slot = s_rec + a.t_rec;
-  uint32_t *const s_query = s_slot + ft_slot_words(a.t_slots);
+  const uint32_t qtop = a.t_rec - FT_REC_PAD - 1;  // the first open pop's word, the others below
   uint32_t *const my_slot = s_slot + lane * (a.t_slots + 1);
   const int32_t smask = (int32_t)a.t_slots - 1;
-  for (uint32_t i = threadIdx.x; i < a.nprod; i += blockDim.x) s_prod[i] = a.tprod[i];
+  for (uint32_t i = threadIdx.x; i < a.nprod; i += blockDim.x) {
+    const uint2 pw = a.tprod[i];  // the node word with and without tokens
+    s_prod[i] = make_uint2((pw.y >> 16) != 0u ? ALPACC_NODE_TERMINAL | ((pw.y >> 16) - 1u) : pw.y,
+                           pw.y & 0xFFFFu);
+    if (!ROWS) s_prec[i] = pw.x;
+  }
   if (ROWS) {
     for (uint32_t i = threadIdx.x; i < 3 * (a.E + 1); i += blockDim.x)
       const_cast<uint4 *>(s_row)[i] = a.trow[i];
@@ -3319,8 +3334,11 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
       np += ft_np(f[i]);
       d += ft_pushes(f[i]) - ft_pops(f[i]);
     }
-    const int32_t d0 = wave_incl_i32(d, 0, OpAdd()) - d;  // depth before the lane, 0 before the tile
-    uint32_t nb = (uint32_t)wave_incl_i32((int32_t)np, 0, OpAdd()) - np;
+    // both in one scan, the depth (at most 32 either way per lane) made positive
+    const uint32_t own = np | ((uint32_t)(d + 32) << 16);
+    const uint32_t ex = (uint32_t)wave_incl_i32((int32_t)own, 0, OpAdd()) - own;
+    const int32_t d0 = (int32_t)(ex >> 16) - 32 * lane;  // depth before the lane, 0 before the tile
+    uint32_t nb = ex & 0xFFFFu;
     int32_t low = d0;
     {
       int32_t dc = d0;
@@ -3344,31 +3362,38 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
       int32_t dc = d0, lowc = d0;
 #pragma unroll
       for (int i = 0; i < PK_IPT; ++i) {
-        const int32_t pops = ft_pops(f[i]), pushes = ft_pushes(f[i]);
-        const uint32_t npi = ft_np(f[i]);
-        const uint32_t rcw[FT_ROW_PRODS] = {rc[i].x, rc[i].y, rc[i].z, rc[i].w};
         const uint32_t rbw[FT_ROW_PUSHES] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
         nbi[i] = nb;
         dci[i] = dc;
         lowi[i] = lowc;
 #pragma unroll
-        for (uint32_t j = 0; j < FT_ROW_PRODS; ++j)
-          if (j < a.t_prods) s_rec[j < npi ? nb + j : trash] = rcw[j] + (nb << 16);
-#pragma unroll
         for (uint32_t r = 0; r < FT_ROW_POPS; ++r) {
           sl[i][r] = 0;
           if (r < a.t_pops) sl[i][r] = my_slot[(dc - 1 - (int32_t)r) & smask];
         }
-        dc -= pops;
+        dc -= ft_pops(f[i]);
         lowc = min(lowc, dc);
+        // every entry writes as many slots as the largest: the ones it does not push are above its
+        // depth and written again before they are read (4 * t_pushes slots hold both)
 #pragma unroll
         for (uint32_t l = 0; l < FT_ROW_PUSHES; ++l)
-          if (l < a.t_pushes)
-            my_slot[(int32_t)l < pushes ? (dc + (int32_t)l) & smask : (int32_t)a.t_slots] =
-                rbw[l] + (nb << 16);
-        dc += pushes;
-        nb += npi;
+          if (l < a.t_pushes) my_slot[(dc + (int32_t)l) & smask] = rbw[l] + (nb << 16);
+        dc += ft_pushes(f[i]);
+        nb += ft_np(f[i]);
       }
+      // every entry writes as many records as the largest, last ones first: the j-th one of an entry
+      // that has fewer is the j'-th of a later entry, j' < j, which comes after it (an entry without
+      // any writes behind the tile's last)
+#pragma unroll
+      for (int j = (int)FT_ROW_PRODS - 1; j >= 0; --j)
+        if ((uint32_t)j < a.t_prods) {
+#pragma unroll
+          for (int i = 0; i < PK_IPT; ++i) {
+            const uint32_t rcw[FT_ROW_PRODS] = {rc[i].x, rc[i].y, rc[i].z, rc[i].w};
+            s_rec[(ft_np(f[i]) ? nbi[i] : a.t_rec - FT_REC_PAD) + (uint32_t)j] = rcw[j] + (nbi[i] << 16);
+          }
+        }
+      const uint32_t qlane = (uint32_t)lane << 11;
 #pragma unroll
       for (int i = 0; i < PK_IPT; ++i) {
         const int32_t pops = ft_pops(f[i]);
@@ -3379,14 +3404,12 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
             const int32_t h = dci[i] - 1 - (int32_t)r;
             const bool valid = (int32_t)r < pops;
             const bool local = valid && h >= lowi[i];
-            const bool owned = raw[r] < 0xFFFF0000u;
             const uint32_t nd = nbi[i] + (raw[r] >> 16);
-            mism |= local && ((sl[i][r] ^ raw[r]) & 0x7FFFu) != 0u;
-            reinterpret_cast<uint16_t *>(s_rec)[2 * (local && owned ? nd : trash) + 1] =
+            mism |= local && (uint16_t)sl[i][r] != (uint16_t)raw[r];
+            reinterpret_cast<uint16_t *>(s_rec)[2 * (local ? nd : trash) + 1] =
                 (uint16_t)(sl[i][r] >> 16);
-            const uint32_t qi = a.t_rec + ft_slot_words(a.t_slots) + (uint32_t)(uheight - h);
-            s_rec[valid && !local ? qi : trash] = (owned ? nd : FT_NO_NODE) |
-                                                  ((uint32_t)lane << 11) | ((raw[r] & 0x7FFFu) << 17);
+            s_rec[valid && !local ? qtop - (uint32_t)(uheight - h) : trash] =
+                (raw[r] << 17) | qlane | nd;
           }
         }
       }
@@ -3397,19 +3420,18 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
         const uint32_t br0 = at[i] & 0xFFFFu, pr0 = at[i] >> 16;
         const int32_t pops = ft_pops(f[i]), pushes = ft_pushes(f[i]);
         const uint32_t npi = ft_np(f[i]);
-        for (uint32_t j = 0; j < npi; ++j) s_rec[nb + j] = s_prod[pr0 + j].x + (nb << 16);
+        for (uint32_t j = 0; j < npi; ++j) s_rec[nb + j] = s_prec[pr0 + j] + (nb << 16);
         for (int32_t r = 0; r < pops; ++r) {
           const uint32_t b = s_br[br0 + (uint32_t)r];
           const int32_t h = dc - 1 - r;
-          const bool owned = b < 0xFFFF0000u;
+          const uint32_t nd = nb + (b >> 16);
           if (h >= lowc) {
             const uint32_t sl = my_slot[h & smask];
-            mism |= ((sl ^ b) & 0x7FFFu) != 0u;
-            if (owned)
-              reinterpret_cast<uint16_t *>(s_rec)[2 * (nb + (b >> 16)) + 1] = (uint16_t)(sl >> 16);
+            mism |= (uint16_t)sl != (uint16_t)b;
+            // (behind the tile's nodes: a pop that no production fills)
+            if (nd < nnode) reinterpret_cast<uint16_t *>(s_rec)[2 * nd + 1] = (uint16_t)(sl >> 16);
           } else {
-            s_query[uheight - h] =
-                (owned ? nb + (b >> 16) : FT_NO_NODE) | ((uint32_t)lane << 11) | ((b & 0x7FFFu) << 17);
+            s_rec[qtop - (uint32_t)(uheight - h)] = (b << 17) | ((uint32_t)lane << 11) | nd;
           }
         }
         dc -= pops;
@@ -3434,7 +3456,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
       for (int32_t q0 = 0; q0 < total; q0 += WAVE) {
         const int32_t q = q0 + lane;
         const bool pop = q < nopen;
-        const uint32_t qw = pop ? s_query[q] : 0u;
+        const uint32_t qw = pop ? s_rec[qtop - (uint32_t)q] : 0u;
         const int ql = pop ? (int)((qw >> 11) & 63u) : WAVE;
         const int32_t hq = __builtin_amdgcn_ds_bpermute(ql << 2, uheight) - q;
         const int32_t h = pop ? hq : tlow + (q - nopen);
@@ -3444,17 +3466,16 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
           const uint32_t nd = qw & 0x7FFu;
           uint32_t par = FT_OPEN;
           if (p > 0) {
-            mism |= ((sl ^ (qw >> 17)) & 0x7FFFu) != 0u;
+            mism |= (uint16_t)sl != (uint16_t)(qw >> 17);
             par = sl >> 16;
           } else {
             a.links[(uint64_t)pre_nb + (uint32_t)(-1 - h)] =
-                make_uint2(nd == FT_NO_NODE ? 0xFFFFFFFFu : node0 + nd, qw >> 17);
+                make_uint2(nd < nnode ? node0 + nd : 0xFFFFFFFFu, qw >> 17);
           }
-          if (nd != FT_NO_NODE) reinterpret_cast<uint16_t *>(s_rec)[2 * nd + 1] = (uint16_t)par;
+          if (nd < nnode) reinterpret_cast<uint16_t *>(s_rec)[2 * nd + 1] = (uint16_t)par;
         } else if (q < total) {
-          const uint32_t own = sl >> 16;
           a.links[(uint64_t)pre_nb + (uint32_t)(h - 2 * tlow)] =
-              make_uint2(own == FT_ROOT ? 0u : node0 - docnode0 + own, sl & 0x7FFFu);
+              make_uint2(node0 - docnode0 + (sl >> 16), sl & 0x7FFFu);
         }
       }
     }
@@ -3611,7 +3632,7 @@ struct alpacc_ctx {
   uint2 *d_tent = nullptr, *d_tprod = nullptr;
   uint32_t *d_tbr = nullptr;
   uint4 *d_trow = nullptr;  // (only when every entry fits a row)
-  uint32_t t_rec = 0, t_slots = 0, t_query = 0, t_prods = 0, t_pops = 0, t_pushes = 0;
+  uint32_t t_rec = 0, t_slots = 0, t_prods = 0, t_pops = 0, t_pushes = 0;
   unsigned tree_threads = 0, tree_bpc = 1;
   size_t tree_lds = 0;
   // scratch (grow-only)
@@ -4269,7 +4290,6 @@ bool parse_args_tree(alpacc_ctx *ctx, PArgs &a, uint64_t ntiles_max) {
   a.tprod = ctx->d_tprod;
   a.t_rec = ctx->t_rec;
   a.t_slots = ctx->t_slots;
-  a.t_query = ctx->t_query;
   a.trow = ctx->d_trow;
   a.t_prods = ctx->t_prods;
   a.t_pops = ctx->t_pops;
@@ -4330,7 +4350,8 @@ void launch_keys_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles_max, bool
 // The tree of about ntiles tiles by workgroups striding over them (each wavefront loads its next
 // tile's words while it works on one): up to TREE_WAVES times as many as the GPU holds at once, which
 // measured 510 us on a 256 MiB batch of sexp documents and 416 us on a 256 MiB JSON document against
-// 586 and 426 us with once (the wavefronts then write and compute in step).
+// 586 and 426 us with once (the wavefronts then write and compute in step), before it was bound by
+// its traffic.
 template <typename S, bool BATCH>
 void launch_tree(alpacc_ctx *ctx, const PArgs &a, uint64_t ntiles, const S *starts, const S *ends,
                  uint32_t *node, S *span, uint32_t *parent, bool link, hipStream_t st) {
@@ -5304,7 +5325,7 @@ bool build_tree_tables(alpacc_ctx *ctx, const alpacc_tables *t, std::string &err
   std::vector<uint2> ent(E), prod;
   std::vector<uint32_t> br;
   std::vector<uint8_t> ends(E, 0);  // 1: pushes unowned symbols, 2: pops symbols nothing fills
-  uint32_t max_np = 1, max_pops = 1, max_pushes = 1;
+  uint32_t max_np = 1, max_pops = 1, max_pushes = 1, max_both = 1;
   bool any_ends = false;
   for (uint32_t e = 0; e < E; ++e) {
     const uint32_t *e4 = t->pair_entry + 4ull * e;
@@ -5316,7 +5337,9 @@ bool build_tree_tables(alpacc_ctx *ctx, const alpacc_tables *t, std::string &err
       if (!(t->stacks[s] & 0x8000u)) return true;
     if (np > MAX_PROD || pops > MAX_RUN || pushes > MAX_RUN) return true;
     std::vector<uint32_t> open;                  // owners of the symbols left open
-    std::vector<uint32_t> fills(pops, 0xFFFFu);  // production that fills every popped symbol
+    // production that fills every popped symbol; without one, the record behind the entry's own: at
+    // the document's last position, where such entries stand, no node's
+    std::vector<uint32_t> fills(pops, np);
     uint32_t filled = 0, nt = 0;
     const uint32_t pst = (uint32_t)prod.size();
     for (uint32_t j = 0; j < np; ++j) {
@@ -5344,9 +5367,12 @@ bool build_tree_tables(alpacc_ctx *ctx, const alpacc_tables *t, std::string &err
       br.push_back((uint32_t)(t->stacks[e4[0] + r] & 0x7FFFu) | (fills[r] << 16));
     for (uint32_t l = 0; l < pushes; ++l)
       br.push_back((uint32_t)(t->stacks[e4[0] + pops + l] & 0x7FFFu) |
-                   ((ends[e] == 1 ? FT_ROOT : open[l]) << 16));
+                   // an unowned symbol is as good as owned by the document's first node, which
+                   // fills it: the parent of the root is the root
+                   ((ends[e] == 1 ? 0u : open[l]) << 16));
     ent[e] = make_uint2(np | (nt << 4) | (pops << 8) | (pushes << 12), sst | (pst << 16));
     max_np = std::max(max_np, np);
+    max_both = std::max(max_both, np + pops);
     max_pops = std::max(max_pops, pops);
     max_pushes = std::max(max_pushes, pushes);
   }
@@ -5373,15 +5399,14 @@ bool build_tree_tables(alpacc_ctx *ctx, const alpacc_tables *t, std::string &err
   }
   uint32_t slots = 8;
   while (slots < PK_IPT * max_pushes) slots *= 2;
-  ctx->t_rec = FT_TILE * max_np;
+  ctx->t_rec = FT_TILE * max_both + FT_REC_GAP + FT_REC_PAD;
   ctx->t_slots = slots;
-  ctx->t_query = FT_TILE * max_pops;
   if (br.empty()) br.push_back(0);
   if (prod.empty()) prod.push_back(make_uint2(0, 0));
   // (the array lengths are those of build_parser_tables: a.nstack, a.nprod)
   const bool rows = max_pops <= FT_ROW_POPS && max_pushes <= FT_ROW_PUSHES && max_np <= FT_ROW_PRODS;
   const size_t tables = 4ull * ft_table_words(rows, E, (uint32_t)br.size(), (uint32_t)prod.size());
-  const size_t wave = 4ull * (ctx->t_rec + ft_slot_words(slots) + ctx->t_query);
+  const size_t wave = 4ull * (ctx->t_rec + ft_slot_words(slots));
   unsigned waves = 4;
   while (waves > 1 && tables + waves * wave > (64u << 10)) waves /= 2;
   if (tables + waves * wave > (64u << 10)) return true;
