@@ -981,7 +981,7 @@ lex_emit(LexArgs p) {
     // boundary follows a kept byte and starts at j where a boundary precedes one. Per byte that is
     // the class address, the row address and one v_alignbit_b32 that shifts bit 0 into the boundary
     // mask; labels are packed four at a time and their top bits gathered by v_dot4_u32_u8.
-    // (902 -> 623 VALU and 488 -> 176 scalar instructions per wavefront with the staging below.)
+    // (902 -> 740 VALU and 488 -> 176 scalar instructions per wavefront with the staging below.)
     uint32_t row = row0, bm = 0, km = 0;
     uint32_t labs[LEX_IPT / 4];
     uint32_t xs[4];

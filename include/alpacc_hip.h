@@ -204,14 +204,15 @@ int alpacc_test_force_timeout(alpacc_ctx *ctx, int on);
  *                       (sizes, buffers, flags) repeats the previous call's, and replay that graph
  *                       while it keeps repeating; 2 = capture every new plan.
  *   lex_blocks_per_cu : persistent lex_reduce workgroups per CU (1..8, default 2)
- *   keys_blocks_per_cu: persistent parse_keys2 workgroups per CU (1..8, default 2)
+ *   keys_blocks_per_cu: persistent workgroups per CU of the kernel that looks up the pair entries
+ *                       (1..8, default 2)
  *   search_max_blocks : largest grid of bracket_match / parse_parents, in workgroups of 256
- *                       threads (64..2^20, default 16384)
+ *                       threads (64..2^20, default 16384); the tree parser does not run them
  *   search_block_threads: workgroup size of bracket_match / parse_parents (256, 512 or 1024;
  *                       default 256)
- *   brackets_per_kib  : brackets per KiB of input the batched bracket scratch is first sized for
- *                       (1..2^20, default 256); a batch with more runs again sized exactly, and
- *                       the estimate grows to what calls needed
+ *   brackets_per_kib  : brackets (tree parser: open ends of its tiles) per KiB of input the
+ *                       scratch is first sized for (1..2^20, default 256); a call with more runs again sized exactly, and the estimate
+ *                       grows to what calls needed
  *   lexer_tables_in_lds: 1 (default) = the lexer's tables in LDS where they fit (the
  *                       (endo x class) table up to 160 KiB, the DFA table up to 4096 entries),
  *                       read from L2 otherwise; 0 = every lexer table read from L2
@@ -237,13 +238,15 @@ int alpacc_get_tuning(alpacc_ctx *ctx, alpacc_tuning *t);
 uint64_t alpacc_device_bytes(alpacc_ctx *ctx);
 
 /* Element counts of the last parser call on `ctx`: counts[0] tokens, [1] key positions (T + 2;
- * tile-padded in batched calls), [2] brackets written for the bracket search (those left after
- * neighbouring positions' matching brackets cancel), [3] productions (tree nodes). */
+ * tile-padded in batched calls), [2] pops and pushes of the stack that a tile of 256 positions leaves
+ * open (tree parser), or brackets written for the bracket search (those left after neighbouring
+ * positions' matching brackets cancel), [3] productions (tree nodes). */
 int alpacc_last_counts(alpacc_ctx *ctx, uint64_t *counts);
 
 /* Device-time profiling: when enabled, every call records HIP events on its stream around each
- * stage (lex_reduce, lex_scan, lex_emit, parse, and inside parse: parse_keys, parse_expand,
- * bracket_match, parse_parents). alpacc_profile_read fills up to max_stages
+ * stage (lex_reduce, lex_scan, lex_emit, parse, and inside parse: parse_keys, then parse_tree and
+ * link_tiles, or for what the tree parser does not take parse_expand, bracket_match and
+ * parse_parents). alpacc_profile_read fills up to max_stages
  * names, accumulated milliseconds and call counts since the last read, resets them, and returns
  * the number of stages filled. */
 int alpacc_profile_enable(alpacc_ctx *ctx, int on);
