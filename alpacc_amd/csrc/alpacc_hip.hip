@@ -1186,8 +1186,13 @@ lex_emit(LexArgs p) {
         p.starts64[g] = cs;
         p.ends64[g] = ce;
       } else {
-        p.starts[g] = sv;
-        p.ends[g] = (uint32_t)tbase + at + 1;
+        // streamed past the caches, unlike the kinds, which the parser reads right away: the spans
+        // (8 bytes a token) are read once and later, and left in L2 their write-back and the lines
+        // they displace cost the kernels after this one more than the plain stores save here.
+        // 256 MiB batch of sexp documents: 1042 -> 1012 us (parse_tree 517 -> 492, lex_emit
+        // 228 -> 232); 256 MiB of JSON lexed alone 358 -> 356, with the parser unchanged (824).
+        __builtin_nontemporal_store(sv, p.starts + g);
+        __builtin_nontemporal_store((uint32_t)tbase + at + 1, p.ends + g);
       }
     }
     wave_lds_sync();
@@ -3224,7 +3229,7 @@ __device__ __forceinline__ void ft_load_doc(const PArgs &a, FtTile<ET> &t) {
 // The sequential walk per lane needs a few instructions per position where a cooperative search
 // over 64 elements needed 160, and the matches are read from LDS instead of written and searched.
 // 256 MiB JSON document: 346 us and link_tiles 30, against 567 + 125 + 349 us of parse_expand2,
-// bracket_match and parse_parents; 256 MiB batch of sexp documents: 509 + 41 against 805 + 105 + 588.
+// bracket_match and parse_parents; 256 MiB batch of sexp documents: 492 + 41 against 805 + 105 + 588.
 // What bounds it now is the 1.75 GB (sexp: 2.5 GB) it moves, at 5.0 TB/s where a large copy reaches
 // 5.2. On the way: entry rows and straight-line step 1 760 -> 700 us, no load among the stores
 // 700 -> 598, the next tile's words loaded ahead 598 -> 425, a larger grid 425 -> 415; open pops in
