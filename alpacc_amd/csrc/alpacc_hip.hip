@@ -2092,6 +2092,14 @@ constexpr uint32_t FT_REC_GAP = 4;           // record words behind the last nod
                                              // but not read
 constexpr uint32_t FT_REC_PAD = 8;           // the same behind all of them, for entries without nodes
 
+// The parent in a node record (its upper half), written over a record that was stored as a word: a
+// type of its own, since plain 16-bit and 32-bit stores count as never meeting each other and the
+// compiler may then put the record's store behind the parent's.
+typedef uint16_t __attribute__((may_alias)) ft_half;
+__device__ __forceinline__ void ft_set_parent(uint32_t *rec, uint32_t parent) {
+  reinterpret_cast<ft_half *>(rec)[1] = (ft_half)parent;
+}
+
 // Word x of a pair entry: productions | terminal productions << 4 | pops << 8 | pushes << 12. Word
 // y: first bracket | first production << 16.
 __device__ __forceinline__ uint32_t ft_np(uint32_t f) { return f & 15u; }
@@ -3388,7 +3396,9 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
       }
       // every entry writes as many records as the largest, last ones first: the j-th one of an entry
       // that has fewer is the j'-th of a later entry, j' < j, which comes after it (an entry without
-      // any writes behind the tile's last)
+      // any writes behind the tile's last). That later entry may be another lane's, so the rounds are
+      // kept in order for the whole wavefront (a wavefront's LDS operations are carried out in order:
+      // the fence is for the compiler and no instruction)
 #pragma unroll
       for (int j = (int)FT_ROW_PRODS - 1; j >= 0; --j)
         if ((uint32_t)j < a.t_prods) {
@@ -3397,6 +3407,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
             const uint32_t rcw[FT_ROW_PRODS] = {rc[i].x, rc[i].y, rc[i].z, rc[i].w};
             s_rec[(ft_np(f[i]) ? nbi[i] : a.t_rec - FT_REC_PAD) + (uint32_t)j] = rcw[j] + (nbi[i] << 16);
           }
+          wave_lds_sync();
         }
       const uint32_t qlane = (uint32_t)lane << 11;
 #pragma unroll
@@ -3411,8 +3422,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
             const bool local = valid && h >= lowi[i];
             const uint32_t nd = nbi[i] + (raw[r] >> 16);
             mism |= local && (uint16_t)sl[i][r] != (uint16_t)raw[r];
-            reinterpret_cast<uint16_t *>(s_rec)[2 * (local ? nd : trash) + 1] =
-                (uint16_t)(sl[i][r] >> 16);
+            ft_set_parent(s_rec + (local ? nd : trash), sl[i][r] >> 16);
             s_rec[valid && !local ? qtop - (uint32_t)(uheight - h) : trash] =
                 (raw[r] << 17) | qlane | nd;
           }
@@ -3434,7 +3444,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
             const uint32_t sl = my_slot[h & smask];
             mism |= (uint16_t)sl != (uint16_t)b;
             // (behind the tile's nodes: a pop that no production fills)
-            if (nd < nnode) reinterpret_cast<uint16_t *>(s_rec)[2 * nd + 1] = (uint16_t)(sl >> 16);
+            if (nd < nnode) ft_set_parent(s_rec + nd, sl >> 16);
           } else {
             s_rec[qtop - (uint32_t)(uheight - h)] = (b << 17) | ((uint32_t)lane << 11) | nd;
           }
@@ -3477,7 +3487,7 @@ __global__ void __launch_bounds__(256) parse_tree(PArgs a, const S *starts, cons
             a.links[(uint64_t)pre_nb + (uint32_t)(-1 - h)] =
                 make_uint2(nd < nnode ? node0 + nd : 0xFFFFFFFFu, qw >> 17);
           }
-          if (nd < nnode) reinterpret_cast<uint16_t *>(s_rec)[2 * nd + 1] = (uint16_t)par;
+          if (nd < nnode) ft_set_parent(s_rec + nd, par);
         } else if (q < total) {
           a.links[(uint64_t)pre_nb + (uint32_t)(h - 2 * tlow)] =
               make_uint2(node0 - docnode0 + (sl >> 16), sl & 0x7FFFu);
