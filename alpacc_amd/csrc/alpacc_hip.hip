@@ -3057,7 +3057,10 @@ __device__ __forceinline__ void link_run(const PArgs &a, const Levels &lv, uint3
       int32_t su = __builtin_amdgcn_ds_bpermute(s4, u), sv = __builtin_amdgcn_ds_bpermute(s4, v);
       int32_t slow = __builtin_amdgcn_ds_bpermute(s4, low);
       const uint32_t qdoc = BATCH ? (uint32_t)__builtin_amdgcn_ds_bpermute(l4, (int)doc) : 0u;
-      if (pop) {
+      // A height below the document's start is met in a batch only, in a document that its depth has
+      // rejected, and ends nowhere: searched for, it climbs through all documents before (a batch with
+      // 8 MiB of closing brackets in it: 166.8 ms, and 1.0 without).
+      if (pop && h >= 0) {
         const uint2 me = a.links[lnk];
         bool found = p > 0;
         if (!found) {
@@ -3071,7 +3074,7 @@ __device__ __forceinline__ void link_run(const PArgs &a, const Levels &lv, uint3
             found = true;
           }
         }
-        // (in a rejected document the found tile may be another document's: no push at h then)
+        // (in a rejected document the found tile may lack a push at h)
         found = found && h - slow < sv;
         uint2 at = make_uint2(0u, 0xFFFFFFFFu);
         if (found) at = a.links[(uint64_t)soff + (uint32_t)(su + (h - slow))];
