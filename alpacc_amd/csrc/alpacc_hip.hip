@@ -181,10 +181,11 @@ struct LexArgs {
   uint32_t *host_result;      // when set: pinned host copy of result
   // chunked mode (the reference's chunk loop, lexer.fut:144-172): n and all positions are those of
   // the virtual string in which every chunk [j*chunk, min(j*chunk + chunk + 1, n_orig)) is laid end to
-  // end, so the byte shared by two neighbouring chunks appears twice; `in` is the original string,
-  // which the loads map to (laying it out took 46 us for 48 MiB).
+  // end, so the byte shared by two neighbouring chunks appears twice. `in` is the original string,
+  // which the loads map to, or (laid_out, short chunks) the virtual string itself.
   uint32_t chunk;             // chunk size in bytes of the original string
   uint32_t nchunks;           // K = ceil(n_orig / chunk)
+  uint32_t laid_out;
   uint64_t n_orig;
   uint64_t *starts64;         // [cap] token starts as the reference computes them (i64 there)
   uint64_t *ends64;
@@ -929,7 +930,8 @@ lex_emit(LexArgs p) {
   const uint64_t base = tbase + (uint64_t)lane * LEX_IPT;
   const int valid = (tile >= p.num_tiles || base >= n) ? 0 : (int)min((uint64_t)LEX_IPT, n - base);
   uint32_t wds[LEX_IPT / 4];
-  if (CHUNKED) load_words_chunked(p.in, p.n_orig, p.chunk + 1, (uint32_t)base, valid, wds);
+  const bool mapped = CHUNKED && !p.laid_out;
+  if (mapped) load_words_chunked(p.in, p.n_orig, p.chunk + 1, (uint32_t)base, valid, wds);
   else load_words(tv.ptr, tv.aligned, base, valid, n, wds);
   // class of the lane's byte j (j a constant)
 #define LEX_C(j) ((uint32_t)s_cls[(wds[(j) >> 2] >> (8 * ((j)&3))) & 0xFFu])
@@ -962,7 +964,7 @@ lex_emit(LexArgs p) {
   uint32_t b_next = (uint32_t)dpp_i32<DPP_WAVE_SHL1>(0, (int32_t)(wds[0] & 0xFFu));
   if (lane == WAVE - 1 && tbase + LEX_TILE < n) {
     const uint32_t nb = (uint32_t)(tbase + LEX_TILE);
-    b_next = CHUNKED ? p.in[nb - nb / (p.chunk + 1)] : tv.ptr[nb];
+    b_next = mapped ? p.in[nb - nb / (p.chunk + 1)] : tv.ptr[nb];
   }
 
   // ---- one walk: token-end mask, token-start mask and the label after every byte
@@ -1276,6 +1278,16 @@ __global__ void lex_chunk_fixup(LexArgs p) {
     p.kinds[c - 1] = (uint32_t)p.chunk_info[4ull * j + 1];
     p.starts64[c - 1] = p.chunk_info[4ull * j + 2];
     p.ends64[c - 1] = p.chunk_info[4ull * j + 3];
+  }
+}
+
+// Chunked mode, short chunks: lay the chunks [j*chunk, min(j*chunk + chunk + 1, n)) end to end.
+__global__ void lex_chunk_expand(const uint8_t *in, uint32_t chunk, uint64_t nv, uint8_t *out) {
+  const uint32_t cp1 = chunk + 1;
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < nv;
+       v += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t vv = (uint32_t)v;
+    out[v] = in[vv - vv / cp1];
   }
 }
 
@@ -3770,6 +3782,7 @@ enum BufId {
   B_SX,
   B_DL1,
   B_SL1,
+  B_VIRT,
   B_CHUNK_INFO,
   B_TOK_START64,
   B_TOK_END64,
@@ -3955,6 +3968,12 @@ int lex_verdict(alpacc_ctx *ctx, uint64_t *num_tokens, hipStream_t st) {
   return hw[0] ? ALPACC_ACCEPT : ALPACC_REJECT;
 }
 
+// Chunks shorter than this are laid out (a copy of the virtual string) before they are lexed. A lane
+// that a chunk ends in gathers its bytes one by one and its wavefront waits, which costs more than the
+// copy where it is the rule: 48 MiB of JSON in chunks of 100 bytes 212 us mapped, 152 laid out, of 2000
+// 164 and 148, of 3000 159 and 149, of 5000 147 and 149, of 10000 140 and 151, of 100000 127 and 153.
+constexpr uint64_t LEX_CHUNK_MAPPED = 4096;
+
 // The lexer. chunk == 0: unchunked (kinds/starts/ends as u32). chunk > 0: the reference's chunk
 // loop with chunks of `chunk` bytes (kinds, starts64/ends64).
 // sync = false (unchunked only): return ALPACC_ACCEPT once the kernels are queued; the verdict,
@@ -3986,6 +4005,17 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   if (fixed && chunk > 0) {
     ctx->err = "the chunked lexer has no fixed-scratch form";
     return ALPACC_ERR_ARG;
+  }
+  const bool laid_out = K > 1 && chunk < LEX_CHUNK_MAPPED;
+  if (laid_out) {
+    uint8_t *virt = (uint8_t *)ctx->buf(B_VIRT, n + 16);
+    if (!virt) {
+      ctx->err = "scratch allocation failed";
+      return ALPACC_ERR_HIP;
+    }
+    lex_chunk_expand<<<grid_for(n, 256, 1u << 14), 256, 0, st>>>(d_in, (uint32_t)chunk, n, virt);
+    ctx->launches++;
+    d_in = virt;
   }
   uint64_t *chunk_info = nullptr;
   if (chunk > 0) {
@@ -4057,6 +4087,7 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
   ctx->h_small[2] = a.timeout0;
   a.chunk = (uint32_t)chunk;
   a.nchunks = (uint32_t)K;
+  a.laid_out = laid_out ? 1u : 0u;
   a.n_orig = n_orig;
   a.starts64 = starts64;
   a.ends64 = ends64;
@@ -4080,7 +4111,7 @@ int run_lex(alpacc_ctx *ctx, const uint8_t *d_in, uint64_t n, uint32_t *kinds, u
     return sync ? lex_verdict(ctx, num_tokens, st) : ALPACC_ACCEPT;
   }
   ctx->prof_begin(S_LEX_REDUCE, st);
-  if (chunk > 0) launch_lex_reduce<false, true>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
+  if (chunk > 0 && !laid_out) launch_lex_reduce<false, true>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
   else launch_lex_reduce<false, false>(ctx->lex_tab, (unsigned)blocks, ctx->lex_lds, a, st);
   ctx->prof_end(S_LEX_REDUCE, st);
   ctx->prof_begin(S_LEX_SCAN, st);
