@@ -3679,10 +3679,46 @@ struct alpacc_ctx {
   std::vector<uint8_t> gplan;         // the plan gexec was captured from
   std::vector<uint8_t> last_plan;     // the previous call's plan (graph_mode 1)
   uint64_t graph_launches = 0, graph_captures = 0;
-  // brackets per input byte the batched scratch is sized for (grows with what calls need)
-  double b_per_byte = 0.25;
-  // key positions per input byte the batched expansion's grid is sized for (grows likewise)
-  double p_per_byte = 0.25;
+  // Brackets (tree parser: open ends) that scratch is sized for: so many per input byte, and no less
+  // than what a call of this context needed that had more (b_need; b_seen is that call's per byte, for
+  // alpacc_get_tuning). The need is kept as a number: kept per byte, that of one deeply nested request
+  // of 600 bytes made the next 256 MiB document allocate 5.0 GB of links, against 0.5 in a new context.
+  double b_per_byte = 0.25, b_seen = 0.0;
+  uint64_t b_need = 0;
+  uint64_t bracket_cap(uint64_t nbytes, uint64_t bound, uint64_t least) const {
+    return std::min(bound, std::max({least, b_need, (uint64_t)(b_per_byte * (double)nbytes)}));
+  }
+  uint64_t bracket_learn(uint64_t B, uint64_t nbytes) {
+    b_need = std::max(b_need, B + B / 8 + 256);
+    if (nbytes) b_seen = 1.125 * (double)B / (double)nbytes;
+    return b_need;
+  }
+  uint32_t brackets_per_kib() const {
+    return (uint32_t)std::min(std::max(b_per_byte, b_seen) * 1024.0 + 0.5, (double)(1u << 20));
+  }
+  // Key positions per input byte that grids are sized by, and kernels chosen by: grows when a call has
+  // more (short ones aside, that run the same kernels anyway), and comes down when P_IDLE calls in a
+  // row had less than half (a plan that repeats keeps its estimate, and its graph).
+  static constexpr double P_PER_BYTE = 0.25;
+  static constexpr int P_IDLE = 8;
+  double p_per_byte = P_PER_BYTE;
+  int p_idle = 0;
+  // a call of nbytes in ndocs documents had so many tiles of tpos positions, est expected
+  void positions_learn(uint64_t tiles, uint64_t est, uint64_t ndocs, uint64_t tpos, uint64_t nbytes) {
+    if (nbytes == 0) return;
+    const double need =
+        1.25 * (double)((tiles - std::min(tiles, ndocs)) * tpos) / (double)nbytes;
+    if (tiles > est && tiles > 8) {
+      p_per_byte = std::min(4.0, std::max(p_per_byte, need));
+      p_idle = 0;
+    } else if (p_per_byte > P_PER_BYTE && 2 * need < p_per_byte) {
+      if (++p_idle < P_IDLE) return;
+      p_per_byte = std::max(P_PER_BYTE, need);
+      p_idle = 0;
+    } else {
+      p_idle = 0;
+    }
+  }
   // launch shapes (alpacc_set_tuning): persistent lex_reduce / parse_keys2 blocks per CU, and the
   // largest grid of the search kernels (16384 workgroups of 256 threads: 8 per SIMD's worth of
   // waves several times over; larger grids measured slower on a 256 MiB JSON document)
@@ -4559,8 +4595,7 @@ int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *e
   const uint64_t tiles_est =
       lexed ? std::min<uint64_t>(tiles_max, (uint64_t)(ctx->p_per_byte * (double)T) / FT_TILE + 1)
             : tiles_max;
-  uint64_t bcap = std::min<uint64_t>(P * std::max<uint32_t>(ctx->max_nb, 1),
-                                     std::max<uint64_t>(256, (uint64_t)(ctx->b_per_byte * (double)T)));
+  uint64_t bcap = ctx->bracket_cap(T, P * std::max<uint32_t>(ctx->max_nb, 1), 256);
   uint32_t *small = (uint32_t *)ctx->buf(B_SMALL, 64 * sizeof(uint32_t));
   uint16_t *ent = (uint16_t *)ctx->buf(B_ENT, ctx->E < 255 ? tiles_max * FT_TILE + 16
                                                            : (tiles_max * FT_TILE + 8) * sizeof(uint16_t));
@@ -4644,16 +4679,13 @@ int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *e
     ctx->last_counts[2] = B;
     ctx->last_counts[3] = N;
     *num_nodes = N;
-    if (lexed && tile_count(true, P) > tiles_est)  // widen the estimate the grids are sized by
-      ctx->p_per_byte =
-          std::min(4.0, std::max(ctx->p_per_byte, 1.25 * (double)P / (double)std::max<uint64_t>(a.T, 1)));
+    if (lexed) ctx->positions_learn(tile_count(true, P), tiles_est, 1, FT_TILE, a.T);
     if (B > bcap) {  // more open ends than records: the tree kernels wrote nothing
       if (attempt > 0) {
         ctx->err = "link scratch sizing did not converge";
         return ALPACC_ERR_HIP;
       }
-      bcap = B + B / 8 + 256;
-      if (a.T) ctx->b_per_byte = std::max(ctx->b_per_byte, (double)bcap / (double)a.T);
+      bcap = ctx->bracket_learn(B, a.T);
       a.bcap = bcap;
       a.links = (uint2 *)ctx->buf(B_LINKS, (bcap + 16) * sizeof(uint2));
       if (!a.links) {
@@ -5109,9 +5141,7 @@ int run_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offset
   for (uint32_t d = 0; d < ndocs; ++d) nbytes += lengths[d];
   // brackets (the tree parser: open ends, fewer): at most max_nb per key position (T + 2 <= length + 2 per document)
   const uint64_t b_bound = (nbytes + 2ull * ndocs) * std::max<uint32_t>(ctx->max_nb, 1);
-  uint64_t bcap = std::min<uint64_t>(
-      b_bound, std::max<uint64_t>(ctx->tree_ok ? 256 : 4096,
-                                  (uint64_t)(ctx->b_per_byte * (double)nbytes)));
+  uint64_t bcap = ctx->bracket_cap(nbytes, b_bound, ctx->tree_ok ? 256 : 4096);
   for (int attempt = 0; attempt < 2; ++attempt) {
     ParseBatchPlan pl;
     int rc = plan_parse_batch(ctx, d_in, offsets, lengths, ndocs, parent, node, span, cap, bcap,
@@ -5146,12 +5176,9 @@ int run_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offset
       ctx->err = "output capacity too small";
       return ALPACC_ERR_CAPACITY;
     }
-    if (ntiles > pl.tiles_est && nbytes)  // the striding pass ran: widen the estimate
-      ctx->p_per_byte = std::min(
-          4.0, std::max(ctx->p_per_byte, 1.25 * (double)positions / (double)nbytes));
+    ctx->positions_learn(ntiles, pl.tiles_est, ndocs, 1ull << pl.a.tshift, nbytes);
     if (B > bcap) {  // the first pass wrote nothing: size the brackets for this batch
-      bcap = B + B / 8 + 4096;
-      if (nbytes) ctx->b_per_byte = std::max(ctx->b_per_byte, (double)bcap / (double)nbytes);
+      bcap = ctx->bracket_learn(B, nbytes);
       continue;
     }
     memcpy(results, pl.h_results, ndocs * sizeof(alpacc_doc_result));
@@ -5634,7 +5661,11 @@ int alpacc_set_tuning(alpacc_ctx *ctx, const alpacc_tuning *t) {
   ctx->lex_bpc = t->lex_blocks_per_cu;
   ctx->keys_bpc = t->keys_blocks_per_cu;
   ctx->search_cap = t->search_max_blocks;
-  ctx->b_per_byte = t->brackets_per_kib / 1024.0;
+  if (t->brackets_per_kib != ctx->brackets_per_kib()) {  // (else nothing that calls showed is lost)
+    ctx->b_per_byte = t->brackets_per_kib / 1024.0;
+    ctx->b_seen = 0.0;
+    ctx->b_need = 0;
+  }
   ctx->search_bs = t->search_block_threads;
   if ((t->lexer_tables_in_lds != 0) != (ctx->lex_tables_lds != 0) && ctx->has_lexer) {
     ctx->lex_tables_lds = t->lexer_tables_in_lds != 0;
@@ -5655,7 +5686,7 @@ int alpacc_get_tuning(alpacc_ctx *ctx, alpacc_tuning *t) {
   t->lex_blocks_per_cu = ctx->lex_bpc;
   t->keys_blocks_per_cu = ctx->keys_bpc;
   t->search_max_blocks = ctx->search_cap;
-  t->brackets_per_kib = (uint32_t)std::min(ctx->b_per_byte * 1024.0 + 0.5, (double)(1u << 20));
+  t->brackets_per_kib = ctx->brackets_per_kib();
   t->search_block_threads = ctx->search_bs;
   t->lexer_tables_in_lds = ctx->lex_tables_lds;
   t->graph_launches = ctx->graph_launches;

@@ -211,8 +211,10 @@ int alpacc_test_force_timeout(alpacc_ctx *ctx, int on);
  *   search_block_threads: workgroup size of bracket_match / parse_parents (256, 512 or 1024;
  *                       default 256)
  *   brackets_per_kib  : brackets (tree parser: open ends of its tiles) per KiB of input the
- *                       scratch is first sized for (1..2^20, default 256); a call with more runs again sized exactly, and the estimate
- *                       grows to what calls needed
+ *                       scratch is first sized for (1..2^20, default 256). A call with more runs its
+ *                       last kernels (batched: all) again sized exactly; what it needed, a number and
+ *                       not a ratio, is kept for later calls, and read back here per KiB of that call.
+ *                       Setting another value drops it
  *   lexer_tables_in_lds: 1 (default) = the lexer's tables in LDS where they fit (the
  *                       (endo x class) table up to 160 KiB, the DFA table up to 4096 entries),
  *                       read from L2 otherwise; 0 = every lexer table read from L2
