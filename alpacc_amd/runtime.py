@@ -201,10 +201,13 @@ class DeviceBuffer:
 
 COPY_SPLIT = 16 << 20     # bytes per host copy task
 PINNED_MIN = 1 << 20      # uploads from this size go through pinned staging
-LEASE_MIN = 128 << 10     # downloads from this size land in pinned memory that the arrays keep ...
+LEASE_MIN = 128 << 10     # result arrays from this size are over blocks that are used again ...
 LEASE_MAX = 16 << 20      # ... up to this size
-LEASE_TOTAL = 64 << 20    # pinned memory one context lends at most
-DIRECT_MAX = 4 << 20      # downloads below this size are copied out of pinned staging in one piece
+LEASE_TOTAL = 64 << 20    # bytes of such blocks one context holds at most
+# Downloads below this size are copied out of pinned staging by the caller's thread, larger ones by
+# the pool of threads: on fresh pages, which a program that keeps its results always has, one thread is
+# slower from here on (trees of 512 and 800 KiB of JSON: 738 and 1086 us against 566 and 775).
+DIRECT_MAX = 2 << 20
 _COPY_POOL = None
 _COPY_POOL_LOCK = threading.Lock()
 
@@ -338,66 +341,69 @@ class HostBuffer:
 
 
 class _Lease:
-    """A pinned block while arrays view it; it goes back to its pool with the last of them."""
+    """A block while arrays view it; it goes back to its pool with the last of them."""
 
-    def __init__(self, pool, buf):
-        self.pool, self.buf = pool, buf
+    def __init__(self, pool, block):
+        self.pool, self.block = pool, block
 
     def __del__(self):
         try:
-            self.pool.give(self.buf)
+            self.pool.give(self.block)
         except Exception:
             pass
 
 
-class PinnedPool:
-    """Pinned blocks that downloaded arrays are made of: 1 MiB comes back in 50 us, against 81
-    through staging and one host copy and 166 through sliced copies by the thread pool; 16 MiB in
-    330 against 830 and 645. A copy out of staging reads what the DMA has just written to memory, at
-    about 20 GB/s. Blocks are powers of two; at most LEASE_TOTAL bytes are allocated, lent and free
-    together (beyond it the caller copies). A block may come back from any thread (the last array's
-    owner), so the free lists are deques, whose appends and pops are atomic; take() is called by the
-    context's one thread."""
+class BlockPool:
+    """Blocks of ordinary memory that result arrays are made of, used again when the last array over
+    one is gone, so that a program that drops its results writes to the same pages whatever its
+    allocator does with freed memory: where it gives it back (glibc with a fixed trim threshold),
+    host trees of 256 KiB of JSON take 184 us against 374, of 800 KiB 331 against 876; where it keeps
+    it there is no difference.
+    The blocks are not the pinned memory that the device writes to, although that would save the host
+    copy (140 us at 256 KiB): a forked child does not get pinned memory, and a caller's asynchronous
+    copy out of an array that is then dropped might still be running when the block is lent again (out
+    of ordinary memory, such a copy has read its source when the call returns).
+    Blocks are powers of two; at most LEASE_TOTAL bytes are lent and free together (beyond it arrays
+    are allocated one by one). A block may come back from any thread (the last array's owner), so
+    the free lists are deques, whose appends and pops are atomic; take() is called by the context's
+    one thread."""
 
-    def __init__(self, lib):
-        self.lib = lib
+    def __init__(self):
         self.free = {}
         self.allocated = 0
         self.closed = False
 
     def take(self, nbytes: int):
-        """A uint8 array over a pinned block of at least nbytes, or None."""
+        """A uint8 array over a block of at least nbytes, or None."""
         size = max(LEASE_MIN, 1 << max(nbytes - 1, 1).bit_length())
         try:
-            buf = self.free.setdefault(size, collections.deque()).pop()
+            block = self.free.setdefault(size, collections.deque()).pop()
         except IndexError:
             for other in list(self.free.values()):  # room from free blocks of other sizes
                 while self.allocated + size > LEASE_TOTAL and other:
                     self._drop(other)
             if self.allocated + size > LEASE_TOTAL:
                 return None
-            try:
-                buf = HostBuffer(size, self.lib)
-            except MemoryError:
-                return None
+            block = np.empty(size, dtype=np.uint8)
             self.allocated += size
-        raw = (ctypes.c_uint8 * nbytes).from_address(buf.ptr)
-        raw.lease = _Lease(self, buf)  # arrays over raw keep it, and with it the block
+        raw = (ctypes.c_uint8 * nbytes).from_buffer(block)
+        raw.lease = _Lease(self, block)  # arrays over raw keep it, and with it the block
         return np.frombuffer(raw, dtype=np.uint8)
+
+    def empty(self, nbytes: int) -> np.ndarray:
+        """A uint8 array of nbytes for the caller to keep, over a block where there is one for it."""
+        mem = self.take(nbytes) if LEASE_MIN <= nbytes <= LEASE_MAX else None
+        return np.empty(nbytes, dtype=np.uint8) if mem is None else mem
 
     def _drop(self, blocks):
         try:
-            buf = blocks.pop()
+            self.allocated -= blocks.pop().nbytes
         except IndexError:
             return
-        self.allocated -= buf.nbytes
-        buf.free()
 
-    def give(self, buf: HostBuffer):
-        if self.closed:
-            buf.free()
-        else:
-            self.free[buf.nbytes].append(buf)
+    def give(self, block: np.ndarray):
+        if not self.closed:
+            self.free[block.nbytes].append(block)
 
     def close(self):
         self.closed = True
@@ -483,7 +489,7 @@ class Context:
         self._bufs: dict = {}
         self._pins: dict = {}  # grow-only pinned staging for large transfers
         self._events = None    # events of pipelined downloads
-        self._lent = PinnedPool(self.lib)  # pinned blocks that downloaded arrays keep
+        self._lent = BlockPool()  # blocks that downloaded arrays are made of
 
     def close(self):
         for b in list(self._bufs.values()) + list(self._pins.values()):
@@ -542,10 +548,10 @@ class Context:
         return buf, n
 
     def download_arrays(self, parts) -> list:
-        """[(DeviceBuffer, dtype, count), ...] -> host arrays, one block for all of them: small ones
-        copied out of pinned staging, those of LEASE_MIN .. LEASE_MAX bytes in a pinned block of the
-        context's pool that the arrays keep, larger ones (and any when LEASE_TOTAL is lent out)
-        through pinned staging with parallel host copies."""
+        """[(DeviceBuffer, dtype, count), ...] -> host arrays of ordinary memory, through pinned
+        staging: below DIRECT_MAX bytes in all, every part is queued into it, waited for once and
+        copied to an array of its own; larger results go in slices, whose host copies run in
+        parallel, to one block that the arrays share."""
         sizes = [np.dtype(dt).itemsize * int(c) for _, dt, c in parts]
         offs = [0]
         for size in sizes:
@@ -554,29 +560,25 @@ class Context:
         for (b, _, _), size in zip(parts, sizes):
             if size > b.nbytes:
                 raise ValueError("download larger than the buffer")
-        mem = self._lent.take(total) if LEASE_MIN <= total <= LEASE_MAX else None
-        if mem is not None or total < DIRECT_MAX:
-            # every part queued into pinned memory, one wait, and one host copy where it is staging
-            lent = mem is not None
-            if lent:
-                dst = mem.ctypes.data
-            else:
-                pin = self.pinned("out", max(1 << 20, 1 << max(total - 1, 1).bit_length()))
-                dst = pin.ptr
+        if total < DIRECT_MAX:
+            pin = self.pinned("out", max(1 << 20, 1 << max(total - 1, 1).bit_length()))
             for (b, _, _), size, off in zip(parts, sizes, offs):
-                if self.lib.alpacc_copy_to_host_async(ctypes.c_void_p(dst + off),
+                if self.lib.alpacc_copy_to_host_async(ctypes.c_void_p(pin.ptr + off),
                                                       ctypes.c_void_p(b.ptr), size,
                                                       self.stream) != 0:
                     raise RuntimeError("device to host copy failed")
             if self.lib.alpacc_stream_sync(self.stream) != 0:
                 raise RuntimeError("device to host copy failed")
-            if not lent:
-                mem = pin.array[:total].copy()
-            return [mem[off:off + size].view(dt) for (_, dt, _), size, off in zip(parts, sizes, offs)]
+            out = []
+            for (_, dt, _), size, off in zip(parts, sizes, offs):
+                mem = self._lent.empty(size)
+                np.copyto(mem, pin.array[off:off + size])
+                out.append(mem.view(dt))
+            return out
         pin = self.pinned("out", total)
         if self._events is None:
             self._events = SliceEvents(self.lib)
-        mem = np.empty(total, dtype=np.uint8)
+        mem = self._lent.empty(total)
         pipelined_download(self.lib, self.stream,
                            [(b.ptr, size, off) for (b, _, _), size, off in zip(parts, sizes, offs)
                             if size], pin, mem, self._events)
