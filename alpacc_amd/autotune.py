@@ -7,11 +7,12 @@ the kernels take their launch choices at run time, so they are timed instead:
 
 * lexer_tables_in_lds: the lexer's tables in LDS where they fit, or all of them read from L2;
 * lex_blocks_per_cu / keys_blocks_per_cu: persistent workgroups per CU of lex_reduce (its LDS holds
-  the grammar's (endomorphism x byte class) table, whose size sets how many fit) and of parse_keys2
-  (its LDS holds the pair index);
-* search_block_threads / search_max_blocks: workgroup size and grid of the two searches;
-* brackets_per_kib: the first size of the batched bracket scratch, from the brackets a sample batch
-  needed (a batch that needs more than its estimate runs twice);
+  the grammar's (endomorphism x byte class) table, whose size sets how many fit) and of
+  parse_keys_tree / parse_keys2 (their LDS holds the pair index);
+* search_block_threads / search_max_blocks: workgroup size and grid of the two searches, for grammars
+  that run them (those the tree parser takes do not, and a candidate there could only win by noise);
+* brackets_per_kib: the first size of the bracket (tree parser: open end) scratch, from what a sample
+  batch needed (a batch that needs more than its estimate runs twice);
 * graph_mode: whether batched calls that repeat their plan replay a HIP graph.
 
 A tuning record is keyed by the grammar's table sizes (endomorphisms, byte classes, DFA states,
@@ -32,6 +33,8 @@ import numpy as np
 DEFAULTS = {"graph_mode": 1, "lex_blocks_per_cu": 2, "keys_blocks_per_cu": 2,
             "search_max_blocks": 16384, "search_block_threads": 256, "brackets_per_kib": 256,
             "lexer_tables_in_lds": 1}
+
+SEARCHES = ("search_block_threads", "search_max_blocks")
 
 SPACE = (
     ("lexer_tables_in_lds", (1, 0)),
@@ -147,6 +150,10 @@ def tune(bundle, docs, reps: int = 3, path: str | None = None, save_result: bool
         # the bracket scratch estimate: what this batch needed, with a quarter more
         brackets = ctx.last_counts()["brackets"]
         kib = max(batch.nbytes / 1024.0, 1.0)
+        ctx.profile(True)
+        batch.run()
+        searches = ctx.read_profile()["bracket_match"][1] > 0
+        ctx.profile(False)
         params = dict(DEFAULTS)
         params["brackets_per_kib"] = int(min(1 << 20, max(1, math.ceil(1.25 * brackets / kib))))
         ctx.set_tuning(**params)
@@ -154,6 +161,8 @@ def tune(bundle, docs, reps: int = 3, path: str | None = None, save_result: bool
         best_ms = base_ms
         tried = []
         for name, values in SPACE:
+            if name in SEARCHES and not searches:
+                continue
             for v in values:
                 if v == params[name]:
                     continue
