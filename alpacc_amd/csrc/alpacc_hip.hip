@@ -1191,7 +1191,7 @@ lex_emit(LexArgs p) {
         // streamed past the caches, unlike the kinds, which the parser reads right away: the spans
         // (8 bytes a token) are read once and later, and left in L2 their write-back and the lines
         // they displace cost the kernels after this one more than the plain stores save here.
-        // 256 MiB batch of sexp documents: 1042 -> 1012 us (parse_tree 517 -> 492, lex_emit
+        // 256 MiB batch of sexp documents: 1042 -> 1012 to 1018 us (parse_tree 517 -> 492, lex_emit
         // 228 -> 232); 256 MiB of JSON lexed alone 358 -> 356, with the parser unchanged (824).
         __builtin_nontemporal_store(sv, p.starts + g);
         __builtin_nontemporal_store((uint32_t)tbase + at + 1, p.ends + g);
@@ -3708,7 +3708,7 @@ struct alpacc_ctx {
     if (nbytes == 0) return;
     const double need =
         1.25 * (double)((tiles - std::min(tiles, ndocs)) * tpos) / (double)nbytes;
-    if (tiles > est && tiles > 8) {
+    if (tiles > est && tiles * tpos > 2048) {
       p_per_byte = std::min(4.0, std::max(p_per_byte, need));
       p_idle = 0;
     } else if (p_per_byte > P_PER_BYTE && 2 * need < p_per_byte) {
@@ -4391,7 +4391,10 @@ constexpr unsigned TREE_WAVES = 16;
 // workgroup, two rounds of its wavefronts, a launch less
 constexpr uint64_t TREE_LINK_MAX = 8;
 // highest level of the tiles' min hierarchy: up to 16384 tiles (of the bound) have no level above the
-// one that the tile scan writes, which saves a launch; only pops that end far away search it
+// one that the tile scan writes, which saves a launch; only pops that end far away search it. Against
+// 64: 2 MiB of brackets nested to the middle 300 us and 319, ordinary JSON of 1 and 2 MiB 66 and 67.5,
+// 70 and 71.5, larger documents the same. With 1024 the search of nested ones shows: 4 MiB 802 us
+// against 578.
 constexpr uint64_t TILE_TOP = 256;
 
 // tiles of `positions` key positions, of the tree parser or the element-level one
@@ -4577,7 +4580,7 @@ int run_parse_tokens(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, co
 
 // run_parse_tokens for the tree parser: one queue, with one host synchronisation at its end. The
 // kernels size themselves by the device's counts (tree_verdict), the records of open ends by an
-// estimate from T (b_per_byte, grown to what calls needed): a call that needs more runs the tree
+// estimate from T and what earlier calls needed (bracket_cap): a call that needs more runs the tree
 // kernels again. The synchronisation in the middle that sized the element scratch cost about 25 us.
 template <typename S>
 int run_tree(alpacc_ctx *ctx, const uint32_t *kinds, const S *starts, const S *ends, uint64_t T,
@@ -4977,8 +4980,8 @@ int plan_parse_batch(alpacc_ctx *ctx, const uint8_t *d_in, const uint64_t *offse
   }
   pl.tiles_max = tiles_max;
   // the grid of parse_tree / parse_expand2: the tiles of an estimate of the key positions
-  // (p_per_byte of the input, grown to what calls needed; the bound from the input bytes is several
-  // times the count); parse_tree strides over any tiles past it, parse_expand2 has a striding pass
+  // (p_per_byte of the input, which follows what calls needed; the bound from the input bytes is
+  // several times the count); parse_tree strides over any tiles past it, parse_expand2 has a striding pass
   pl.tiles_est = std::min<uint64_t>(
       tiles_max, (uint64_t)(ctx->p_per_byte * (double)nbytes) / tpos + ndocs + 1);
   pl.stride_blocks =

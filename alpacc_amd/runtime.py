@@ -632,7 +632,8 @@ class Context:
             b.nbytes for b in self._bufs.values())
 
     def last_counts(self) -> dict:
-        """Element counts of the last parser call: tokens, positions, brackets, productions."""
+        """Element counts of the last parser call: tokens, positions, brackets (tree parser: the pops
+        and pushes that its tiles leave open), productions."""
         out = np.zeros(4, dtype=np.uint64)
         self.lib.alpacc_last_counts(self.handle, out.ctypes.data)
         return dict(zip(("tokens", "positions", "brackets", "productions"), (int(x) for x in out)))

@@ -435,6 +435,7 @@ def main():
     #                                           per bracket; s, node word and span per node out
     #   bracket_match : 6 B                     depth + symbol per bracket
     #   parse_parents : 8 N                     s in, parent out
+    # (counts["brackets"] is B for these three; where the tree parser ran, its tiles' open ends)
     cnt = ctx.last_counts() if args.workload == "parse" else {}
     P, B, N_ = cnt.get("positions", 0), cnt.get("brackets", 0), cnt.get("productions", 0)
     alg = {"lex_reduce": n, "lex_emit": n + (9 if args.workload == "parse" else 12) * T}
